@@ -162,11 +162,14 @@ int pasif_last_timing(const pasif_driver* d, double* kernel_ms, uint32_t* launch
  * (default): the lane kernel for the structures that fit it (the 8 with the
  * most work), the tile kernel for the rest, launched side by side, and the
  * row-parallel path for systems that fit neither.  PASIF_KERNEL_BIG: every
- * instance on the row-parallel path -- one workgroup of 1024 threads per
- * (system, excitation), rows strided over its threads, state and stage
- * vectors in device memory, a barrier between stages; any system size, no
- * trajectory or amplitude window (PASIF_ERR_UNSUPPORTED), not for pool jobs
- * or pasif_solve_noalloc. */
+ * instance on the row-parallel path -- one workgroup of up to 1024 threads
+ * per (system, excitation), rows spread over its threads, a barrier between
+ * stages, stage vectors in LDS (systems of more rows than LDS holds: in
+ * device memory); any system size, no trajectory or amplitude window
+ * (PASIF_ERR_UNSUPPORTED), not for pool jobs or pasif_solve_noalloc.
+ * PASIF_KERNEL_AUTO also takes this path for systems of more than 129 rows
+ * that no lane layout holds; those that fit a tile keep trajectories, windows
+ * and pasif_solve_noalloc there. */
 int pasif_set_kernel(pasif_driver* d, int kernel);
 /* what the packed problem runs on: kernel (TILE, LANE, BIG or MIXED), structure classes
  * (lane kernel; 0 for tiles) and the checkpoint interval the adjoint uses

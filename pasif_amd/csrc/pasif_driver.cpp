@@ -21,6 +21,7 @@
 #include <limits>
 #include <memory>
 #include <map>
+#include <mutex>
 #include <set>
 #include <thread>
 #include <numeric>
@@ -30,6 +31,7 @@
 #include "../../include/pasif.h"
 #include "pasif_host.hpp"
 #include "pasif_lane.hpp"
+#include "pasif_rows_pack.hpp"
 #include "pasif_tiles.hpp"
 
 using namespace pasif;
@@ -246,6 +248,18 @@ struct Packed {
   uint32_t b_part_max = 0;             // most segments of one instance's side
   uint64_t b_vec_f = 0, b_vec_a = 0, b_ck = 0, b_seg = 0;
   uint32_t b_tmax = 0, b_every = 1;
+  // row kernel (pasif_rows.hpp): instances, the unique systems' programs,
+  // per-instance scratch sizes (elements), launch width and LDS slots
+  bool rows = false;
+  uint32_t nrow = 0;
+  DevBuf r_inst, r_blk, r_val, r_word, r_init, r_force, r_row, r_piece, r_sink;
+  uint64_t r_vec_f = 0, r_vec_a = 0, r_ck = 0, r_seg = 0, r_path = 0;
+  uint32_t r_tmax = 0, r_every = 1, r_waves = 0, r_slots = 0, r_ys = 0, r_xs = 0, r_ps = 0;
+  bool r_resident = false;
+  // some system is on the row-parallel path because nothing else takes it
+  // (or because the caller asked for that path): no per-step outputs, no
+  // allocation-free solve
+  bool big_only = false;
   uint32_t max_forced = 0;
   size_t program_bytes = 0;
   void release() {
@@ -254,7 +268,8 @@ struct Packed {
                      &a_steps, &a_exc,   &a_fslot, &a_force, &a_val,  &a_idx, &a_init,
                      &ck_tile, &b_inst,  &b_rf,    &b_vf,    &b_xf,    &b_ff,  &b_if,
                      &b_ra,    &b_va,    &b_xa,    &b_ia,    &b_sgf,   &b_spf, &b_sga,
-                     &b_spa};
+                     &b_spa,   &r_inst,  &r_blk,   &r_val,   &r_word,  &r_init, &r_force,
+                     &r_row,   &r_piece, &r_sink};
     for (DevBuf* b : all) b->release();
     lparts.clear();
     lshapes.clear();
@@ -264,8 +279,13 @@ struct Packed {
     tile = false;
     big = false;
     nbig = 0;
+    b_tmax = 0;
     b_part = 0;
     b_part_max = 0;
+    rows = false;
+    nrow = 0;
+    r_tmax = 0;
+    big_only = false;
     ltmax = 0;
     valid = false;
   }
@@ -312,7 +332,9 @@ struct pasif_driver {
   int lane_bias = 0;
   // lane class of every system in the packed problem, -1: tile kernel
   std::vector<int32_t> lane_cls;
-  // systems on the row-parallel path (too large for a tile), by system
+  // systems on the row-parallel path, by system: kRowSys the row kernel,
+  // kBigSys the kernel with every vector in device memory, 0 neither
+  enum : uint8_t { kBigSys = 1, kRowSys = 2 };
   std::vector<uint8_t> big_sys;
   // structure of every system in the lane plan before classes were merged
   std::vector<uint32_t> lane_struct;
@@ -345,6 +367,7 @@ struct pasif_driver {
   DevBuf qstate, lstate, mxstate, progress, out_q, out_max, traj, out_grad, ckpt, segbuf;
   // run buffers of the row-parallel path
   DevBuf bvec_f, bvec_a, bsetp, bckpt, bseg, bprog, bpart;
+  DevBuf rvec_f, rvec_a, rckpt, rseg, rprog;
   // results of the last solve (host, double)
   std::vector<double> res_q, res_max;
   bool have_max = false;
@@ -355,6 +378,7 @@ struct pasif_driver {
   // destroyed by its owner while a tick in flight still ran it: the pool
   // deletes it once the tick is over
   bool orphan = false;
+  bool counted = false;  // one of the device's handles in the path pool
   uint32_t pool_ck = 0;
   // a pool job's lane kernel arguments, one vector per lane part (ticks
   // copy them into the pool's per-module tables)
@@ -531,6 +555,112 @@ int guarded(pasif_driver* d, F&& f) {
   }
 }
 
+// ------------------------------------------------------- stored-path memory
+// Device memory for the forward paths that adjoint solves store instead of
+// recomputing: leased for the length of one (synchronous) solve and kept for
+// the next solve of any handle on the device, since paths are large and the
+// driver clears freed device memory before it hands it out again (freeing
+// and allocating 32 GB in turn took 0.9 s a time).  Bounded: a lease is
+// granted only while all of it together stays within 32 GiB and the new
+// buffer within a quarter of the free memory; without one a solve recomputes
+// from checkpoints.  Given back when an allocation of the library's needs
+// the room and when the device's last handle is destroyed.
+struct PathPool {
+  struct Buf {
+    int dev;
+    void* p;
+    size_t bytes;
+    bool busy;
+  };
+  std::mutex mu;
+  std::vector<Buf> bufs;
+  std::map<int, uint32_t> handles;
+
+  void trim_locked(int dev) {
+    for (size_t i = bufs.size(); i-- > 0;)
+      if (bufs[i].dev == dev && !bufs[i].busy) {
+        (void)hipFree(bufs[i].p);
+        bufs.erase(bufs.begin() + long(i));
+      }
+  }
+  bool trim(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    const size_t n = bufs.size();
+    trim_locked(dev);
+    return bufs.size() != n;
+  }
+  size_t idle(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    size_t b = 0;
+    for (const Buf& x : bufs)
+      if (x.dev == dev && !x.busy) b += x.bytes;
+    return b;
+  }
+  void* take(int dev, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu);
+    Buf* best = nullptr;
+    size_t busy = 0;
+    for (Buf& x : bufs) {
+      if (x.dev != dev) continue;
+      if (x.busy)
+        busy += x.bytes;
+      else if (x.bytes >= bytes && (!best || x.bytes < best->bytes))
+        best = &x;
+    }
+    if (best) {
+      best->busy = true;
+      return best->p;
+    }
+    if (bytes + busy > (size_t(32) << 30)) return nullptr;
+    trim_locked(dev);
+    size_t f = 0, t = 0;
+    if (hipMemGetInfo(&f, &t) != hipSuccess || bytes > f / 4) return nullptr;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    bufs.push_back({dev, p, bytes, true});
+    return p;
+  }
+  void give(void* p) {
+    std::lock_guard<std::mutex> lk(mu);
+    for (Buf& x : bufs)
+      if (x.p == p) x.busy = false;
+  }
+  void attach(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    ++handles[dev];
+  }
+  void detach(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    if (--handles[dev] == 0) trim_locked(dev);
+  }
+};
+PathPool& path_pool() {
+  static PathPool* p = new PathPool;  // outlives every handle
+  return *p;
+}
+
+// The leases of one solve, returned when it is over (after a failed launch:
+// once the device is idle).
+struct PathLease {
+  std::vector<void*> held;
+  PathLease() = default;
+  PathLease(const PathLease&) = delete;
+  PathLease& operator=(const PathLease&) = delete;
+  void* take(int dev, size_t bytes) {
+    void* p = path_pool().take(dev, bytes);
+    if (p) held.push_back(p);
+    return p;
+  }
+  ~PathLease() {
+    if (held.empty()) return;
+    if (std::uncaught_exceptions() > 0) (void)hipDeviceSynchronize();
+    for (void* p : held) path_pool().give(p);
+  }
+};
+
 static_assert(kScratchBytes == PASIF_NOALLOC_SCRATCH_BYTES, "scratch size stated in pasif.h");
 
 // set while pasif_solve_noalloc runs on this thread: any device allocation
@@ -554,6 +684,10 @@ void dev_alloc(pasif_driver* d, DevBuf& b, size_t bytes) {
     return;
   }
   hipError_t e = hipMalloc(&b.p, bytes);
+  if (e != hipSuccess && path_pool().trim(d->dev)) {
+    (void)hipGetLastError();
+    e = hipMalloc(&b.p, bytes);
+  }
   if (e != hipSuccess) {
     b.p = nullptr;
     set_err(d, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorName(e));
@@ -1170,6 +1304,11 @@ template <typename R>
 void pack_big(pasif_driver* d, bool adjoint) {
   Packed& pk = d->pk;
   std::vector<Instance> inst = make_instances(d, adjoint, kPartBig);
+  inst.erase(std::remove_if(inst.begin(), inst.end(),
+                            [&](const Instance& in) {
+                              return d->big_sys[in.sys] != pasif_driver::kBigSys;
+                            }),
+             inst.end());
   const double eps = std::numeric_limits<R>::epsilon();
   struct Side {
     std::vector<uint32_t> rptr, idx, seg, sptr;
@@ -1289,6 +1428,115 @@ void pack_big(pasif_driver* d, bool adjoint) {
   pk.out_len_a = adjoint ? (d->mapped ? d->adj.n : d->adj.n * d->n_exc) : 0;
   if (d->d_compute)
     printf("[pasif] %zu instances on the row-parallel path, T max %u\n", inst.size(), tmax);
+}
+
+// Units of both sides of system s for the row kernel; false if it does not
+// hold the system.
+bool row_plan(const pasif_driver* d, uint32_t s, bool adjoint, size_t el, RowUnits* f,
+              RowUnits* a) {
+  *f = row_units(d->fwd, s, row_published(d->fwd, s, false, adjoint ? &d->adj : nullptr));
+  if (adjoint) *a = row_units(d->adj, s, row_published(d->adj, s, true, nullptr));
+  return row_units_fit(*f, adjoint ? a : nullptr, el);
+}
+
+// Row-kernel packing: each system's program once (instances of several
+// excitations share it), the instances' scratch offsets.
+template <typename R>
+void pack_rows(pasif_driver* d, bool adjoint) {
+  Packed& pk = d->pk;
+  std::vector<Instance> inst = make_instances(d, adjoint, kPartBig);
+  inst.erase(std::remove_if(inst.begin(), inst.end(),
+                            [&](const Instance& in) {
+                              return d->big_sys[in.sys] != pasif_driver::kRowSys;
+                            }),
+             inst.end());
+  uint32_t tmax = 0, K = 1;
+  for (const Instance& in : inst) tmax = std::max(tmax, in.steps);
+  if (adjoint)
+    K = std::max<uint32_t>(1, std::min<uint32_t>(d->ck_every ? d->ck_every : 256u,
+                                                 std::max<uint32_t>(tmax, 1)));
+  RowPacked<R> o;
+  struct Prog {
+    RowProg f, a;
+    uint32_t waves;
+  };
+  std::map<uint32_t, Prog> progs;
+  std::vector<RowInst> ri(inst.size());
+  pk.r_vec_f = pk.r_vec_a = pk.r_ck = pk.r_seg = pk.r_path = 0;
+  pk.r_waves = pk.r_slots = pk.r_ys = pk.r_xs = pk.r_ps = 0;
+  pk.r_resident = true;
+  const uint32_t per = adjoint && d->adj_mode ? 4u : 1u;  // values kept per step and row
+  for (size_t i = 0; i < inst.size(); ++i) {
+    const Instance& in = inst[i];
+    auto it = progs.find(in.sys);
+    if (it == progs.end()) {
+      RowUnits uf, ua;
+      (void)row_plan(d, in.sys, adjoint, sizeof(R), &uf, &ua);
+      Prog p{};
+      const uint32_t zy = std::max(uf.pub, ua.pub);
+      p.f = row_emit(o, d->fwd, in.sys, uf, false, uf.slot, d->fwd.off[in.sys], zy, zy);
+      if (adjoint)
+        p.a = row_emit(o, d->adj, in.sys, ua, true, uf.slot, d->adj.xoff[in.sys], zy, uf.pub);
+      // as few slots per thread as 1,024 threads allow, then as few waves
+      const uint32_t units =
+          uint32_t(std::max<size_t>(1, std::max(uf.main.size(), ua.main.size())));
+      const uint32_t slots = (units + kRowThreads - 1) / kRowThreads;
+      p.waves = (units + 64u * slots - 1) / (64u * slots);
+      pk.r_waves = std::max(pk.r_waves, p.waves);
+      pk.r_slots = std::max(pk.r_slots, slots);
+      pk.r_ys = std::max(pk.r_ys, zy + 1u);
+      if (adjoint) pk.r_xs = std::max(pk.r_xs, uf.pub + 1u);
+      for (const RowUnits* u : {&uf, &ua})
+        for (const RowUnit& x : u->main)
+          if (x.cnt[0] > kRowRes1 || x.cnt[1] > kRowRes2 || x.cnt[2] > kRowRes3 ||
+              x.cnt[3] > kRowRes4)
+            pk.r_resident = false;
+      for (const RowUnits* u : {&uf, &ua})
+        pk.r_ps = std::max<uint32_t>(pk.r_ps, uint32_t(std::max<size_t>(u->aux.size(), u->pieces)));
+      it = progs.emplace(in.sys, p).first;
+    }
+    RowInst& r = ri[i];
+    r.f = it->second.f;
+    r.a = it->second.a;
+    r.waves = it->second.waves;
+    r.n_f = d->fwd.size[in.sys];
+    r.steps = in.steps;
+    r.out_f = in.out_f;
+    r.out_a = adjoint ? in.out_a : 0u;
+    r.exc = in.exc;
+    r.vec_f = pk.r_vec_f;
+    pk.r_vec_f += 2ull * r.f.units + r.f.nsink;
+    if (adjoint) {
+      r.vec_a = pk.r_vec_a;
+      pk.r_vec_a += r.a.units;
+      r.ck = pk.r_ck;
+      pk.r_ck += uint64_t(std::max<uint32_t>(1, (in.steps + K - 1) / K)) * r.n_f;
+      r.seg = pk.r_seg;
+      pk.r_seg += (per > 1 ? uint64_t(per) * K : K + 1ull) * r.f.pub;
+      r.path = pk.r_path;
+      pk.r_path += (per > 1 ? uint64_t(per) * in.steps : in.steps + 1ull) * r.f.pub;
+    }
+  }
+  upload(d, pk.r_inst, ri);
+  upload(d, pk.r_blk, o.blk);
+  upload(d, pk.r_val, o.val);
+  upload(d, pk.r_word, o.word);
+  upload(d, pk.r_init, o.init);
+  upload(d, pk.r_force, o.force);
+  upload(d, pk.r_row, o.row);
+  upload(d, pk.r_piece, o.piece);
+  upload(d, pk.r_sink, o.sink);
+  if (d->dev >= 0) PASIF_HIP(hipStreamSynchronize(d->stream));
+  pk.big = true;
+  pk.rows = true;
+  pk.nrow = uint32_t(inst.size());
+  pk.r_tmax = tmax;
+  pk.r_every = K;
+  pk.out_len_f = d->mapped ? d->fwd.n : d->fwd.n * d->n_exc;
+  pk.out_len_a = adjoint ? (d->mapped ? d->adj.n : d->adj.n * d->n_exc) : 0;
+  if (d->d_compute)
+    printf("[pasif] %zu instances on the row kernel (%u waves, %u units per thread), T max %u\n",
+           inst.size(), pk.r_waves, pk.r_slots, tmax);
 }
 
 // Whether system s fits one tile under some slot configuration the tile
@@ -2554,6 +2802,9 @@ void require_device(pasif_driver* d) {
 template <typename R>
 void pool_lane_parts(pasif_driver* d, bool adjoint);
 
+// rows of a system that fits a tile above which the row kernel takes it
+constexpr uint32_t kTileRows = 129;
+
 void ensure_packed(pasif_driver* d, bool adjoint) {
   PASIF_REQUIRE(d->sys_ready, PASIF_ERR_STATE, "the system must be allocated before solving");
   if (adjoint)
@@ -2572,9 +2823,10 @@ void ensure_packed(pasif_driver* d, bool adjoint) {
   PASIF_REQUIRE(!(d->pool && d->kernel_path == PASIF_KERNEL_BIG), PASIF_ERR_UNSUPPORTED,
                 "pool jobs run on the tile and lane kernels");
   const uint32_t S = uint32_t(d->fwd.size.size());
+  bool pk_only = d->kernel_path == PASIF_KERNEL_BIG;
   if (d->pool && exact) d->lane_cls.clear();  // the pool's lane modules run the reference recursion
   if (d->kernel_path == PASIF_KERNEL_BIG) {
-    d->big_sys.assign(S, 1);
+    d->big_sys.assign(S, pasif_driver::kBigSys);
   } else if (d->kernel_path != PASIF_KERNEL_TILE && !d->pool) {
     if (d->precision == 64)
       (void)lane_plan<double>(d, adjoint);
@@ -2586,23 +2838,57 @@ void ensure_packed(pasif_driver* d, bool adjoint) {
     else
       pool_lane_parts<float>(d, adjoint);
   }
-  // under the automatic choice, systems the lane kernel did not take that do
-  // not fit a tile run on the row-parallel path (not for pool jobs)
+  // Under the automatic choice, systems the lane kernel did not take run on
+  // the row-parallel path when they do not fit a tile or have more rows than
+  // a 64-DOF chain with its probe (not for pool jobs).  Above that line a
+  // system fills a workgroup alone, and the tile kernel's serial sums of long
+  // rows set the step; forward + adjoint, tiles against the row kernel:
+  // 48 chains of 65 DOF x 500 steps 14.0 / 2.4 ms, 1,500 of them x 200 steps
+  // 23.1 / 4.1 ms, 48 chains of 150 DOF x 1,000 steps 52.1 / 5.1 ms.  Below
+  // it tiles pack several systems to a workgroup and keep what the lane
+  // kernel leaves.
   if (!d->pool && d->kernel_path == PASIF_KERNEL_AUTO) {
     d->big_sys.assign(S, 0);
     bool any = false;
-    for (uint32_t s = 0; s < S; ++s)
-      if (in_part(d, s, kPartTile) && !fits_tile(d, s, adjoint)) {
-        d->big_sys[s] = 1;
-        any = true;
-      }
+    for (uint32_t s = 0; s < S; ++s) {
+      if (!in_part(d, s, kPartTile)) continue;
+      const bool tile = fits_tile(d, s, adjoint);
+      if (tile && d->fwd.size[s] <= kTileRows) continue;
+      d->big_sys[s] = tile ? pasif_driver::kRowSys : pasif_driver::kBigSys;
+      if (!tile) pk_only = true;
+      any = true;
+    }
     if (!any) d->big_sys.clear();
   }
   if (!d->big_sys.empty()) {
-    if (d->precision == 64)
-      pack_big<double>(d, adjoint);
-    else
-      pack_big<float>(d, adjoint);
+    // the row kernel takes what its LDS and threads hold, the kernel with
+    // every vector in device memory the rest (a system that fits a tile and
+    // not the row kernel stays on tiles)
+    const size_t el = d->precision == 64 ? 8 : 4;
+    bool big = false, rows = false;
+    for (uint32_t s = 0; s < S; ++s) {
+      if (!d->big_sys[s]) continue;
+      RowUnits uf, ua;
+      const bool fit = row_plan(d, s, adjoint, el, &uf, &ua);
+      if (fit)
+        d->big_sys[s] = pasif_driver::kRowSys;
+      else if (d->big_sys[s] == pasif_driver::kRowSys)
+        d->big_sys[s] = 0;
+      big = big || d->big_sys[s] == pasif_driver::kBigSys;
+      rows = rows || d->big_sys[s] == pasif_driver::kRowSys;
+    }
+    if (big) {
+      if (d->precision == 64)
+        pack_big<double>(d, adjoint);
+      else
+        pack_big<float>(d, adjoint);
+    }
+    if (rows) {
+      if (d->precision == 64)
+        pack_rows<double>(d, adjoint);
+      else
+        pack_rows<float>(d, adjoint);
+    }
   }
   // the tile kernel takes every other system
   bool rest = false;
@@ -2618,7 +2904,8 @@ void ensure_packed(pasif_driver* d, bool adjoint) {
     d->pk.tmax = 0;
   }
   Packed& pk = d->pk;
-  pk.tmax = std::max(pk.tmax, std::max(pk.ltmax, pk.b_tmax));
+  pk.tmax = std::max(std::max(pk.tmax, pk.r_tmax), std::max(pk.ltmax, pk.b_tmax));
+  pk.big_only = pk_only;
   if (pk.lane && !pk.tile) {
     pk.ntiles = 0;  // reported: the lane launch's workgroups
     for (const auto& lp : pk.lparts) pk.ntiles += lp->blocks;
@@ -2796,6 +3083,73 @@ BigArgs<R> big_run_args(pasif_driver* d, bool adjoint, RunMem& mem, void* out_q,
     a.adjoint = 1;
     a.exact = d->adj_mode != 0 ? 1u : 0u;
     work = 3ull * pk.b_tmax;
+  }
+  *work_out = work;
+  return a;
+}
+
+// Arguments of a run of the row-kernel instances, as big_run_args; `lease`
+// (null: none) is where the stored path's memory comes from.
+template <typename R>
+RowArgs<R> row_run_args(pasif_driver* d, bool adjoint, uint32_t save_steps, uint32_t nslots,
+                        RunMem& mem, void* out_q, void* out_grad, PathLease* lease,
+                        uint64_t* work_out) {
+  Packed& pk = d->pk;
+  RowArgs<R> a{};
+  a.inst = pk.r_inst.as<RowInst>();
+  a.blk = pk.r_blk.as<uint4>();
+  a.val = pk.r_val.as<R>();
+  a.word = pk.r_word.as<uint32_t>();
+  a.init = pk.r_init.as<R>();
+  a.force = pk.r_force.as<R>();
+  a.row = pk.r_row.as<uint32_t>();
+  a.piece = pk.r_piece.as<uint32_t>();
+  a.sink = pk.r_sink.as<uint32_t>();
+  a.excit = d->ext_exc ? static_cast<const R*>(d->ext_exc) : d->d_exc.as<R>();
+  a.exc_len = d->exc_len;
+  a.interp = d->interp_w ? (d->ext_interp ? static_cast<const R*>(d->ext_interp)
+                                          : d->d_interp.as<R>())
+                         : nullptr;
+  a.interp_w = d->interp_w;
+  const R h = R(1.0 / double(d->sample_rate));
+  a.h = h;
+  a.h2 = R(double(h) / 2.0);
+  a.h6 = R(double(h) / 6.0);
+  const size_t el = sizeof(R);
+  a.vec_f = static_cast<R*>(mem.get(d->rvec_f, size_t(pk.r_vec_f) * el));
+  if (d->window) mem.zero(a.vec_f, size_t(pk.r_vec_f) * el);
+  a.progress = static_cast<uint32_t*>(mem.get(d->rprog, size_t(pk.nrow) * 4 * sizeof(uint32_t)));
+  mem.zero(a.progress, size_t(pk.nrow) * 4 * sizeof(uint32_t));
+  a.out_q = static_cast<R*>(out_q);
+  a.out_max = d->window ? d->out_max.as<R>() : nullptr;
+  a.window = d->window;
+  a.traj = save_steps ? d->traj.as<R>() : nullptr;
+  a.save_every = save_steps;
+  a.nslots = nslots;
+  a.out_len = pk.out_len_f;
+  a.ck_every = pk.r_every;
+  a.resident = pk.r_resident ? 1u : 0u;
+  a.y_slots = pk.r_ys;
+  a.x_slots = pk.r_xs;
+  a.part_slots = pk.r_ps;
+  uint64_t work = pk.r_tmax;
+  if (adjoint) {
+    a.vec_a = static_cast<R*>(mem.get(d->rvec_a, size_t(pk.r_vec_a) * el));
+    // With an interval of the caller's choice its checkpoints are kept and
+    // segments recomputed; with the automatic one the whole path is stored
+    // when it fits (one pass less of forward work; the plan's footprint
+    // stays that of the checkpoints, which always suffice).
+    if (lease && d->ck_every == 0)
+      a.segbuf = static_cast<R*>(lease->take(d->dev, size_t(pk.r_path) * el));
+    a.store = a.segbuf ? 1u : 0u;
+    if (!a.store) {
+      a.ckpt = static_cast<R*>(mem.get(d->rckpt, size_t(pk.r_ck) * el, true));
+      a.segbuf = static_cast<R*>(mem.get(d->rseg, size_t(pk.r_seg) * el));
+    }
+    a.out_grad = static_cast<R*>(out_grad);
+    a.adjoint = 1;
+    a.exact = d->adj_mode != 0 ? 1u : 0u;
+    work = (a.store ? 2ull : 3ull) * pk.r_tmax;
   }
   *work_out = work;
   return a;
@@ -3058,7 +3412,9 @@ void run_footprint(pasif_driver* d, bool adjoint, uint32_t save_steps, size_t* t
   if (pk.tile)
     (void)tile_run_args<R>(d, adjoint, save_steps, m, nullptr, nullptr, nullptr, nullptr, &work,
                            &nslots);
-  if (pk.big) (void)big_run_args<R>(d, adjoint, m, nullptr, nullptr, &work);
+  if (pk.nbig) (void)big_run_args<R>(d, adjoint, m, nullptr, nullptr, &work);
+  if (pk.rows) (void)row_run_args<R>(d, adjoint, save_steps, nslots, m, nullptr, nullptr, nullptr,
+                                      &work);
   for (auto& lp : pk.lparts) {
     auto args = lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, nullptr, nullptr, &m,
                                   nullptr, nullptr);
@@ -3075,7 +3431,8 @@ size_t held_run_bytes(const pasif_driver* d) {
   const DevBuf* own[] = {&d->qstate, &d->lstate, &d->mxstate, &d->progress, &d->out_q,
                          &d->out_max, &d->traj,   &d->out_grad, &d->ckpt,  &d->segbuf,
                          &d->bvec_f, &d->bvec_a,  &d->bsetp,    &d->bckpt, &d->bseg,
-                         &d->bprog,  &d->bpart};
+                         &d->bprog,  &d->bpart,   &d->rvec_f,   &d->rvec_a, &d->rckpt,
+                         &d->rseg,   &d->rprog};
   for (const DevBuf* x : own) b += x->bytes;
   for (const auto& lp : d->pk.lparts)
     for (const auto& c : lp->cls)
@@ -3094,7 +3451,11 @@ void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   size_t need = 0, ck = 0, freeb = 0, totalb = 0;
   run_footprint<R>(d, adjoint, save_steps, &need, &ck);
   PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
-  const double avail = 0.8 * double(freeb + held_run_bytes(d));
+  double avail = 0.8 * double(freeb + held_run_bytes(d));
+  if (double(need) > avail && path_pool().trim(d->dev)) {
+    PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
+    avail = 0.8 * double(freeb + held_run_bytes(d));
+  }
   PASIF_REQUIRE(double(need) <= avail, PASIF_ERR_MEMORY,
                 "the solve needs %zu bytes of run buffers (%zu of them checkpoints), more than "
                 "80%% of the free device memory (%.0f bytes available); lengthen the checkpoint "
@@ -3110,7 +3471,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, std::vector<
   ensure_packed(d, adjoint);
   Packed& pk = d->pk;
   const bool lane = pk.lane, tile = pk.tile, big = pk.big;
-  PASIF_REQUIRE(!big || (save_steps == 0 && d->window == 0), PASIF_ERR_UNSUPPORTED,
+  PASIF_REQUIRE(!pk.big_only || (save_steps == 0 && d->window == 0), PASIF_ERR_UNSUPPORTED,
                 "systems on the row-parallel path (too large for a tile) record neither a "
                 "trajectory nor an amplitude window");
   check_run_memory<R>(d, adjoint, save_steps);
@@ -3119,11 +3480,18 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, std::vector<
   TileArgs<R> ta{};
   if (tile) ta = prepare_run<R>(d, adjoint, save_steps, &twork, &nslots);
   BigArgs<R> ba{};
+  RowArgs<R> ra{};
+  PathLease lease;
+  uint64_t rwork = 0;
   if (big) {
-    (void)run_outputs<R>(d, adjoint, save_steps);
+    nslots = run_outputs<R>(d, adjoint, save_steps);
     RunMem mem;
     mem.d = d;
-    ba = big_run_args<R>(d, adjoint, mem, d->out_q.p, adjoint ? d->out_grad.p : nullptr, &bwork);
+    void* og = adjoint ? d->out_grad.p : nullptr;
+    if (pk.nbig) ba = big_run_args<R>(d, adjoint, mem, d->out_q.p, og, &bwork);
+    if (pk.rows)
+      ra = row_run_args<R>(d, adjoint, save_steps, nslots, mem, d->out_q.p, og, &lease, &rwork);
+    bwork = std::max(bwork, rwork);
   }
   std::vector<std::vector<LaneArgs>> largs;
   if (lane) {
@@ -3137,6 +3505,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, std::vector<
   const uint32_t budget = launch_budget(d, std::max(std::max(twork, lwork), bwork), &launches);
   ta.budget = budget;
   ba.budget = budget;
+  ra.budget = budget;
   for (size_t i = 0; i < largs.size(); ++i) {
     for (LaneArgs& a : largs[i]) a.budget = budget;
     upload(d, pk.lparts[i]->args, largs[i]);
@@ -3171,7 +3540,9 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, std::vector<
                       k < 0 ? d->stream : d->aux[k]);
     }
     if (tile && e == hipSuccess) e = launch_tiles(ta, nt, int(pk.slot_cfg), d->stream);
-    if (big && e == hipSuccess)
+    if (pk.rows && e == hipSuccess)
+      e = launch_rows(ra, pk.nrow, pk.r_waves, pk.r_slots, d->stream);
+    if (nb && e == hipSuccess)
       e = launch_big(ba, nb, ba.part_lds ? size_t(pk.b_part_max) * sizeof(R) : 0, d->stream);
     for (int k = 0; k < nside; ++k) {
       if (e == hipSuccess) e = hipEventRecord(d->join[k], d->aux[k]);
@@ -3205,7 +3576,7 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
   PASIF_REQUIRE(d->solver != PASIF_SOLVER_GRAPH, PASIF_ERR_UNSUPPORTED,
                 "pasif_solve_noalloc runs the persistent or the plain solver, not the graph one");
   PASIF_REQUIRE(!d->pool, PASIF_ERR_UNSUPPORTED, "pool jobs run through pasif_pool_tick");
-  PASIF_REQUIRE(!pk.big, PASIF_ERR_UNSUPPORTED,
+  PASIF_REQUIRE(!pk.big_only, PASIF_ERR_UNSUPPORTED,
                 "pasif_solve_noalloc runs the tile and lane kernels, not the row-parallel path");
   PASIF_REQUIRE(out_q != nullptr, PASIF_ERR_ARGUMENT, "out_q (device, %u values) is required",
                 pk.out_len_f);
@@ -3217,7 +3588,8 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
   const bool lane = pk.lane, tile = pk.tile;
   DevBuf unused;
   TileArgs<R> ta{};
-  uint64_t twork = 0;
+  RowArgs<R> ra{};
+  uint64_t twork = 0, rwork = 0;
   std::vector<std::vector<LaneArgs>> largs;
   std::vector<void*> tables;
   auto plan = [&](RunMem& mem) {
@@ -3227,6 +3599,7 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
     if (tile)
       ta = tile_run_args<R>(d, adjoint, 0, mem, out_q, nullptr, nullptr, out_grad, &twork,
                             &nslots);
+    if (pk.rows) ra = row_run_args<R>(d, adjoint, 0, 0, mem, out_q, out_grad, nullptr, &rwork);
     if (lane)
       for (auto& lp : pk.lparts) {
         largs.push_back(lane_part_args<R>(d, *lp, adjoint, 0, 0, d->d_exc.p, d->d_interp.p,
@@ -3249,8 +3622,9 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
   plan(mem);
   const uint64_t lwork = lane ? (adjoint ? 3ull * pk.ltmax : pk.ltmax) : 0;
   uint64_t launches = 1;
-  const uint32_t budget = launch_budget(d, std::max(twork, lwork), &launches);
+  const uint32_t budget = launch_budget(d, std::max(std::max(twork, rwork), lwork), &launches);
   ta.budget = budget;
+  ra.budget = budget;
   for (size_t i = 0; i < largs.size(); ++i) {
     for (LaneArgs& a : largs[i]) a.budget = budget;
     PASIF_HIP(hipMemcpyAsync(tables[i], largs[i].data(), largs[i].size() * sizeof(LaneArgs),
@@ -3263,6 +3637,8 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
       if (pk.lparts[i]->blocks)
         e = lane_launch(*pk.lparts[i], tables[i], uint32_t(largs[i].size()), d->stream);
     if (tile && e == hipSuccess) e = launch_tiles(ta, nt, int(pk.slot_cfg), d->stream);
+    if (pk.rows && e == hipSuccess)
+      e = launch_rows(ra, pk.nrow, pk.r_waves, pk.r_slots, d->stream);
     return e;
   });
 }
@@ -3345,6 +3721,8 @@ int pasif_create(pasif_driver** out, const double* excitations, uint32_t n_exc, 
       PASIF_HIP(hipGetDeviceCount(&ndev));
       PASIF_REQUIRE(gpu_id < ndev, PASIF_ERR_ARGUMENT, "GPU %d of %d", gpu_id, ndev);
       PASIF_HIP(hipSetDevice(gpu_id));
+      path_pool().attach(gpu_id);
+      d->counted = true;
       PASIF_HIP(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
       PASIF_HIP(hipEventCreate(&d->ev0));
       PASIF_HIP(hipEventCreate(&d->ev1));
@@ -3394,7 +3772,10 @@ int pasif_destroy(pasif_driver* d) {
     if (d->ev1) (void)hipEventDestroy(d->ev1);
     if (d->stream) (void)hipStreamDestroy(d->stream);
   }
+  const int dev = d->dev;
+  const bool counted = d->counted;
   delete d;
+  if (counted) path_pool().detach(dev);
   return PASIF_OK;
 }
 
@@ -3630,7 +4011,7 @@ int pasif_run_footprint(pasif_driver* d, int adjoint, size_t* run_bytes, size_t*
         size_t f = 0, t = 0;
         PASIF_HIP(hipSetDevice(d->dev));
         PASIF_HIP(hipMemGetInfo(&f, &t));
-        *free_bytes = f + held_run_bytes(d);
+        *free_bytes = f + held_run_bytes(d) + path_pool().idle(d->dev);
       }
     }
   });
@@ -3751,7 +4132,7 @@ int pasif_kernel_info(pasif_driver* d, int adjoint, int* kernel, uint32_t* class
     if (checkpoint_every)
       *checkpoint_every = !adjoint ? 0u
                           : pk.lane ? pk.lseg
-                          : (pk.big && !pk.tile) ? pk.b_every
+                          : (pk.big && !pk.tile) ? (pk.rows ? pk.r_every : pk.b_every)
                                                  : (d->ck_every ? d->ck_every : 256u);
   });
 }
