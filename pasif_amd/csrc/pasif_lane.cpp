@@ -435,16 +435,16 @@ bool plan_group(LaneShape& sh, uint32_t G) {
     std::sort(sh.gx.begin(), sh.gx.end());
     sh.gx.erase(std::unique(sh.gx.begin(), sh.gx.end()), sh.gx.end());
   }
-  // forward shared slots no forward term and no adjoint set point reads
-  sh.gf.sink.assign(sh.gf.nl(), 0);
-  for (uint32_t r = sh.gf.RL; r < sh.gf.nl(); ++r) sh.gf.sink[r] = 1;
+  // forward slots no forward term and no adjoint set point reads, adjoint
+  // slots no adjoint term reads
+  sh.gf.sink.assign(sh.gf.nl(), 1);
   for (const GRow& row : sh.gf.rows)
     for (const GTerm& t : row.terms)
-      for (uint32_t a = 0; a <= t.kind; ++a)
-        if (t.f[a].shared) sh.gf.sink[t.f[a].slot] = 0;
-  for (const GSrc& x : sh.gx)
-    if (x.shared) sh.gf.sink[x.slot] = 0;
-  sh.ga.sink.assign(sh.ga.nl(), 0);
+      for (uint32_t a = 0; a <= t.kind; ++a) sh.gf.sink[t.f[a].slot] = 0;
+  for (const GSrc& x : sh.gx) sh.gf.sink[x.slot] = 0;
+  sh.ga.sink.assign(sh.ga.nl(), 1);
+  for (const GRow& row : sh.ga.rows)
+    for (const GTerm& t : row.terms) sh.ga.sink[t.f[0].slot] = 0;
   sh.group = G;
   return true;
 }
@@ -673,37 +673,65 @@ __device__ __forceinline__ R interp_at(const R* e, u32 b, GP(const R) wts, u32 W
   return fmaR(wts[W + j], ei, wts[j] * ei1) * keep;
 }
 
-// one RK4 step of N rows; rhs(k, y, stage).  ALL: every lane is active.
-// K::sink(r): row r is a shared row that no term reads; rhs leaves its
-// group-partial slope in k[r], which is accumulated per lane over the four
-// stages and summed across the group (K::G lanes) once per step.
-struct NoSink {
-  static constexpr unsigned G = 1;
-  static __device__ __forceinline__ constexpr bool sink(int) { return false; }
-};
+// One RK4 step of N rows; rhs(k, y, stage).  ALL: every lane is active.
+// Three kinds of row need less than a slope per stage:
+//   K::sink(r)  no term reads the row (energy probes): rhs adds its terms onto
+//               k[r], which runs through the stages of equal weight (1 and 4,
+//               2 and 3), so a term's multiply-add is its accumulation.  On a
+//               group the row is shared and each lane keeps its own part of
+//               it, summed (K::G lanes) where the row is output.
+//   K::lin(r)   a single linear term c y_j: rhs hands back k[r] = y_j and the
+//               coefficient rides on the step constants hl[lin] = {h2 c, h c,
+//               h6 c} (a product less per stage, and one less in the chain).
+//   K::zero(r)  no terms at all: the row keeps its value.
 template <int N, bool ALL, class K, class F>
-__device__ __forceinline__ void rk4(R* q, F rhs, R h, R h2, R h6, bool active) {
+__device__ __forceinline__ void rk4(R* q, F rhs, const R (*hl)[3], R h, R h2, R h6, bool active) {
   R y[N], k[N], acc[N];
 #pragma unroll
-  for (int r = 0; r < N; ++r) y[r] = q[r];
+  for (int r = 0; r < N; ++r) {
+    y[r] = q[r];
+    k[r] = R(0);
+  }
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+      if (K::sink(r)) {
+        if (s == 1) {
+          acc[r] = k[r];
+          k[r] = R(0);
+        } else if (s == 3) {
+          const R mid = k[r];
+          k[r] = acc[r];
+          acc[r] = mid;
+        }
+      }
     rhs(k, y, s);
 #pragma unroll
     for (int r = 0; r < N; ++r) {
+      if (K::zero(r)) continue;
+      if (K::sink(r)) {
+        if (s == 3) {
+          const R qn = fmaR(h6, fmaR(R(2), acc[r], k[r]), q[r]);
+          q[r] = (ALL || active) ? qn : q[r];
+        }
+        continue;
+      }
+      const R s2 = K::lin(r) >= 0 ? hl[K::lin(r)][0] : h2;
+      const R s1 = K::lin(r) >= 0 ? hl[K::lin(r)][1] : h;
+      const R s6 = K::lin(r) >= 0 ? hl[K::lin(r)][2] : h6;
       if (s == 0) {
         acc[r] = k[r];
-        if (!K::sink(r)) y[r] = fmaR(h2, k[r], q[r]);
+        y[r] = fmaR(s2, k[r], q[r]);
       } else if (s == 1) {
         acc[r] = fmaR(R(2), k[r], acc[r]);
-        if (!K::sink(r)) y[r] = fmaR(h2, k[r], q[r]);
+        y[r] = fmaR(s2, k[r], q[r]);
       } else if (s == 2) {
         acc[r] = fmaR(R(2), k[r], acc[r]);
-        if (!K::sink(r)) y[r] = fmaR(h, k[r], q[r]);
+        y[r] = fmaR(s1, k[r], q[r]);
       } else {
         acc[r] = acc[r] + k[r];
-        if (K::sink(r)) acc[r] = gsum<K::G>(acc[r]);
-        const R qn = fmaR(h6, acc[r], q[r]);
+        const R qn = fmaR(s6, acc[r], q[r]);
         q[r] = (ALL || active) ? qn : q[r];
       }
     }
@@ -711,34 +739,109 @@ __device__ __forceinline__ void rk4(R* q, F rhs, R h, R h2, R h6, bool active) {
 }
 
 // rk4 that hands the inputs of stages 2..4 to rec(s, y) before evaluating
-// them (the exact discrete adjoint's recompute keeps them)
+// them (the exact discrete adjoint's recompute keeps them); sinks keep their
+// value (a recompute does not need them)
 template <int N, bool ALL, class K, class F, class Rec>
-__device__ __forceinline__ void rk4rec(R* q, F rhs, Rec rec, R h, R h2, R h6, bool active) {
-  R y[N], k[N], acc[N];
-#pragma unroll
-  for (int r = 0; r < N; ++r) y[r] = q[r];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
+__device__ __forceinline__ void rk4rec(R* q, F rhs, Rec rec, const R (*hl)[3], R h, R h2, R h6,
+                                       bool active) {
+  rk4<N, ALL, K>(q, [&](R* k, const R* y, int s) {
     if (s > 0) rec(s, y);
     rhs(k, y, s);
+  }, hl, h, h2, h6, active);
+}
+
+// One reverse step of N adjoint rows of class S, reference recursion:
+// eff(e, set point) evaluates the effective coefficients at x_n (0), the
+// midpoint (1, stages 2 and 3) and x_{n-1} (2).  Rows no adjoint term reads
+// (gradient accumulators; S::sink_a) are quadratures: their effective
+// coefficients are those of the two middle stages once, times y2 + y3.
+template <int N, bool ALL, class S, class E>
+__device__ __forceinline__ void rk4_adj(R* lam, E eff, R h, R h2, R h6, bool active) {
+  R y[N], k[N], acc[N], sa[N], ym[N], e[S::NE > 0 ? S::NE : 1];
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    y[r] = lam[r];
+    sa[r] = R(0);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    if (s != 2) eff(e, s == 0 ? 0 : (s == 1 ? 1 : 2));
+    S::lin_a(k, y, e);
+    if (s == 0 || s == 3) S::quad_a(sa, y, e);
 #pragma unroll
     for (int r = 0; r < N; ++r) {
+      if (s == 1) ym[r] = y[r];
+      else if (s == 2) ym[r] = R(2) * (ym[r] + y[r]);
+    }
+    if (s == 2) S::quad_a(sa, ym, e);
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      if (S::zero_a(r)) continue;
+      if (S::sink_a(r)) {
+        if (s == 3) {
+          const R ln = fmaR(h6, sa[r], lam[r]);
+          lam[r] = (ALL || active) ? ln : lam[r];
+        }
+        continue;
+      }
       if (s == 0) {
         acc[r] = k[r];
-        if (!K::sink(r)) y[r] = fmaR(h2, k[r], q[r]);
+        y[r] = fmaR(h2, k[r], lam[r]);
       } else if (s == 1) {
         acc[r] = fmaR(R(2), k[r], acc[r]);
-        if (!K::sink(r)) y[r] = fmaR(h2, k[r], q[r]);
+        y[r] = fmaR(h2, k[r], lam[r]);
       } else if (s == 2) {
         acc[r] = fmaR(R(2), k[r], acc[r]);
-        if (!K::sink(r)) y[r] = fmaR(h, k[r], q[r]);
+        y[r] = fmaR(h, k[r], lam[r]);
       } else {
         acc[r] = acc[r] + k[r];
-        if (K::sink(r)) acc[r] = gsum<K::G>(acc[r]);
-        const R qn = fmaR(h6, acc[r], q[r]);
-        q[r] = (ALL || active) ? qn : q[r];
+        const R ln = fmaR(h6, acc[r], lam[r]);
+        lam[r] = (ALL || active) ? ln : lam[r];
       }
     }
+  }
+}
+
+// One reverse step of the exact discrete adjoint of step n-1 -> n from its
+// stage inputs y1 (the post-step state of step n-1) .. y4, handed out by
+// at(s, x) for s = 4, 3, 2, 1:
+//   a4 = h6 lam,            mu4 = g(a4, y4)
+//   a3 = 2 h6 lam + h mu4,  mu3 = g(a3, y3)
+//   a2 = 2 h6 lam + h2 mu3, mu2 = g(a2, y2)
+//   a1 = h6 lam + h2 mu2,   mu1 = g(a1, y1)
+//   lam += ((mu4 + mu3) + mu2) + mu1
+template <int N, bool ALL, class S, class E>
+__device__ __forceinline__ void exact_adj(R* lam, E eff, R h, R h2, R h6, bool active) {
+  R av[N], mu[N], ac[N], e[S::NE > 0 ? S::NE : 1];
+  const R h3 = R(2) * h6;
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    av[r] = h6 * lam[r];
+    ac[r] = R(0);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    eff(e, s);
+    S::lin_a(mu, av, e);
+    S::quad_a(ac, av, e);
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      if (S::sink_a(r) || S::zero_a(r)) {
+        // av of a row without terms: the next stage's multiple of lam
+        if (s < 3) av[r] = (s < 2 ? h3 : h6) * lam[r];
+        continue;
+      }
+      ac[r] = s == 0 ? mu[r] : ac[r] + mu[r];
+      if (s == 0) av[r] = fmaR(h, mu[r], h3 * lam[r]);
+      else if (s == 1) av[r] = fmaR(h2, mu[r], h3 * lam[r]);
+      else if (s == 2) av[r] = fmaR(h2, mu[r], h6 * lam[r]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    if (S::zero_a(r)) continue;
+    const R ln = lam[r] + ac[r];
+    lam[r] = (ALL || active) ? ln : lam[r];
   }
 }
 
@@ -825,6 +928,12 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   auto orow_a = [&](int r) -> int {
     return r < S::RLA ? S::rowa(r) + (int)p * S::stridea(r) : (p == 0u ? S::rowa(r) : -1);
   };
+  // a shared sink is the sum of its lanes' parts (whole groups reach this);
+  // the row's value at the start belongs to position 0
+  auto fval = [](int r, R v) -> R { return r >= S::RLF && S::sink(r) ? gsum<G>(v) : v; };
+  auto aval = [](int r, R v) -> R { return r >= S::RLA && S::sink_a(r) ? gsum<G>(v) : v; };
+  auto finit = [&](int r) -> R { return r >= S::RLF && S::sink(r) && p != 0u ? R(0) : qi[r * st]; };
+  auto ainit = [&](int r) -> R { return r >= S::RLA && S::sink_a(r) && p != 0u ? R(0) : li[r * st]; };
 
   R q[NF], mx[NF], lam[NA];
 #pragma unroll
@@ -833,11 +942,13 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   for (int r = 0; r < NA; ++r) lam[r] = R(0);
   if (n == 0u && phase == kForward) {
 #pragma unroll
-    for (int r = 0; r < NF; ++r) q[r] = qi[r * st];
+    for (int r = 0; r < NF; ++r) q[r] = finit(r);
     if (fsteps == 0u && valid)
 #pragma unroll
-      for (int r = 0; r < NF; ++r)
-        if (orow_f(r) >= 0) outq[fout + orow_f(r)] = q[r];
+      for (int r = 0; r < NF; ++r) {
+        const R v = fval(r, q[r]);
+        if (orow_f(r) >= 0) outq[fout + orow_f(r)] = v;
+      }
   } else {
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
@@ -872,10 +983,18 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       R pre[NPF];
       fetch_g<G, NPF>(pre, E, Lx, pbase, p);
       bool have = true;
+      R hl[S::NLIN > 0 ? S::NLIN : 1][3];
       // the phase's loads land here: no wait for them inside the step loops,
       // where the in-order load counter would also hold back the prefetched
       // samples of the next chunk
       __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+      for (int r = 0; r < NF; ++r)
+        if (S::lin(r) >= 0) {
+          hl[S::lin(r)][0] = h2 * c[S::linc(r)];
+          hl[S::lin(r)][1] = h * c[S::linc(r)];
+          hl[S::lin(r)][2] = h6 * c[S::linc(r)];
+        }
       if (recompute) {
         if (n == s0) {
 #pragma unroll
@@ -940,22 +1059,21 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
             for (int r = 0; r < NF; ++r) ck[((u64)(n / K) * NF + r) * WAVE] = q[r];
             next_ck += K;
           }
+          auto rhs = [&](R* k, const R* y, int s) {
+            S::template rhs_f<MODE != mRec>(k, y, c, s == 0 ? u0 : (s == 3 ? u3 : u1));
+          };
           if constexpr (EX && MODE == mRec) {
             const u32 mb = 3u * (n - s0);
-            rk4rec<NF, ALL, S>(q, [&](R* k, const R* y, int s) {
-              S::rhs_f(k, y, c, s == 0 ? u0 : (s == 3 ? u3 : u1));
-            }, [&](int s, const R* y) {
+            rk4rec<NF, ALL, S>(q, rhs, [&](int s, const R* y) {
               const u32 m = mb + (u32)(s - 1);
 #pragma unroll
               for (int r = 0; r < NF; ++r) {
                 if (S::segr(r) >= 0) seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = y[r];
                 if (mirror) sb3[((u64)m * NF + r) * st] = y[r];
               }
-            }, h, h2, h6, n < fsteps);
+            }, hl, h, h2, h6, n < fsteps);
           } else {
-            rk4<NF, ALL, S>(q, [&](R* k, const R* y, int s) {
-              S::rhs_f(k, y, c, s == 0 ? u0 : (s == 3 ? u3 : u1));
-            }, h, h2, h6, n < fsteps);
+            rk4<NF, ALL, S>(q, rhs, hl, h, h2, h6, n < fsteps);
           }
           if constexpr (MODE == mRec) {
             const u32 m = n + 1u - s0;
@@ -971,18 +1089,21 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
                 const u32 slot = n / SE;
                 if (slot < (u32)a.nslots && valid)
 #pragma unroll
-                  for (int r = 0; r < NF; ++r)
-                    if (orow_f(r) >= 0) traj[(u64)slot * a.out_len + fout + orow_f(r)] = q[r];
+                  for (int r = 0; r < NF; ++r) {
+                    const R v = fval(r, q[r]);
+                    if (orow_f(r) >= 0) traj[(u64)slot * a.out_len + fout + orow_f(r)] = v;
+                  }
                 next_save += SE;
               }
               if (a.window && (ALL || n < fsteps) && n + 1u + (u32)a.window > fsteps)
 #pragma unroll
-                for (int r = 0; r < NF; ++r) mx[r] = fmaxR(mx[r], absR(q[r]));
+                for (int r = 0; r < NF; ++r) mx[r] = fmaxR(mx[r], absR(fval(r, q[r])));
               if (n + 1u == fsteps && valid) {
 #pragma unroll
                 for (int r = 0; r < NF; ++r) {
+                  const R v = fval(r, q[r]);
                   if (orow_f(r) < 0) continue;
-                  outq[fout + orow_f(r)] = q[r];
+                  outq[fout + orow_f(r)] = v;
                   if (a.window) outm[fout + orow_f(r)] = mx[r];
                 }
               }
@@ -1062,14 +1183,18 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       // range kept its final state since (inactive steps leave it)
       if ((mode == mPlain || mode == mCk) && valid && fsteps > nfirst && fsteps <= nend)
 #pragma unroll
-        for (int r = 0; r < NF; ++r)
-          if (orow_f(r) >= 0) outq[fout + orow_f(r)] = q[r];
+        for (int r = 0; r < NF; ++r) {
+          const R v = fval(r, q[r]);
+          if (orow_f(r) >= 0) outq[fout + orow_f(r)] = v;
+        }
       if (n == e && !recompute && SE && valid) {
         // trajectory slots after the wave's last step hold the final state
         for (u32 slot = (T + SE - 1u) / SE; slot < (u32)a.nslots; ++slot)
 #pragma unroll
-          for (int r = 0; r < NF; ++r)
-            if (orow_f(r) >= 0) traj[(u64)slot * a.out_len + fout + orow_f(r)] = q[r];
+          for (int r = 0; r < NF; ++r) {
+            const R v = fval(r, q[r]);
+            if (orow_f(r) >= 0) traj[(u64)slot * a.out_len + fout + orow_f(r)] = v;
+          }
       }
       if (n == e) {
         if (recompute) {
@@ -1079,7 +1204,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           n = sg * K;
           phase = kRecompute;
 #pragma unroll
-          for (int r = 0; r < NA; ++r) lam[r] = li[r * st];
+          for (int r = 0; r < NA; ++r) lam[r] = ainit(r);
         } else {
           phase = kDone;
           if (adjoint && valid)
@@ -1114,66 +1239,21 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         constexpr bool ALL = decltype(all_t)::value;
         for (; n > stop; --n) {
           if constexpr (EX) {
-            // exact discrete adjoint of step n-1 -> n from its stage inputs
-            // y1 (the post-step state of step n-1) .. y4:
-            //   a4 = h6 lam,            mu4 = g(a4, y4)
-            //   a3 = 2 h6 lam + h mu4,  mu3 = g(a3, y3)
-            //   a2 = 2 h6 lam + h2 mu3, mu2 = g(a2, y2)
-            //   a1 = h6 lam + h2 mu2,   mu1 = g(a1, y1)
-            //   lam += ((mu4 + mu3) + mu2) + mu1
             R y1[NX], y2[NX], y3[NX], y4[NX];
             const u32 mb = 3u * (n - 1u - s0);
             S::xload(y4, y1, seg3 + (mb + 2u) * (NSEG * WAVE), seg + (n - 1u - s0) * (NSEG * WAVE), lane);
             S::xload(y3, y2, seg3 + (mb + 1u) * (NSEG * WAVE), seg3 + mb * (NSEG * WAVE), lane);
-            const R h3 = R(2) * h6;
-            R e[S::NE > 0 ? S::NE : 1];
-            R av[NA], mu[NA], ac[NA];
-#pragma unroll
-            for (int r = 0; r < NA; ++r) av[r] = h6 * lam[r];
-            S::eff_a(e, y4, c);
-            S::lin_a(mu, av, e);
-#pragma unroll
-            for (int r = 0; r < NA; ++r) {
-              ac[r] = mu[r];
-              av[r] = fmaR(h, mu[r], h3 * lam[r]);
-            }
-            S::eff_a(e, y3, c);
-            S::lin_a(mu, av, e);
-#pragma unroll
-            for (int r = 0; r < NA; ++r) {
-              ac[r] = ac[r] + mu[r];
-              av[r] = fmaR(h2, mu[r], h3 * lam[r]);
-            }
-            S::eff_a(e, y2, c);
-            S::lin_a(mu, av, e);
-#pragma unroll
-            for (int r = 0; r < NA; ++r) {
-              ac[r] = ac[r] + mu[r];
-              av[r] = fmaR(h2, mu[r], h6 * lam[r]);
-            }
-            S::eff_a(e, y1, c);
-            S::lin_a(mu, av, e);
-            const bool act = ALL || n <= fsteps;
-#pragma unroll
-            for (int r = 0; r < NA; ++r) {
-              ac[r] = ac[r] + mu[r];
-              const R ln = lam[r] + ac[r];
-              lam[r] = act ? ln : lam[r];
-            }
+            exact_adj<NA, ALL, S>(lam, [&](R* e, int s) {
+              S::eff_a(e, s == 0 ? y4 : (s == 1 ? y3 : (s == 2 ? y2 : y1)), c);
+            }, h, h2, h6, n <= fsteps);
             continue;
           }
           R xc[NX], xb[NX], xp[NX];
           S::xload(xc, xp, seg + (n - s0) * (NSEG * WAVE), seg + (n - 1u - s0) * (NSEG * WAVE), lane);
 #pragma unroll
           for (int j = 0; j < NX; ++j) xb[j] = R(0.5) * (xc[j] + xp[j]);
-          // effective coefficients per set point: x_n, the midpoint (stages
-          // 2 and 3), x_{n-1}
-          R e[S::NE > 0 ? S::NE : 1];
-          rk4<NA, ALL, NoSink>(lam, [&](R* k, const R* y, int s) {
-            if (s == 0) S::eff_a(e, xc, c);
-            else if (s == 1) S::eff_a(e, xb, c);
-            else if (s == 3) S::eff_a(e, xp, c);
-            S::lin_a(k, y, e);
+          rk4_adj<NA, ALL, S>(lam, [&](R* e, int s) {
+            S::eff_a(e, s == 0 ? xc : (s == 1 ? xb : xp), c);
           }, h, h2, h6, n <= fsteps);
         }
       };
@@ -1185,8 +1265,10 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           phase = kDone;
           if (valid)
 #pragma unroll
-            for (int r = 0; r < S::NA; ++r)
-              if (orow_a(r) >= 0 && (u32)orow_a(r) < nao) outg[aout + orow_a(r)] = lam[r];
+            for (int r = 0; r < S::NA; ++r) {
+              const R v = aval(r, lam[r]);
+              if (orow_a(r) >= 0 && (u32)orow_a(r) < nao) outg[aout + orow_a(r)] = v;
+            }
         } else {
           sg -= 1u;
           n = sg * K;
@@ -1673,47 +1755,159 @@ struct Monos {
   }
 };
 
-// Single-wave right-hand side: every row, coefficients c[global slot].
-void emit_rhs(std::ostringstream& o, const LaneSide& sd, bool forced_input, const char* S,
-              const char* X) {
-  const Slots sl = slots_of(sd);
-  const std::string sn(S), xn(X);
-  for (uint32_t r = 0; r < sd.n; ++r)
-    emit_row(o, sd, sl, r, r, forced_input,
-             [](uint32_t gs) { return "c[" + std::to_string(gs) + "]"; },
-             [&](uint32_t j) { return sn + "[" + std::to_string(j) + "]"; },
-             [&](uint32_t j) { return xn + "[" + std::to_string(j) + "]"; });
+// A sum of terms coef * f[0] * f[1] * ... (no factors: a constant).
+struct PTerm {
+  std::string coef;
+  std::vector<std::string> f;
+};
+// Expression of base + the sum of `ts` in factored form: the factor most
+// terms share is taken out, s * (rest of those terms) + the others, and both
+// parts are treated alike (Horner's scheme in several variables).  A term
+// costs about one multiply-add this way instead of a product per factor and
+// one to add it: the 16-DOF chain's velocity row takes 11 instead of 19.
+// These kernels issue vector instructions most of their cycles, so the step
+// time follows the count (with the row kinds of rk4 and rk4_adj): 4,096
+// two-DOF systems x 20,000 steps 4.53 -> 3.33 ms, 8,192 16-DOF chains x
+// 10,000 steps forward + adjoint 22.5 -> 17.8 ms.
+std::string factored(std::ostringstream& o, Monos& monos, const std::vector<PTerm>& ts,
+                     const std::string& base) {
+  std::map<std::string, size_t> count;
+  for (const PTerm& t : ts)
+    for (size_t a = 0; a < t.f.size(); ++a)
+      if (std::find(t.f.begin(), t.f.begin() + long(a), t.f[a]) == t.f.begin() + long(a))
+        ++count[t.f[a]];
+  std::string s;
+  size_t most = 1;
+  for (const auto& c : count)
+    if (c.second > most) {
+      most = c.second;
+      s = c.first;
+    }
+  if (s.empty()) {
+    std::string acc = base;
+    for (const PTerm& t : ts)  // constants first: what follows is added onto them
+      if (t.f.empty()) acc = acc.empty() ? t.coef : "(" + acc + " + " + t.coef + ")";
+    for (const PTerm& t : ts) {
+      if (t.f.empty()) continue;
+      const std::string m = monos.get(o, t.f, t.f.size());
+      acc = acc.empty() ? t.coef + " * " + m : "fmaR(" + t.coef + ", " + m + ", " + acc + ")";
+    }
+    return acc;
+  }
+  std::vector<PTerm> with, rest;
+  for (const PTerm& t : ts) {
+    auto it = std::find(t.f.begin(), t.f.end(), s);
+    if (it == t.f.end()) {
+      rest.push_back(t);
+    } else {
+      PTerm u = t;
+      u.f.erase(u.f.begin() + (it - t.f.begin()));
+      with.push_back(u);
+    }
+  }
+  const std::string r = factored(o, monos, rest, base);
+  const std::string q = factored(o, monos, with, "");
+  if (r.empty()) return "(" + q + ") * " + s;
+  return "fmaR(" + q + ", " + s + ", " + r + ")";
 }
 
-// Single-wave forward right-hand side with shared monomials: each kind
-// summed in term order (coefficient times the cached product of its state
-// factors), kinds added in order, then the force.
-void emit_rhs_forward(std::ostringstream& o, const LaneSide& sd) {
+// Kinds of a side's lane rows (rk4 / rk4_adj in the runtime).
+struct RowKinds {
+  std::vector<uint8_t> sink, zero;  // nothing reads the row; it has no terms
+  std::vector<int> lin, linc;       // single linear term: index, its coefficient slot
+  uint32_t nlin = 0;
+};
+
+// One row of a forward right-hand side: terms over state names, the force,
+// coefficients c[slot].
+void emit_forward_row(std::ostringstream& o, Monos& monos, const RowKinds& rk, uint32_t r,
+                      const std::vector<PTerm>& ts, const std::string& force,
+                      uint32_t gsum) {
+  const std::string kr = "k[" + std::to_string(r) + "]";
+  if (rk.zero[r]) return;
+  if (rk.lin[r] >= 0) {
+    o << "    " << kr << " = " << ts[0].f[0] << ";\n";
+    return;
+  }
+  std::string base = rk.sink[r] ? kr : "";
+  if (!force.empty())
+    base = base.empty() ? force + " * u" : "fmaR(" + force + ", u, " + base + ")";
+  std::ostringstream pre;
+  std::string e = factored(pre, monos, ts, base);
+  if (gsum > 1 && !rk.sink[r]) e = "gsum<" + std::to_string(gsum) + "u>(" + e + ")";
+  if (rk.sink[r])
+    o << "    if constexpr (SINKS) {\n" << pre.str() << "    " << kr << " = " << e << ";\n    }\n";
+  else
+    o << pre.str() << "    " << kr << " = " << e << ";\n";
+}
+
+// Forward right-hand side of a one-lane class.
+void emit_rhs_forward(std::ostringstream& o, const LaneSide& sd, const RowKinds& rk) {
   const Slots sl = slots_of(sd);
   Monos monos;
-  auto y = [](uint32_t j) { return "y[" + std::to_string(j) + "]"; };
-  for (uint32_t r = 0; r < sd.n; ++r) {
-    std::string k;
-    for (int kind = 0; kind < 4; ++kind) {
-      std::string acc;
+  // sinks last: the products they need are theirs alone or already there
+  for (int pass = 0; pass < 2; ++pass)
+    for (uint32_t r = 0; r < sd.n; ++r) {
+      if (int(rk.sink[r]) != pass) continue;
+      std::vector<PTerm> ts;
       uint32_t slot = sl.base[r];
       for (const LaneTerm& tm : sd.rows[r]) {
-        const std::string coef = "c[" + std::to_string(slot++) + "]";
-        if (int(tm.kind) != kind) continue;
-        std::vector<std::string> fs;
-        for (uint32_t a = 0; a <= tm.kind; ++a) fs.push_back(y(tm.f[a]));
-        const std::string m = monos.get(o, fs, fs.size());
-        const std::string prod = acc.empty() ? coef + " * " + m : "fmaR(" + coef + ", " + m + ", " + acc + ")";
-        const std::string name = "s" + std::to_string(kind) + "_" + std::to_string(r);
-        o << "    " << (acc.empty() ? "R " : "") << name << " = " << prod << ";\n";
-        acc = name;
+        PTerm t;
+        t.coef = "c[" + std::to_string(slot++) + "]";
+        for (uint32_t a = 0; a <= tm.kind; ++a) t.f.push_back("y[" + std::to_string(tm.f[a]) + "]");
+        std::sort(t.f.begin(), t.f.end());
+        ts.push_back(t);
       }
-      if (!acc.empty()) k = k.empty() ? acc : "(" + k + " + " + acc + ")";
+      emit_forward_row(o, monos, rk, r, ts,
+                       sl.force[r] >= 0 ? "c[" + std::to_string(sl.force[r]) + "]" : "", 1);
     }
-    if (k.empty()) k = "R(0)";
-    if (sl.force[r] >= 0) k = "fmaR(c[" + std::to_string(sl.force[r]) + "], u, " + k + ")";
-    o << "    k[" << r << "] = " << k << ";\n";
+}
+
+RowKinds one_lane_kinds(const LaneShape& sh, bool forward) {
+  const LaneSide& sd = forward ? sh.f : sh.a;
+  RowKinds rk;
+  rk.sink.assign(sd.n, 1);
+  rk.zero.assign(sd.n, 0);
+  rk.lin.assign(sd.n, -1);
+  rk.linc.assign(sd.n, 0);
+  for (const auto& row : sd.rows)
+    for (const LaneTerm& t : row)
+      for (uint32_t a = 0; a <= (forward ? t.kind : 0u); ++a) rk.sink[t.f[a]] = 0;
+  if (forward && sh.adjoint)
+    for (const auto& row : sh.a.rows)
+      for (const LaneTerm& t : row)
+        for (uint32_t a = 1; a <= t.kind; ++a) rk.sink[t.f[a]] = 0;
+  const Slots sl = slots_of(sd);
+  for (uint32_t r = 0; r < sd.n; ++r) {
+    const bool forced = sl.force[r] >= 0;
+    rk.zero[r] = sd.rows[r].empty() && !forced;
+    if (forward && !rk.sink[r] && !forced && sd.rows[r].size() == 1 && sd.rows[r][0].kind == 0) {
+      rk.lin[r] = int(rk.nlin++);
+      rk.linc[r] = int(sl.base[r]);
+    }
   }
+  return rk;
+}
+
+RowKinds group_kinds(const GSide& gs, bool forward) {
+  RowKinds rk;
+  rk.sink.assign(gs.nl(), 0);
+  rk.zero.assign(gs.nl(), 0);
+  rk.lin.assign(gs.nl(), -1);
+  rk.linc.assign(gs.nl(), 0);
+  uint32_t t = 0;
+  for (uint32_t r = 0; r < gs.nl(); ++r) {
+    const GRow& row = gs.rows[r];
+    rk.sink[r] = gs.sink[r];
+    rk.zero[r] = row.terms.empty() && row.force.empty();
+    if (forward && r < gs.RL && !rk.sink[r] && row.force.empty() && row.terms.size() == 1 &&
+        row.terms[0].kind == 0) {
+      rk.lin[r] = int(rk.nlin++);
+      rk.linc[r] = int(t);
+    }
+    t += uint32_t(row.terms.size()) + (row.force.empty() ? 0u : 1u);
+  }
+  return rk;
 }
 
 // One wave's rows of a side in a multi-wave class: its own coefficient
@@ -1758,43 +1952,45 @@ struct ERow {
   std::vector<ETerm> terms;
   bool shared = false;
 };
-void emit_adjoint_linear(std::ostringstream& oe, std::ostringstream& ol, const std::vector<ERow>& rows,
-                         uint32_t G, uint32_t* ne) {
+void emit_adjoint_linear(std::ostringstream& oe, std::ostringstream& ol, std::ostringstream& oq,
+                         const std::vector<ERow>& rows, const RowKinds& rk, uint32_t G,
+                         uint32_t* ne) {
   uint32_t j = 0;
+  Monos monos;
   for (size_t r = 0; r < rows.size(); ++r) {
     std::vector<std::string> owns;
-    std::vector<std::string> effs;
+    std::vector<std::vector<PTerm>> effs;
     for (const ETerm& t : rows[r].terms) {
       size_t o = 0;
       while (o < owns.size() && owns[o] != t.own) ++o;
       if (o == owns.size()) {
         owns.push_back(t.own);
-        effs.push_back("");
+        effs.emplace_back();
       }
-      const std::string c = "c[" + std::to_string(t.coef) + "]";
-      std::string& e = effs[o];
-      if (t.kind == 0) {
-        e = e.empty() ? c : "(" + e + " + " + c + ")";
-      } else {
-        std::string l = c;
-        for (uint32_t f = 0; f + 1 < t.kind; ++f) l = "(" + l + ") * " + t.xs[f];
-        const std::string last = t.xs[t.kind - 1];
-        e = e.empty() ? "(" + l + ") * " + last : "fmaR(" + l + ", " + last + ", " + e + ")";
-      }
+      PTerm pt;
+      pt.coef = "c[" + std::to_string(t.coef) + "]";
+      pt.f = t.xs;
+      std::sort(pt.f.begin(), pt.f.end());
+      effs[o].push_back(pt);
     }
-    std::string k;
+    const std::string kr = "k[" + std::to_string(r) + "]";
+    std::string k = rk.sink[r] ? kr : "";
     for (size_t o = 0; o < owns.size(); ++o) {
-      oe << "    e[" << j << "] = " << effs[o] << ";\n";
+      const std::string ex = factored(oe, monos, effs[o], "");
+      oe << "    e[" << j << "] = " << ex << ";\n";
       const std::string ej = "e[" + std::to_string(j) + "]";
       k = k.empty() ? ej + " * " + owns[o] : "fmaR(" + ej + ", " + owns[o] + ", " + k + ")";
       ++j;
     }
-    if (k.empty()) {
-      k = "R(0)";
-    } else if (rows[r].shared && G > 1) {
-      k = "gsum<" + std::to_string(G) + "u>(" + k + ")";
+    if (rk.zero[r]) continue;
+    // a sink's terms are added where rk4_adj keeps its running sum; on a
+    // group every lane keeps its part of a shared one
+    if (rk.sink[r]) {
+      oq << "    " << kr << " = " << k << ";\n";
+    } else {
+      if (rows[r].shared && G > 1) k = "gsum<" + std::to_string(G) + "u>(" + k + ")";
+      ol << "    " << kr << " = " << k << ";\n";
     }
-    ol << "    k[" << r << "] = " << k << ";\n";
   }
   *ne = j;
 }
@@ -1842,17 +2038,16 @@ std::vector<ERow> lane_adjoint_rows(const LaneSide& sd) {
   return rows;
 }
 
-// Right-hand side of one side of a lane-group class: the own-state values
-// the program reads from other positions of the group (rotated once per
-// stage), then every lane slot: band slots directly, shared slots as
-// partial sums added across the group.  Coefficients c[t] in per-lane slot
-// order (row by row, terms then force); set points x[j] index `gx`.
-void emit_group_side(std::ostringstream& o, const GSide& gs, uint32_t G, bool forward,
-                     const std::vector<GSrc>& gx) {
+// Forward right-hand side of a lane-group class: the values the program
+// reads from other positions of the group (rotated once per stage), then
+// every lane slot: band slots directly, shared slots as partial sums added
+// across the group (a sink's stay apart: rk4).  Coefficients c[t] in per-lane
+// slot order (row by row, terms then force).
+void emit_group_forward(std::ostringstream& o, const GSide& gs, uint32_t G, const RowKinds& rk) {
   std::vector<GSrc> rem;
   for (const GRow& row : gs.rows)
     for (const GTerm& t : row.terms)
-      for (uint32_t a = 0; a <= (forward ? t.kind : 0u); ++a)
+      for (uint32_t a = 0; a <= t.kind; ++a)
         if (!t.f[a].shared && t.f[a].d != 0) rem.push_back(t.f[a]);
   std::sort(rem.begin(), rem.end());
   rem.erase(std::unique(rem.begin(), rem.end()), rem.end());
@@ -1863,52 +2058,27 @@ void emit_group_side(std::ostringstream& o, const GSide& gs, uint32_t G, bool fo
     return (r.shared || r.d == 0) ? "y[" + std::to_string(r.slot) + "]"
                                   : "y" + std::to_string(r.slot) + "_" + std::to_string(r.d);
   };
-  auto X = [&](const GSrc& r) {
-    if (forward) return S(r);
-    const size_t j = size_t(std::lower_bound(gx.begin(), gx.end(), r) - gx.begin());
-    return "x[" + std::to_string(j) + "]";
-  };
   Monos monos;
-  uint32_t t = 0;
-  for (uint32_t r = 0; r < gs.nl(); ++r) {
-    const GRow& row = gs.rows[r];
-    std::string k;
-    for (int kind = 0; kind < 4; ++kind) {
-      std::string acc;
-      for (size_t e = 0; e < row.terms.size(); ++e) {
-        const GTerm& tm = row.terms[e];
-        if (int(tm.kind) != kind) continue;
-        const std::string coef = "c[" + std::to_string(t + e) + "]";
-        std::string prod;
-        if (kind == 0) {
-          prod = acc.empty() ? coef + " * " + S(tm.f[0])
-                             : "fmaR(" + coef + ", " + S(tm.f[0]) + ", " + acc + ")";
-        } else if (forward) {
-          std::vector<std::string> fs{S(tm.f[0])};
-          for (int f = 1; f <= kind; ++f) fs.push_back(X(tm.f[f]));
-          const std::string m = monos.get(o, fs, fs.size());
-          prod = acc.empty() ? coef + " * " + m : "fmaR(" + coef + ", " + m + ", " + acc + ")";
-        } else {
-          std::string l = coef + " * " + S(tm.f[0]);
-          for (int f = 1; f < kind; ++f) l = "(" + l + ") * " + X(tm.f[f]);
-          const std::string last = X(tm.f[kind]);
-          prod = acc.empty() ? "(" + l + ") * " + last : "fmaR(" + l + ", " + last + ", " + acc + ")";
+  for (int pass = 0; pass < 2; ++pass) {
+    uint32_t t = 0;
+    for (uint32_t r = 0; r < gs.nl(); ++r) {
+      const GRow& row = gs.rows[r];
+      const uint32_t tf = t + uint32_t(row.terms.size());
+      if (int(rk.sink[r]) == pass) {
+        std::vector<PTerm> ts;
+        for (size_t e = 0; e < row.terms.size(); ++e) {
+          PTerm pt;
+          pt.coef = "c[" + std::to_string(t + e) + "]";
+          for (uint32_t a = 0; a <= row.terms[e].kind; ++a) pt.f.push_back(S(row.terms[e].f[a]));
+          std::sort(pt.f.begin(), pt.f.end());
+          ts.push_back(pt);
         }
-        const std::string name = "s" + std::to_string(kind) + "_" + std::to_string(r);
-        o << "    " << (acc.empty() ? "R " : "") << name << " = " << prod << ";\n";
-        acc = name;
+        emit_forward_row(o, monos, rk, r, ts,
+                         row.force.empty() ? "" : "c[" + std::to_string(tf) + "]",
+                         r >= gs.RL ? G : 1u);
       }
-      if (!acc.empty()) k = k.empty() ? acc : "(" + k + " + " + acc + ")";
+      t = tf + (row.force.empty() ? 0u : 1u);
     }
-    const bool empty = k.empty() && (!forward || row.force.empty());
-    const bool sink = r < gs.sink.size() && gs.sink[r];
-    if (k.empty()) k = "R(0)";
-    const uint32_t tf = t + uint32_t(row.terms.size());
-    if (forward && !row.force.empty()) k = "fmaR(c[" + std::to_string(tf) + "], u, " + k + ")";
-    // a sink's partial slope is summed across the group once per step (rk4)
-    if (r >= gs.RL && G > 1 && !empty && !sink) k = "gsum<" + std::to_string(G) + "u>(" + k + ")";
-    o << "    k[" << r << "] = " << k << ";\n";
-    t = tf + (row.force.empty() ? 0u : 1u);
   }
 }
 
@@ -2140,7 +2310,12 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
       << ", RLF = " << (grp ? sh.gf.RL : nf) << ", RLA = " << (grp ? sh.ga.RL : na)
       << ", NX = " << (grp ? uint32_t(sh.gx.size()) : nf);
     std::vector<int> segmap;
-    if (!mw) o << ", NSEG = " << lane_seg_rows(sh, &segmap);
+    RowKinds kf, ka;
+    if (!mw) {
+      kf = grp ? group_kinds(sh.gf, true) : one_lane_kinds(sh, true);
+      if (sh.adjoint) ka = grp ? group_kinds(sh.ga, false) : one_lane_kinds(sh, false);
+      o << ", NSEG = " << lane_seg_rows(sh, &segmap) << ", NLIN = " << kf.nlin;
+    }
     o << " };\n";
     if (!mw) {
       o << "  static __device__ __forceinline__ constexpr int segr(int r) { return "
@@ -2159,21 +2334,31 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
           << ternary_map(sh.gf.stride) << "; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridea(int r) { return "
           << ternary_map(sh.ga.stride) << "; }\n";
-        std::string sk = "false";
-        for (uint32_t r = 0; r < sh.gf.sink.size(); ++r)
-          if (sh.gf.sink[r]) sk = "r == " + std::to_string(r) + " || " + sk;
-        o << "  static __device__ __forceinline__ constexpr bool sink(int r) { return " << sk
-          << "; }\n";
       } else {
         o << "  static __device__ __forceinline__ constexpr int rowf(int r) { return r; }\n";
         o << "  static __device__ __forceinline__ constexpr int rowa(int r) { return r; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridef(int) { return 1; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridea(int) { return 1; }\n";
-        o << "  static __device__ __forceinline__ constexpr bool sink(int) { return false; }\n";
       }
-      o << "  static __device__ __forceinline__ void rhs_f(R* k, const R* y, const R* c, R u) {\n";
-      if (grp) emit_group_side(o, sh.gf, G, true, sh.gx);
-      else emit_rhs_forward(o, sh.f);
+      auto rows_of = [&](const char* name, const std::vector<uint8_t>& v) {
+        std::string e = "false";
+        for (uint32_t r = uint32_t(v.size()); r-- > 0;)
+          if (v[r]) e = "r == " + std::to_string(r) + " || " + e;
+        o << "  static __device__ __forceinline__ constexpr bool " << name << "(int r) { return "
+          << e << "; }\n";
+      };
+      rows_of("sink", kf.sink);
+      rows_of("zero", kf.zero);
+      rows_of("sink_a", ka.sink);
+      rows_of("zero_a", ka.zero);
+      o << "  static __device__ __forceinline__ constexpr int lin(int r) { return "
+        << ternary_map_i(kf.lin) << "; }\n";
+      o << "  static __device__ __forceinline__ constexpr int linc(int r) { return "
+        << ternary_map_i(kf.linc) << "; }\n";
+      o << "  template <bool SINKS>\n"
+           "  static __device__ __forceinline__ void rhs_f(R* k, const R* y, const R* c, R u) {\n";
+      if (grp) emit_group_forward(o, sh.gf, G, kf);
+      else emit_rhs_forward(o, sh.f, kf);
       o << "  }\n";
       // set points of the reverse step: forward values read from the
       // segment in LDS (another position's column for rotated sources)
@@ -2206,31 +2391,34 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
         }
       }
       o << "  }\n";
-      std::ostringstream oe, ol;
+      std::ostringstream oe, ol, oq;
       uint32_t ne = 0;
       if (sh.adjoint) {
         const std::vector<ERow> rows = grp ? group_adjoint_rows(sh.ga, sh.gx) : lane_adjoint_rows(sh.a);
         if (grp) {
           // own-state values of other positions, rotated once per stage
-          std::vector<GSrc> rem;
-          for (const GRow& row : sh.ga.rows)
-            for (const GTerm& t : row.terms)
-              if (!t.f[0].shared && t.f[0].d != 0) rem.push_back(t.f[0]);
-          std::sort(rem.begin(), rem.end());
-          rem.erase(std::unique(rem.begin(), rem.end()), rem.end());
-          for (const GSrc& r : rem)
-            ol << "    const R y" << r.slot << "_" << r.d << " = rot<" << G << "u, " << r.d
-               << "u>(y[" << r.slot << "]);\n";
+          for (int pass = 0; pass < 2; ++pass) {
+            std::vector<GSrc> rem;
+            for (uint32_t r = 0; r < sh.ga.nl(); ++r)
+              if (int(ka.sink[r]) == pass)
+                for (const GTerm& t : sh.ga.rows[r].terms)
+                  if (!t.f[0].shared && t.f[0].d != 0) rem.push_back(t.f[0]);
+            std::sort(rem.begin(), rem.end());
+            rem.erase(std::unique(rem.begin(), rem.end()), rem.end());
+            for (const GSrc& r : rem)
+              (pass ? oq : ol) << "    const R y" << r.slot << "_" << r.d << " = rot<" << G << "u, "
+                               << r.d << "u>(y[" << r.slot << "]);\n";
+          }
         }
-        std::ostringstream ol2;
-        emit_adjoint_linear(oe, ol2, rows, G, &ne);
-        ol << ol2.str();
+        emit_adjoint_linear(oe, ol, oq, rows, ka, G, &ne);
       }
       o << "  enum { NE = " << ne << " };\n";
       o << "  static __device__ __forceinline__ void eff_a(R* e, const R* x, const R* c) {\n"
         << oe.str() << "  }\n";
       o << "  static __device__ __forceinline__ void lin_a(R* k, const R* y, const R* e) {\n"
         << ol.str() << "  }\n";
+      o << "  static __device__ __forceinline__ void quad_a(R* k, const R* y, const R* e) {\n"
+        << oq.str() << "  }\n";
     }
     o << "};\n";
     if (!mw) continue;
