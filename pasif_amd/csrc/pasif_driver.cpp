@@ -186,6 +186,10 @@ struct LaneCls {
   // single-wave adjoint: checkpoint elements, each wave's block sized by its
   // longest instance (offsets in ckoff)
   uint64_t ck_elems = 0;
+  // stored path of every wave: elements, and what one forward step of a wave
+  // costs against its bytes (path_plan)
+  uint64_t path_elems = 0;
+  double fwd_cost = 0;
   // the longest instance of each workgroup (instances are sorted by step
   // count, descending, so this is its first; 0 past the last instance) and
   // the workgroups a pool tick still launches: a prefix, since a workgroup
@@ -195,7 +199,7 @@ struct LaneCls {
   // program arrays: views into the part's one program buffer
   const void *coef_f = nullptr, *coef_a = nullptr, *init_f = nullptr, *init_a = nullptr,
              *steps = nullptr, *exc = nullptr, *out_f = nullptr, *out_a = nullptr,
-             *na_out = nullptr, *ckoff = nullptr;
+             *na_out = nullptr, *ckoff = nullptr, *pathoff = nullptr;
   DevBuf qstate, lstate, mxstate, progress, ckpt, segbuf;  // run
 };
 
@@ -595,6 +599,23 @@ struct PathPool {
     for (const Buf& x : bufs)
       if (x.dev == dev && !x.busy) b += x.bytes;
     return b;
+  }
+  // bytes a lease could get now
+  size_t limit(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    size_t busy = 0, spare = 0, largest = 0, f = 0, t = 0;
+    for (const Buf& x : bufs) {
+      if (x.dev != dev) continue;
+      if (x.busy) {
+        busy += x.bytes;
+      } else {
+        spare += x.bytes;
+        largest = std::max(largest, x.bytes);
+      }
+    }
+    if (hipMemGetInfo(&f, &t) != hipSuccess) return largest;
+    const size_t cap = size_t(32) << 30;
+    return std::max(largest, std::min((f + spare) / 4, busy < cap ? cap - busy : 0));
   }
   void* take(int dev, size_t bytes) {
     std::lock_guard<std::mutex> lk(mu);
@@ -2383,6 +2404,8 @@ bool lane_plan(pasif_driver* d, bool adjoint) {
     LaneLayout lay;
     lay.ilp = waves <= device_simds(d->dev);
     lay.exact = exact;
+    // an interval of the caller's choice keeps its checkpoints
+    lay.store = adjoint && !exact && d->ck_every == 0;
     const uint32_t by_waves =
         uint32_t(std::min(8.0, std::max(1.0, std::ceil(waves / device_simds(d->dev)))));
     const size_t m0 = mods.size();
@@ -2592,7 +2615,7 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
   const uint32_t out_len_a = adjoint ? (d->mapped ? d->adj.n : d->adj.n * d->n_exc) : 0;
   // classes and their fields' places
   struct Fields {
-    size_t cf, ca, qf, qa, stp, ex, of, oa, na, ck;
+    size_t cf, ca, qf, qa, stp, ex, of, oa, na, ck, pt;
   };
   std::vector<Fields> fld(shapes.size());
   for (size_t c = 0; c < shapes.size(); ++c) {
@@ -2632,6 +2655,7 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
     const uint32_t TA = adjoint ? (grp ? sh.ga.coefs() : sh.a.coefs()) : 0;
     Fields& f = fld[c];
     f.ck = (adjoint && lay.waves == 1) ? place(&L->ckoff, L->waves * sizeof(uint64_t)) : 0;
+    f.pt = lay.store ? place(&L->pathoff, L->waves * sizeof(uint64_t)) : 0;
     f.cf = place(&L->coef_f, size_t(std::max<uint32_t>(TF, 1)) * st * sizeof(R));
     f.ca = place(&L->coef_a, size_t(std::max<uint32_t>(TA, 1)) * st * sizeof(R));
     f.qf = place(&L->init_f, size_t(L->nf) * st * sizeof(R));
@@ -2773,6 +2797,17 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
         tot += uint64_t(std::max<uint32_t>(1, (Tw + L->seg - 1) / L->seg)) * L->nf * kLaneWave;
       }
       L->ck_elems = tot;
+      if (lay.store) {
+        uint64_t* po = reinterpret_cast<uint64_t*>(host.data() + f.pt);
+        const uint64_t rows = lane_seg_rows(sh);
+        uint64_t pt = 0;
+        for (uint32_t w = 0; w < L->waves; ++w) {
+          po[w] = pt;
+          pt += (uint64_t(L->wave_t[w]) + 1) * rows * kLaneWave;
+        }
+        L->path_elems = pt;
+        L->fwd_cost = lane_forward_cost(sh, int(sizeof(R) * 8));
+      }
     }
   }
   const auto u0 = std::chrono::steady_clock::now();
@@ -3299,6 +3334,56 @@ uint32_t run_outputs(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   return nslots;
 }
 
+// Room for the lane parts' stored paths, from `lease`: elements of the
+// working type for each class of each part (0: recompute).  A stored path
+// saves the recompute pass (and its phase switches) and costs a write and a
+// read of the segment rows of every step.  The write runs beside the forward
+// pass, so it pays as long as the memory keeps up: the room is at most what
+// one and a half times the forward pass takes at kPathRate (the counted
+// instructions at 4 cycles each and 2.4 GHz, the longest wave or the whole
+// chip's work, whichever is longer; the pass itself runs at about 1.3 of
+// that), and what the lease grants.  Each class gets its share, its longest
+// waves first.  8,192 chains of 16 DOF x 10,000 steps (21 GB, the chip full):
+// 17.1 ms recomputed, 13.8 ms stored; 4,096 uneven systems 14.2 and 9.7 ms;
+// a batch of one- and two-DOF systems that fills the chip moves 10 TB/s at
+// its forward rate and keeps most of its waves on checkpoints.
+constexpr double kPathRate = 4.5e12;
+template <typename R>
+std::vector<std::vector<uint64_t>> path_plan(pasif_driver* d, PathLease& lease,
+                                             std::vector<void*>* base) {
+  Packed& pk = d->pk;
+  std::vector<std::vector<uint64_t>> room(pk.lparts.size());
+  double elems = 0, work = 0, chain = 0;
+  for (size_t i = 0; i < pk.lparts.size(); ++i) {
+    room[i].assign(pk.lparts[i]->cls.size(), 0);
+    for (const auto& L : pk.lparts[i]->cls) {
+      if (!L->pathoff) continue;
+      elems += double(L->path_elems);
+      for (uint32_t t : L->wave_t) work += double(t) * L->fwd_cost;
+      chain = std::max(chain, double(L->tmax) * L->fwd_cost);
+    }
+  }
+  base->assign(pk.lparts.size(), nullptr);
+  if (elems == 0 || d->window) return room;
+  const double fwd_s = std::max(work / device_simds(d->dev), chain) * 4.0 / 2.4e9;
+  const double want = std::min(elems * sizeof(R), 1.5 * fwd_s * kPathRate);
+  const size_t bytes = size_t(std::min(want, double(path_pool().limit(d->dev))));
+  void* p = bytes > (size_t(1) << 16) ? lease.take(d->dev, bytes) : nullptr;
+  if (!p) return room;
+  const double share = double(bytes) / (elems * sizeof(R));
+  unsigned char* at = static_cast<unsigned char*>(p);
+  for (size_t i = 0; i < pk.lparts.size(); ++i) {
+    (*base)[i] = at;
+    for (size_t c = 0; c < room[i].size(); ++c) {
+      const LaneCls& L = *pk.lparts[i]->cls[c];
+      if (!L.pathoff) continue;
+      room[i][c] = uint64_t(double(L.path_elems) * std::min(share, 1.0)) / 64 * 64;
+      at += room[i][c] * sizeof(R);
+    }
+  }
+  return room;
+}
+
 // Run buffers of one lane part and its per-class kernel arguments (budget
 // filled in by the caller).  K is the part's checkpoint interval.  Buffers
 // come from `mem` (null: the driver's own), outputs are the driver's unless
@@ -3307,7 +3392,9 @@ template <typename R>
 std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
                                      uint32_t save_steps, uint32_t nslots, const void* excit,
                                      const void* interp, RunMem* mem_in = nullptr,
-                                     void* out_q = nullptr, void* out_grad = nullptr) {
+                                     void* out_q = nullptr, void* out_grad = nullptr,
+                                     void* path = nullptr,
+                                     const std::vector<uint64_t>* path_room = nullptr) {
   Packed& pk = d->pk;
   RunMem own;
   own.d = d;
@@ -3346,6 +3433,12 @@ std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
     a.out_a = L.out_a;
     a.na_out = L.na_out;
     a.ck_off = L.ckoff;
+    if (path && path_room && (*path_room)[c]) {
+      a.path = path;
+      a.path_off = L.pathoff;
+      a.path_cap = (*path_room)[c];
+      path = static_cast<unsigned char*>(path) + (*path_room)[c] * sizeof(R);
+    }
     a.out_q = out_q;
     a.out_max = d->window ? d->out_max.p : nullptr;
     a.traj = save_steps ? d->traj.p : nullptr;
@@ -3496,9 +3589,12 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, std::vector<
   std::vector<std::vector<LaneArgs>> largs;
   if (lane) {
     nslots = run_outputs<R>(d, adjoint, save_steps);
-    for (auto& lp : pk.lparts)
-      largs.push_back(lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, d->d_exc.p,
-                                        d->d_interp.p));
+    std::vector<void*> pbase;
+    const auto room = path_plan<R>(d, lease, &pbase);
+    for (size_t i = 0; i < pk.lparts.size(); ++i)
+      largs.push_back(lane_part_args<R>(d, *pk.lparts[i], adjoint, save_steps, nslots, d->d_exc.p,
+                                        d->d_interp.p, nullptr, nullptr, nullptr, pbase[i],
+                                        &room[i]));
   }
   const uint64_t lwork = lane ? (adjoint ? 3ull * pk.ltmax : pk.ltmax) : 0;
   uint64_t launches = 1;

@@ -308,10 +308,6 @@ double gside_stage_cost(const GSide& gs, uint32_t G, bool setpoints_own, int bit
       stage += t.kind + 1.0;
       kinds[t.kind] = true;
     }
-    const int nk = kinds[0] + kinds[1] + kinds[2] + kinds[3];
-    stage += nk > 1 ? nk - 1 : 0;
-    stage += row.force.empty() ? 0 : 1;
-    if (r >= gs.RL) stage += lg * (rot + 1.0);
   }
   return stage + remote_count(gs, setpoints_own) * rot;
 }
@@ -479,6 +475,12 @@ uint32_t lane_live(const LaneShape& sh) {
   return std::max(fwd, adj);
 }
 
+double lane_forward_cost(const LaneShape& sh, int bits) {
+  LaneShape f = sh;
+  f.adjoint = false;
+  return lane_step_cost(f, bits);
+}
+
 double lane_step_cost(const LaneShape& sh, int bits) {
   const uint32_t G = sh.group;
   auto side = [&](const LaneSide& sd, const GSide& gs, bool setpoints_own) {
@@ -494,10 +496,6 @@ double lane_step_cost(const LaneShape& sh, int bits) {
         const int nk = kinds[0] + kinds[1] + kinds[2] + kinds[3];
         stage += nk > 1 ? nk - 1 : 0;
       }
-      stage += double(sd.forced.size()) + 2.0 * rows;
-    } else {
-      rows = gs.nl();
-      stage = gside_stage_cost(gs, G, setpoints_own, bits);
     }
     return 4.0 * stage + 2.0 * rows;
   };
@@ -505,7 +503,7 @@ double lane_step_cost(const LaneShape& sh, int bits) {
   const double f = side(sh.f, sh.gf, true) + forcing + loop;
   if (!sh.adjoint) return f;
   const double nx = G <= 1 ? sh.f.n : double(sh.gx.size());
-  const double a = side(sh.a, sh.ga, false) + 3.0 * nx + loop;
+  const double a = side(sh.a, sh.ga, false) + 4.0 * nx + loop;
   return 2.0 * f + a;
 }
 
@@ -653,6 +651,13 @@ __device__ __forceinline__ void put_g(R* e, const R (&v)[NPF], u32 Lx, u32 b, bo
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
   }
+}
+
+// LDS written by the wave's other lanes is visible
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 // Mi[1][j] e[i] + Mi[0][j] e[i+1] on the half step i0*W + j0 + t, zero
@@ -882,6 +887,9 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   const bool adjoint = S::ADJ && a.adjoint != 0ull;
   const u32 K = adjoint ? (u32)a.ck_every : 1u;
   constexpr bool EX = EXACT != 0 && S::ADJ;
+  // steps of a stored path read ahead at once (registers, then the segment's
+  // place in LDS)
+  constexpr u32 PB = NSEG >= 16u ? 1u : (NSEG <= 2u ? 8u : 16u / NSEG);
   R* seg3 = seg + (K + 1u) * NSEG * WAVE;
   const u32 W = (u32)a.interp_w;
   const u32 Lx = (u32)a.exc_len;
@@ -907,6 +915,17 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   GP(R) ls = (GP(R))a.lstate + col;
   // checkpoints: the wave's block [nck_w][NF][WAVE] (sized by its longest instance)
   GP(R) ck = (GP(R))a.ckpt + (adjoint ? ((GP(const u64))a.ck_off)[wave] : 0ull) + lane;
+  // Stored path: the forward pass writes every step's set points to the
+  // wave's block [T + 1][NSEG][WAVE] and the reverse pass streams them back,
+  // instead of checkpoints and recomputed segments (where the launch gave
+  // the wave room for it; waves come longest first).
+  u64 po = 0ull;
+  bool stored = false;
+  if (STORE && adjoint && a.path != 0) {
+    po = ((GP(const u64))a.path_off)[wave];
+    po = ((u64)uni((u32)(po >> 32)) << 32) | (u64)uni((u32)po);
+  }
+  GP(R) ph = (GP(R))a.path + po + lane;
   GP(R) sb = (GP(R))a.segbuf + col;
   GP(R) sb3 = sb + (u64)(K + 1u) * NF * st;
   GP(R) outq = (GP(R))a.out_q;
@@ -920,6 +939,9 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   u32 phase = uni(pst[1]);
   u32 sg = uni(pst[2]);
   u32 budget = (u32)a.budget;
+  if (STORE && adjoint && a.path != 0)
+    stored = SE == 0u && a.window == 0ull &&
+             po + (u64)(T + 1u) * (NSEG * WAVE) <= (u64)a.path_cap;
   // output row of lane slot r: band slots hold row rowf(r) + p stridef(r), a
   // shared slot's row is written by position 0 only (-1 elsewhere)
   auto orow_f = [&](int r) -> int {
@@ -1018,6 +1040,10 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         }
         seg_here = true;
       }
+      if (STORE && stored && n == 0u)
+#pragma unroll
+        for (int r = 0; r < NF; ++r)
+          if (S::segr(r) >= 0) ph[S::segr(r) * WAVE] = q[r];
       const u32 e = recompute ? umin(T, s0 + K) : T;
       const u32 nend = (e - n < budget) ? e : n + budget;
       budget -= nend - n;
@@ -1054,7 +1080,8 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
               hi += 1u;
             }
           }
-          if ((MODE == mCk || MODE == mFull) && adjoint && !recompute && n == next_ck) {
+          if ((MODE == mCk || MODE == mFull) && adjoint && !recompute && !(STORE && stored) &&
+              n == next_ck) {
 #pragma unroll
             for (int r = 0; r < NF; ++r) ck[((u64)(n / K) * NF + r) * WAVE] = q[r];
             next_ck += K;
@@ -1074,6 +1101,14 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
             }, hl, h, h2, h6, n < fsteps);
           } else {
             rk4<NF, ALL, S>(q, rhs, hl, h, h2, h6, n < fsteps);
+          }
+          if constexpr (STORE && MODE == mCk) {
+            if (stored) {
+              GP(R) o = ph + (u64)(n + 1u) * (NSEG * WAVE);
+#pragma unroll
+              for (int r = 0; r < NF; ++r)
+                if (S::segr(r) >= 0) o[S::segr(r) * WAVE] = q[r];
+            }
           }
           if constexpr (MODE == mRec) {
             const u32 m = n + 1u - s0;
@@ -1200,9 +1235,14 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         if (recompute) {
           phase = kBackward;
         } else if (adjoint && T > 0u) {
-          sg = (T - 1u) / K;
-          n = sg * K;
-          phase = kRecompute;
+          if (STORE && stored) {
+            sg = 0u;
+            phase = kBackward;
+          } else {
+            sg = (T - 1u) / K;
+            n = sg * K;
+            phase = kRecompute;
+          }
 #pragma unroll
           for (int r = 0; r < NA; ++r) lam[r] = ainit(r);
         } else {
@@ -1218,7 +1258,27 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #pragma unroll
       for (int t = 0; t < S::TA; ++t) c[t] = ca[t * st];
       const u32 s0 = sg * K;
-      if (!seg_here) {
+      // first step LDS holds; of a stored path PB steps at a time (at most
+      // the K + 1 states the segment has room for), the next ones in registers
+      u32 base = s0;
+      const u32 pb = umin(PB, K);
+      R pre[STORE ? PB * NSEG : 1u];
+      auto path_fetch = [&]() {
+        const u32 nb = base > pb ? base - pb : 0u;
+#pragma unroll
+        for (u32 m = 0; m < PB; ++m)
+          if (m < base - nb)
+#pragma unroll
+            for (u32 j = 0; j < NSEG; ++j)
+              pre[m * NSEG + j] = ph[((u64)(nb + m) * NSEG + j) * WAVE];
+      };
+      if (STORE && stored) {
+        base = n > pb ? n - pb : 0u;
+        for (u32 m = 0; m <= n - base; ++m)
+#pragma unroll
+          for (u32 j = 0; j < NSEG; ++j)
+            seg[(m * NSEG + j) * WAVE + lane] = ph[((u64)(base + m) * NSEG + j) * WAVE];
+      } else if (!seg_here) {
         // resumed in the reverse phase: reload the segment this launch needs
         for (u32 m = 0; m <= n - s0; ++m)
 #pragma unroll
@@ -1249,7 +1309,8 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
             continue;
           }
           R xc[NX], xb[NX], xp[NX];
-          S::xload(xc, xp, seg + (n - s0) * (NSEG * WAVE), seg + (n - 1u - s0) * (NSEG * WAVE), lane);
+          S::xload(xc, xp, seg + (n - base) * (NSEG * WAVE), seg + (n - 1u - base) * (NSEG * WAVE),
+                   lane);
 #pragma unroll
           for (int j = 0; j < NX; ++j) xb[j] = R(0.5) * (xc[j] + xp[j]);
           rk4_adj<NA, ALL, S>(lam, [&](R* e, int s) {
@@ -1257,9 +1318,29 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           }, h, h2, h6, n <= fsteps);
         }
       };
-      // steps n > Tmin leave some lanes inactive; from Tmin down all are active
-      if (n > Tmin) back_to(Flag<false>(), Tmin > nend ? Tmin : nend);
-      if (n > nend) back_to(Flag<true>(), nend);
+      if (STORE && stored) path_fetch();
+      while (n > nend) {
+        const u32 lo = base > nend ? base : nend;
+        // steps n > Tmin leave some lanes inactive; from Tmin down all are active
+        if (n > Tmin) back_to(Flag<false>(), Tmin > lo ? Tmin : lo);
+        if (n > lo) back_to(Flag<true>(), lo);
+        if (STORE && stored && n > nend) {
+          // the steps before: x_base moves up, the fetched ones go below it
+          const u32 nb = base > pb ? base - pb : 0u, cnt = base - nb;
+          wave_lds();
+#pragma unroll
+          for (u32 j = 0; j < NSEG; ++j)
+            seg[(cnt * NSEG + j) * WAVE + lane] = seg[j * WAVE + lane];
+#pragma unroll
+          for (u32 m = 0; m < PB; ++m)
+            if (m < cnt)
+#pragma unroll
+              for (u32 j = 0; j < NSEG; ++j) seg[(m * NSEG + j) * WAVE + lane] = pre[m * NSEG + j];
+          wave_lds();
+          base = nb;
+          path_fetch();
+        }
+      }
       if (n == s0) {
         if (sg == 0u) {
           phase = kDone;
@@ -2285,7 +2366,8 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
     << "u\n#define NFMAX " << dims.nfmax << "u\n#define SEGK " << lay.seg << "u\n#define SEGN "
     << (dims.adjoint ? size_t(lay.seg + 1) * dims.nfmax * lay.lw : 0) << "u\n#define FORCING "
     << lay.forcing << "\n#define FULL " << (lay.full ? 1 : 0) << "\n#define EXACT "
-    << (lay.exact && !mw ? 1 : 0) << "\n";
+    << (lay.exact && !mw ? 1 : 0) << "\n#define STORE "
+    << (lay.store && !lay.exact && !mw ? 1 : 0) << "\n";
   if (bits == 64) {
     o << "__device__ __forceinline__ R fmaR(R a, R b, R c) { return __builtin_fma(a, b, c); }\n"
          "__device__ __forceinline__ R absR(R a) { return __builtin_fabs(a); }\n"

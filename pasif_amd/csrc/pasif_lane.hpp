@@ -41,6 +41,11 @@ namespace pasif {
   X(const void*, ck_off)   /* u64 [waves] first element of each wave's      \
                               checkpoint block [nck_w][NF][64] (single-wave) */ \
   X(void*, segbuf)         /* [K+1][NF][stride] recomputed segment */       \
+  X(void*, path)           /* stored set points (null: none): per-wave      \
+                              blocks [T_w + 1][segment rows][64] */         \
+  X(const void*, path_off) /* u64 [waves] first element of each block */    \
+  X(uint64_t, path_cap)    /* elements of `path`: waves whose block ends    \
+                              beyond it recompute */                        \
   X(void*, out_q)                                                            \
   X(void*, out_max)                                                          \
   X(void*, traj)                                                             \
@@ -159,6 +164,8 @@ uint32_t lane_seg_rows(const LaneShape& sh, std::vector<int>* map = nullptr);
 // estimated vector instructions per step of one wave: forward step, and
 // forward + recompute + reverse step of an adjoint run
 double lane_step_cost(const LaneShape& sh, int bits);
+// of that, one forward step
+double lane_forward_cost(const LaneShape& sh, int bits);
 // system coefficient slots (lane_coefs order) -> the lane coefficients of
 // position p of a group side (0 where the position has no such term)
 void lane_group_coefs(const GSide& gs, const std::vector<double>& sys, uint32_t p,
@@ -188,6 +195,9 @@ struct LaneLayout {
   // (the pool) does not need; smaller code compiles faster
   uint32_t forcing = 0;
   bool full = true;
+  // single-wave adjoint kernels (reference recursion): compiled so that a
+  // launch may hand waves room to store their path
+  bool store = false;
 };
 // Values per lane and set-point row that a checkpoint segment of K steps
 // keeps: K + 1 post-step states, and three stage inputs per step for the
