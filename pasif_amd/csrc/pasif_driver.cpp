@@ -2009,25 +2009,38 @@ void choose_groups(std::vector<LaneShape>& shapes, const std::vector<ClassLoad>&
     return opt[c][k].second * load[c].steps_sum * opt[c][k].first / double(kLaneWave);
   };
   auto chain = [&](size_t c, size_t k) { return opt[c][k].second * load[c].steps_max; };
-  auto estimate = [&](const std::vector<size_t>& s, size_t* crit) {
-    double w = 0, ch = 0;
+  // steps alike in length: waves beyond a multiple of the SIMDs leave the
+  // last round partly empty
+  double steps = 0, inst = 0, longest = 0;
+  for (size_t c = 0; c < C; ++c) {
+    steps += load[c].steps_sum;
+    inst += load[c].inst;
+    longest = std::max(longest, load[c].steps_max);
+  }
+  const bool even = steps > 0.95 * inst * longest;
+  auto estimate = [&](const std::vector<size_t>& s) {
+    double w = 0, ch = 0, waves = 0;
     for (size_t c = 0; c < C; ++c) {
       if (opt[c].empty()) continue;
       w += work(c, s[c]);
-      if (chain(c, s[c]) > ch) {
-        ch = chain(c, s[c]);
-        if (crit) *crit = c;
-      }
+      waves += std::ceil(load[c].inst * opt[c][s[c]].first / double(kLaneWave));
+      ch = std::max(ch, chain(c, s[c]));
     }
+    const double rounds = waves / simds;
+    if (even && rounds > 1.0) w *= std::ceil(rounds) / rounds;
     return std::max(w / simds, ch);
   };
   for (int it = 0; it < 64 && !want; ++it) {
-    size_t m = 0;
-    const double est = estimate(sel, &m);
-    if (opt[m].empty() || sel[m] + 1 >= opt[m].size()) break;
+    // the classes whose waves run longest, together: sizes of one family
+    // often carry the same program (d DOFs a lane) and tie
+    const double est = estimate(sel);
+    double ch = 0;
+    for (size_t c = 0; c < C; ++c)
+      if (!opt[c].empty()) ch = std::max(ch, chain(c, sel[c]));
     std::vector<size_t> t = sel;
-    t[m] += 1;
-    if (estimate(t, nullptr) >= 0.99 * est) break;
+    for (size_t c = 0; c < C; ++c)
+      if (!opt[c].empty() && chain(c, sel[c]) > 0.97 * ch && sel[c] + 1 < opt[c].size()) t[c] += 1;
+    if (estimate(t) >= 0.99 * est) break;
     sel = t;
   }
   for (size_t c = 0; c < C; ++c) {

@@ -280,36 +280,129 @@ void build_gside(const LaneSide& sd, uint32_t G, const GMap& own, const GMap& se
   }
 }
 
-uint32_t remote_count(const GSide& gs, bool setpoints_own) {
+std::vector<GSrc> remote_sources(const GSide& gs, bool setpoints_own) {
   std::vector<GSrc> v;
   for (const GRow& row : gs.rows)
     for (const GTerm& t : row.terms)
       for (uint32_t a = 0; a <= (setpoints_own ? t.kind : 0u); ++a)
         if (!t.f[a].shared && t.f[a].d != 0) v.push_back(t.f[a]);
   std::sort(v.begin(), v.end());
-  return uint32_t(std::unique(v.begin(), v.end()) - v.begin());
+  v.erase(std::unique(v.begin(), v.end()), v.end());
+  return v;
+}
+uint32_t remote_count(const GSide& gs, bool setpoints_own) {
+  return uint32_t(remote_sources(gs, setpoints_own).size());
 }
 
 }  // namespace
 
 namespace {
 
-// Per-stage vector instructions of one lane of a group side: its union
-// terms, kind sums, forces, butterflies of shared rows and rotations.
-double gside_stage_cost(const GSide& gs, uint32_t G, bool setpoints_own, int bits) {
-  const uint32_t lg = log2u(G);
-  const double words = bits == 64 ? 2.0 : 1.0;
-  const double rot = G == 8 ? 3.0 * words : (G >= 32 ? 2.0 * words : words);
-  double stage = 2.0 * gs.nl();
-  for (uint32_t r = 0; r < gs.nl(); ++r) {
-    const GRow& row = gs.rows[r];
-    bool kinds[4] = {false, false, false, false};
-    for (const GTerm& t : row.terms) {
-      stage += t.kind + 1.0;
-      kinds[t.kind] = true;
+// Multiply-adds of a sum of products emitted in factored form (the same
+// greedy choice as `factored`; a term is its factors' numbers, none for a
+// constant), onto a base or not.
+using Term = std::vector<uint32_t>;
+uint32_t factored_ops(const std::vector<Term>& ts, bool base) {
+  if (ts.empty()) return 0;
+  std::map<uint32_t, uint32_t> count;
+  for (const Term& t : ts)
+    for (size_t a = 0; a < t.size(); ++a)
+      if (std::find(t.begin(), t.begin() + long(a), t[a]) == t.begin() + long(a)) ++count[t[a]];
+  uint32_t most = 1, s = 0;
+  for (const auto& c : count)
+    if (c.second > most) {
+      most = c.second;
+      s = c.first;
+    }
+  if (most == 1) {
+    uint32_t ops = 0;
+    for (const Term& t : ts)
+      if (t.empty()) {
+        ops += base ? 1 : 0;
+        base = true;
+      }
+    for (const Term& t : ts) ops += uint32_t(t.size());
+    return ops;
+  }
+  std::vector<Term> with, rest;
+  for (const Term& t : ts) {
+    auto it = std::find(t.begin(), t.end(), s);
+    if (it == t.end()) {
+      rest.push_back(t);
+    } else {
+      Term u = t;
+      u.erase(u.begin() + (it - t.begin()));
+      with.push_back(u);
     }
   }
-  return stage + remote_count(gs, setpoints_own) * rot;
+  return factored_ops(rest, base) + factored_ops(with, false) + 1;
+}
+
+// One row of a side for the cost model: its terms as (own factor, set-point
+// factors) numbers; forward terms have every factor in `x`.
+struct CostRow {
+  std::vector<uint32_t> own;    // adjoint: own factor of each term
+  std::vector<Term> x;
+  bool forced = false, shared = false, sink = false;
+};
+
+// Vector instructions per step of a side's rows: the factored sums of the
+// four stages (adjoint: effective coefficients at three set points, then a
+// multiply-add per own factor and stage -- three for a quadrature), the
+// state updates (7 per row, 2 for a sink), and butterflies of shared rows.
+double rows_step_cost(const std::vector<CostRow>& rows, bool forward, double gsum) {
+  double c = 0;
+  for (const CostRow& r : rows) {
+    if (r.x.empty() && !r.forced) continue;
+    if (forward) {
+      const bool lin = !r.shared && !r.sink && !r.forced && r.x.size() == 1 && r.x[0].size() == 1;
+      if (!lin) c += 4.0 * (factored_ops(r.x, r.forced || r.sink) + (r.forced ? 1 : 0));
+    } else {
+      std::map<uint32_t, std::vector<Term>> eff;
+      for (size_t t = 0; t < r.x.size(); ++t) eff[r.own[t]].push_back(r.x[t]);
+      for (const auto& e : eff) {
+        const bool constant = e.second.size() == 1 && e.second[0].empty();
+        c += 3.0 * (constant ? 0 : factored_ops(e.second, false));
+      }
+      c += (r.sink ? 3.0 : 4.0) * double(eff.size());
+    }
+    if (r.shared && !r.sink) c += 4.0 * gsum;
+    c += r.sink ? 2.0 : 7.0;
+  }
+  return c;
+}
+
+// rows_step_cost of a group side, with the rotations of every stage.
+double gside_step_cost(const GSide& gs, uint32_t G, bool forward, int bits) {
+  const double words = bits == 64 ? 2.0 : 1.0;
+  // a rotation: DPP moves (with a select in groups of 8 and 32), or the LDS
+  // crossbar, counted with the wait it costs a lone wave
+  const double rot = G == 8 || G == 32 ? 2.0 * words : words;
+  const double far = 8.0 * words;
+  std::vector<uint8_t> read(gs.nl(), 0);
+  for (const GRow& row : gs.rows)
+    for (const GTerm& t : row.terms)
+      for (uint32_t a = 0; a <= (forward ? t.kind : 0u); ++a) read[t.f[a].slot] = 1;
+  auto num = [](const GSrc& x) { return (x.slot * 64u + x.d) * 2u + (x.shared ? 1u : 0u); };
+  std::vector<CostRow> rows(gs.nl());
+  for (uint32_t r = 0; r < gs.nl(); ++r) {
+    CostRow& cr = rows[r];
+    cr.forced = !gs.rows[r].force.empty();
+    cr.shared = r >= gs.RL;
+    cr.sink = !read[r];
+    for (const GTerm& t : gs.rows[r].terms) {
+      Term x;
+      for (uint32_t a = forward ? 0u : 1u; a <= t.kind; ++a) x.push_back(num(t.f[a]));
+      if (!forward) cr.own.push_back(num(t.f[0]));
+      cr.x.push_back(x);
+    }
+  }
+  double rots = 0;
+  for (const GSrc& x : remote_sources(gs, forward))
+    rots += G >= 32 && x.d != 1 && x.d != G - 1 ? far : rot;
+  const double gsum = log2u(std::min(G, 16u)) * (words + 1.0) +
+                      (G > 16 ? log2u(G / 16) * (far + 1.0) : 0.0);
+  return rows_step_cost(rows, forward, gsum) + 4.0 * rots;
 }
 
 // The cheapest of the candidate band plans of a side (each built exactly).
@@ -348,7 +441,7 @@ bool best_gside(const LaneSide& sd, uint32_t G, const GSide* mirror, uint32_t nm
     if (gs.RL == 0) continue;
     const GMap own = group_map(sd.n, G, gs);
     build_gside(sd, G, own, setp ? *setp : own, setp == nullptr, &gs);
-    const double c = gside_stage_cost(gs, G, setp == nullptr, bits);
+    const double c = gside_step_cost(gs, G, setp == nullptr, bits);
     if (best < 0 || c < best) {
       best = c;
       *out = std::move(gs);
@@ -483,24 +576,28 @@ double lane_forward_cost(const LaneShape& sh, int bits) {
 
 double lane_step_cost(const LaneShape& sh, int bits) {
   const uint32_t G = sh.group;
-  auto side = [&](const LaneSide& sd, const GSide& gs, bool setpoints_own) {
-    double stage = 0, rows = 0;
-    if (G <= 1) {
-      rows = sd.n;
-      for (const auto& row : sd.rows) {
-        bool kinds[4] = {false, false, false, false};
-        for (const LaneTerm& t : row) {
-          stage += t.kind + 1.0;
-          kinds[t.kind] = true;
-        }
-        const int nk = kinds[0] + kinds[1] + kinds[2] + kinds[3];
-        stage += nk > 1 ? nk - 1 : 0;
+  auto side = [&](const LaneSide& sd, const GSide& gs, bool forward) {
+    if (G > 1) return gside_step_cost(gs, G, forward, bits);
+    std::vector<uint8_t> read(sd.n, 0);
+    for (const auto& row : sd.rows)
+      for (const LaneTerm& t : row)
+        for (uint32_t a = 0; a <= (forward ? t.kind : 0u); ++a) read[t.f[a]] = 1;
+    std::vector<CostRow> rows(sd.n);
+    for (uint32_t r = 0; r < sd.n; ++r) {
+      rows[r].sink = !read[r];
+      for (const LaneTerm& t : sd.rows[r]) {
+        rows[r].x.emplace_back(t.f + (forward ? 0 : 1), t.f + t.kind + 1);
+        if (!forward) rows[r].own.push_back(t.f[0]);
       }
     }
-    return 4.0 * stage + 2.0 * rows;
+    for (uint32_t r : sd.forced) rows[r].forced = true;
+    return rows_step_cost(rows, forward, 0.0);
   };
-  const double forcing = 14.0, loop = 8.0;
-  const double f = side(sh.f, sh.gf, true) + forcing + loop;
+  // forcing and loop: measured beside the counted instructions (112.5 vector
+  // and 13.5 scalar instructions a forward step of the 16-DOF chain, of which
+  // the model counts 104)
+  const double loop = 16.0;
+  const double f = side(sh.f, sh.gf, true) + loop;
   if (!sh.adjoint) return f;
   const double nx = G <= 1 ? sh.f.n : double(sh.gx.size());
   const double a = side(sh.a, sh.ga, false) + 4.0 * nx + loop;
@@ -582,9 +679,33 @@ __device__ __forceinline__ R rot(R x) {
     return ((threadIdx.x & 7u) + D < 8u) ? a : b;
   } else if constexpr (G == 16u) {
     return dpp<0x120 + 16 - (int)D, R>(x);  // row_ror:(16 - D)
+  } else if constexpr (G == 64u && D == 1u) {
+    return dpp<0x134, R>(x);  // wave_rol:1
+  } else if constexpr (G == 64u && D == 63u) {
+    return dpp<0x13C, R>(x);  // wave_ror:1
   } else {
     const u32 l = threadIdx.x & 63u;
     return bperm<R>(x, (l & ~(G - 1u)) | ((l + D) & (G - 1u)));
+  }
+}
+// rot where no position uses a value that wraps around the group's end (the
+// ends of a chain): those positions get 0 instead (not a neighbouring
+// instance's value, which a zero coefficient would not hide when it is not
+// finite).  Groups of 8: one shift and a select instead of two shifts and a
+// select; groups of 32, by one: a shift of the whole wave and a select
+// instead of a trip through the LDS crossbar.
+template <u32 G, u32 D>
+__device__ __forceinline__ R shift0(R x) {
+  constexpr bool left = 2u * D <= G;
+  constexpr u32 d = left ? D : G - D;
+  const u32 p = threadIdx.x & (G - 1u);
+  const bool in = left ? p + d < G : p >= d;
+  if constexpr (G == 8u) {
+    const R v = dpp<(left ? 0x100 : 0x110) + (int)d, R>(x);
+    return in ? v : R(0);
+  } else {
+    const R v = dpp<left ? 0x134 : 0x13C, R>(x);
+    return in ? v : R(0);
   }
 }
 // Sum over the group by an xor butterfly: lanes add their partner's value
@@ -1899,6 +2020,31 @@ struct RowKinds {
   uint32_t nlin = 0;
 };
 
+// Whether shift0 stands for the rotation by d in groups of G: no position
+// that wraps uses a term reading source `src` as one of its first `nf(t)`
+// factors.
+bool zero_shift(const GSide& gs, uint32_t G, const GSrc& src, bool forward) {
+  const bool left = 2 * src.d <= G;
+  const uint32_t d = left ? src.d : G - src.d;
+  if (!(G == 8 || (G == 32 && d == 1))) return false;
+  for (const GRow& row : gs.rows)
+    for (const GTerm& t : row.terms)
+      for (uint32_t a = 0; a <= (forward ? t.kind : 0u); ++a)
+        if (t.f[a] == src)
+          for (uint32_t p = 0; p < G; ++p)
+            if (t.coef[p] >= 0 && (left ? p + d >= G : p < d)) return false;
+  return true;
+}
+
+// Declaration of the value of another position that a program reads.
+std::string rotated(const GSide& gs, uint32_t G, const GSrc& r, bool forward) {
+  std::ostringstream o;
+  o << "    const R y" << r.slot << "_" << r.d << " = "
+    << (zero_shift(gs, G, r, forward) ? "shift0" : "rot") << "<" << G << "u, " << r.d << "u>(y["
+    << r.slot << "]);\n";
+  return o.str();
+}
+
 // One row of a forward right-hand side: terms over state names, the force,
 // coefficients c[slot].
 void emit_forward_row(std::ostringstream& o, Monos& monos, const RowKinds& rk, uint32_t r,
@@ -2132,9 +2278,7 @@ void emit_group_forward(std::ostringstream& o, const GSide& gs, uint32_t G, cons
         if (!t.f[a].shared && t.f[a].d != 0) rem.push_back(t.f[a]);
   std::sort(rem.begin(), rem.end());
   rem.erase(std::unique(rem.begin(), rem.end()), rem.end());
-  for (const GSrc& r : rem)
-    o << "    const R y" << r.slot << "_" << r.d << " = rot<" << G << "u, " << r.d << "u>(y["
-      << r.slot << "]);\n";
+  for (const GSrc& r : rem) o << rotated(gs, G, r, true);
   auto S = [&](const GSrc& r) {
     return (r.shared || r.d == 0) ? "y[" + std::to_string(r.slot) + "]"
                                   : "y" + std::to_string(r.slot) + "_" + std::to_string(r.d);
@@ -2488,8 +2632,7 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
             std::sort(rem.begin(), rem.end());
             rem.erase(std::unique(rem.begin(), rem.end()), rem.end());
             for (const GSrc& r : rem)
-              (pass ? oq : ol) << "    const R y" << r.slot << "_" << r.d << " = rot<" << G << "u, "
-                               << r.d << "u>(y[" << r.slot << "]);\n";
+              (pass ? oq : ol) << rotated(sh.ga, G, r, false);
           }
         }
         emit_adjoint_linear(oe, ol, oq, rows, ka, G, &ne);
