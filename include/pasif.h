@@ -112,6 +112,11 @@ int pasif_get_amplitudes(pasif_driver* d, double* out, size_t cap, size_t* len);
  * [slot][replica][dof]. */
 int pasif_get_trajectory(pasif_driver* d, uint32_t save_steps, double* out, size_t cap,
                          size_t* len);
+/* The same solve with the result laid out [replica][dof][slot] (extension:
+ * the rows PASIf.getTrajectory returns, transposed on the device).  The
+ * length comes from pasif_get_trajectory. */
+int pasif_get_trajectory_rows(pasif_driver* d, uint32_t save_steps, double* out, size_t cap,
+                              size_t* len);
 /* _getGradient (src/__GpuDriver.cu:502-587): lambda_0 of the adjoint
  * system, [replica][adjoint dof], over the full schedule T..1.  `save` is
  * accepted for signature compatibility; nonzero values are rejected. */

@@ -428,12 +428,8 @@ class PASIf(_GpuDriver):
         if not self.systemSet:
             raise ValueError("The system must be set before computing the trajectory.")
         self.saveSteps = saveSteps
-        trajectory = self._getTrajectory(saveSteps)
-        n_out = self._out_len()
-        n_saved = trajectory.size // n_out if n_out else 0
-        out = np.zeros((n_out + 1, n_saved))
-        out[0] = np.arange(n_saved) * self.saveSteps / self.sampleRate
-        out[1:] = trajectory.reshape(n_saved, n_out).T
+        out = self._getTrajectoryRows(saveSteps, time_row=1)
+        out[0] = np.arange(out.shape[1]) * self.saveSteps / self.sampleRate
         return out
 
     def getGradient(self, save: int = 0):

@@ -170,6 +170,20 @@ class __GpuDriver:  # noqa: N801  (the reference's class name)
     def _getTrajectory(self, saveSteps_=1) -> np.ndarray:
         return self._get(self._pl.pasif_get_trajectory, C.c_uint32(int(saveSteps_)))
 
+    def _getTrajectoryRows(self, saveSteps_: int, time_row: int = 0) -> np.ndarray:
+        """The trajectory as ``[time_row + replica dof][slot]``; the first
+        ``time_row`` rows are left for the caller to fill."""
+        n = C.c_size_t(0)
+        save = C.c_uint32(int(saveSteps_))
+        self._chk(self._pl.pasif_get_trajectory(self._h, save, None, 0, C.byref(n)))
+        n_out = self._out_len()
+        slots = n.value // n_out if n_out else 0
+        out = np.empty((n_out + time_row, slots), dtype=np.float64)
+        rows = out[time_row:]
+        self._chk(self._pl.pasif_get_trajectory_rows(self._h, save, _p(rows, C.c_double),
+                                                     rows.size, C.byref(n)))
+        return out
+
     def _getGradient(self, save=0) -> np.ndarray:
         return self._get(self._pl.pasif_get_gradient, C.c_uint32(int(save)))
 

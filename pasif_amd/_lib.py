@@ -56,6 +56,8 @@ _SIGS = {
     "pasif_set_modulation_buffer": (C.c_int, [_h, _f64p, C.c_size_t]),
     "pasif_get_amplitudes": (C.c_int, [_h, _f64p, C.c_size_t, C.POINTER(C.c_size_t)]),
     "pasif_get_trajectory": (C.c_int, [_h, C.c_uint32, _f64p, C.c_size_t, C.POINTER(C.c_size_t)]),
+    "pasif_get_trajectory_rows": (C.c_int, [_h, C.c_uint32, _f64p, C.c_size_t,
+                                            C.POINTER(C.c_size_t)]),
     "pasif_get_gradient": (C.c_int, [_h, C.c_uint32, _f64p, C.c_size_t, C.POINTER(C.c_size_t)]),
     "pasif_set_systems_layout": (C.c_int, [_h, C.c_uint32, _u32p, _u32p, _i32p, _u32p]),
     "pasif_set_precision": (C.c_int, [_h, C.c_int]),

@@ -203,6 +203,11 @@ constexpr uint32_t kBigThreads = 1024;
 // lds: bytes of dynamic LDS for the partial sums (0 when they stay in device memory)
 hipError_t launch_big(const BigArgs<double>& a, uint32_t ninst, size_t lds, hipStream_t s);
 hipError_t launch_big(const BigArgs<float>& a, uint32_t ninst, size_t lds, hipStream_t s);
+// rows [r0, r0 + nr) of a trajectory [slots][rows], as doubles [nr][slots]
+hipError_t launch_traj_rows(const double* traj, double* out, uint32_t slots, uint32_t rows,
+                            uint32_t r0, uint32_t nr, hipStream_t s);
+hipError_t launch_traj_rows(const float* traj, double* out, uint32_t slots, uint32_t rows,
+                            uint32_t r0, uint32_t nr, hipStream_t s);
 // Size of the static device scratch array that holds the run buffers of
 // pasif_solve_noalloc, and the address of `dev`'s copy of it (looked up once
 // per device).
