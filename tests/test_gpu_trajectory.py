@@ -20,3 +20,31 @@ def test_trajectory_rows_are_the_slots_transposed(n, steps, save, bits):
     slots = p._getTrajectory(save).reshape(steps // save, 4 * n)
     np.testing.assert_array_equal(rows[1:], slots.T)
     np.testing.assert_array_equal(rows[0], np.arange(steps // save) * save / w.sample_rate)
+
+
+@pytest.mark.parametrize("window,save", [(1, 0), (16, 17), (29, 3), (33, 16), (1000, 1)])
+@pytest.mark.parametrize("even", [True, False])
+def test_window_and_saved_steps_are_the_states_of_every_step(even, window, save):
+    """Steps of the window, saved steps and the others run in loops of their
+    own: the amplitudes and the saved states are those of the states after
+    every step, for windows that begin inside a chunk of samples, before the
+    first step and at a different step in each lane of a wave."""
+    print(f"[gpu case] window {window}, save {save}, even {even}", flush=True)
+    n = 70
+    w = W.duffing(n_systems=n, steps=50)
+    steps = np.full(n, 50)
+    if not even:
+        steps = np.arange(n) % 50 + 1
+        w.steps_of_system = steps
+    p = W.make_solver(w)
+    per = w.vecM[0].shape[0]
+    every = p._getTrajectory(1).reshape(-1, per * n)
+    q, mx = p.getMaxAmplitudes(window=window)
+    rows = np.repeat(np.arange(n), per)
+    for r in range(per * n):
+        s = steps[rows[r]]
+        assert q[r] == every[s - 1, r], r
+        assert mx[r] == np.abs(every[max(0, s - window):s, r]).max(), r
+    if save:
+        saved = p._getTrajectory(save).reshape(-1, per * n)
+        np.testing.assert_array_equal(saved, every[::save][:saved.shape[0]])
