@@ -1616,7 +1616,7 @@ constexpr uint32_t kLaneMultiWaveBodies = 16;
 // multi-wave: waves per workgroup and values one wave's share may keep live
 constexpr uint32_t kLaneMaxWaves = 16;
 constexpr uint32_t kLaneMaxWaveLive = 100;
-constexpr size_t kLaneMaxLds = 64 * 1024;
+constexpr size_t kLaneMaxLds = 64 * 1024 + kLaneWts * sizeof(double);  // and the weights
 
 // Terms of row r of system s with identical monomials merged: for the
 // forward side every factor is the state, so a term is identified by its
@@ -2103,7 +2103,7 @@ uint32_t single_wave_segs(std::vector<LaneShape>& shapes, const std::vector<Clas
     for (size_t c = 0; c < shapes.size(); ++c) {
       LaneShape& sh = shapes[c];
       const uint32_t G = sh.group > 1 ? sh.group : 1u;
-      const size_t stage = size_t(kLaneStage + (G > 1 ? 3 * kLaneChunk : 0)) * (kLaneWave / G) * el;
+      const size_t stage = lane_stage_values(G) * el;
       // a step of the segment in LDS: the rows the reverse step reads; a
       // checkpoint: the whole forward state
       const size_t step = size_t(lane_seg_rows(sh)) * kLaneWave * el;
@@ -4752,7 +4752,7 @@ LaneLayout pool_single_layout(std::vector<LaneShape>& shapes, uint32_t Kreq, siz
     if (!sh.adjoint) continue;
     adj = true;
     const uint32_t G = sh.group > 1 ? sh.group : 1u;
-    const size_t stage = size_t(kLaneStage + (G > 1 ? 3 * kLaneChunk : 0)) * (kLaneWave / G) * el;
+    const size_t stage = lane_stage_values(G) * el;
     const size_t step = size_t(lane_seg_rows(sh)) * kLaneWave * el;
     const size_t b = std::min<size_t>(kLaneMaxLds, std::max<size_t>(kMaxLdsBytes / 8, stage + 6 * step));
     const size_t fit = b > stage ? (b - stage) / step : 0;

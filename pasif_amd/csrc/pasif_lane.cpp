@@ -625,9 +625,9 @@ enum : u32 { kForward = 0, kRecompute = 1, kBackward = 2, kDone = 3 };
 template <bool B> struct Flag { static constexpr bool value = B; };
 // per-step bookkeeping of a forward step loop: none, checkpoints (forward
 // pass of an adjoint run), the recomputed segment, a step with outputs or lanes
-// that enter the window at different steps (checkpoints too), and the window
-// with every lane in it
-enum : u32 { mPlain = 0, mCk = 1, mRec = 2, mFull = 3, mWin = 4 };
+// that enter the window at different steps (checkpoints too), the window with
+// every lane in it, and the stored path of an adjoint run
+enum : u32 { mPlain = 0, mCk = 1, mRec = 2, mFull = 3, mWin = 4, mSt = 5 };
 template <u32 M> struct Mode { static constexpr u32 value = M; };
 
 // ------------------------------------------------------------ lane groups
@@ -798,6 +798,23 @@ __device__ __forceinline__ R interp_at(const R* e, u32 b, GP(const R) wts, u32 W
   // at which a lone wave waits for them at once)
   const R keep = i > 0u ? R(1) : R(0);
   return fmaR(wts[W + j], ei, wts[j] * ei1) * keep;
+}
+
+// the next half step's position i W + j
+__device__ __forceinline__ void half_step(u32& i, u32& j, u32 W) {
+  j += 1u;
+  if (j >= W) {
+    j -= W;
+    i += 1u;
+  }
+}
+// the same from staged weights: pair w of the LDS copy, sample d of the chunk
+// (not masked for the first sample)
+typedef R R2 __attribute__((ext_vector_type(2)));
+template <u32 SS>
+__device__ __forceinline__ R interp_w(const R* e, const R* wl, u32 d, u32 w) {
+  const R2 g = ((const R2*)wl)[w];
+  return fmaR(g.x, e[d * SS], g.y * e[(d + 1u) * SS]);
 }
 
 // One RK4 step of N rows; rhs(k, y, stage).  ALL: every lane is active.
@@ -993,9 +1010,9 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   constexpr u32 G = S::G;
   constexpr u32 IPW = WAVE / G;  // instances per wave
   constexpr u32 NPF = (STAGE + G - 1u) / G;  // samples each lane of a group stages
-  // groups with interpolated forcing: the chunk's forcing values (3 per
-  // step) computed once by the group's lanes into a table
-  constexpr u32 FT = G > 1u ? 3u * CHUNK : 0u;
+  // groups with interpolated forcing: the chunk's forcing values (the two new
+  // half steps of every step) computed once by the group's lanes into a table
+  constexpr u32 FT = G > 1u ? 2u * CHUNK : 0u;
   constexpr u32 NFT = (FT + G - 1u) / G;
   const u32 lane = threadIdx.x;
   const u32 p = lane & (G - 1u);
@@ -1003,9 +1020,10 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   const u32 col = wave * WAVE + lane;
   const u32 i = wave * IPW + lane / G;
   const bool valid = i < (u32)a.count;
-  R* eb = smem + lane / G;                // the instance's staged samples
-  R* ft = smem + STAGE * IPW + lane / G;  // its forcing table (groups)
-  R* seg = smem + (STAGE + FT) * IPW;
+  R* wl = smem;                                  // interpolation weights (pairs)
+  R* eb = smem + WTS + lane / G;                 // the instance's staged samples
+  R* ft = smem + WTS + STAGE * IPW + lane / G;   // its forcing table (groups)
+  R* seg = smem + WTS + (STAGE + FT) * IPW;
   const bool adjoint = S::ADJ && a.adjoint != 0ull;
   const u32 K = adjoint ? (u32)a.ck_every : 1u;
   constexpr bool EX = EXACT != 0 && S::ADJ;
@@ -1108,6 +1126,23 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   // next launch can rebuild its LDS copy; one that runs to the end does not
   const bool mirror = a.budget != 0xFFFFFFFFull;
 
+  // Forcing: samples are staged for CS steps at a time (half steps are a sample
+  // apart at W = 1: fewer steps).  Such a chunk moves the cursor by dI samples
+  // and dJ half steps, a table entry is gI samples and gJ half steps from the
+  // lane's one before, so that only a phase divides by W.  All weights of a
+  // short window are staged here, of a longer one each chunk's.
+  const u32 CS = W == 1u ? CHUNK / 2u : CHUNK;
+  const u32 dI = W ? (2u * CS) / W : 0u, dJ = W ? 2u * CS - dI * W : 0u;
+  const u32 gI = W ? G / W : 0u, gJ = W ? G - gI * W : 0u;
+  const bool wall = W <= 2u * CHUNK;
+  if (FORCING != 2 && wall && W != 0u) {
+    if (lane < W) {
+      wl[2u * lane] = wts[W + lane];
+      wl[2u * lane + 1u] = wts[lane];
+    }
+    wave_lds();
+  }
+
   while (budget > 0u && phase != kDone) {
     if (phase != kBackward) {
       const bool recompute = phase == kRecompute;
@@ -1120,13 +1155,20 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       if (recompute && n == s0)
 #pragma unroll
         for (int r = 0; r < NF; ++r) q[r] = ck[((u64)sg * NF + r) * WAVE];
-      // forcing cursor: half-step position 2n = hi*W + hj, staged chunk
+      // forcing cursor: half-step position 2n = hi*W + hj of a chunk's start
       u32 hi = W ? (2u * n) / W : 0u, hj = W ? 2u * n - hi * W : 0u;
       u32 ebase = 0, left = 0, nchunk = 0;
-      u32 pbase = W ? hi : n;
       R pre[NPF];
-      fetch_g<G, NPF>(pre, E, Lx, pbase, p);
-      bool have = true;
+      fetch_g<G, NPF>(pre, E, Lx, W ? hi : n, p);
+      R uc = R(0);              // forcing at the half step 2n
+      u32 ci = hi, cj = hj;     // its position where no table is built (G = 1)
+      // the lane's first table entry, half step 2n + 1 + p, and G further
+      u32 ti = 0, tj = 0;
+      if (FORCING != 2 && FT > 0u && W != 0u) {
+        ti = (hj + 1u + p) / W;
+        tj = hj + 1u + p - ti * W;
+        ti += hi;
+      }
       R hl[S::NLIN > 0 ? S::NLIN : 1][3];
       // the phase's loads land here: no wait for them inside the step loops,
       // where the in-order load counter would also hold back the prefetched
@@ -1171,7 +1213,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       budget -= nend - n;
       const u32 nfirst = n;
       // per-step bookkeeping only as far as the phase needs it
-      const u32 mode = recompute ? mRec : (adjoint ? mCk : mPlain);
+      const u32 mode = recompute ? mRec : (adjoint ? (STORE && stored ? mSt : mCk) : mPlain);
 #if FULL
       // the amplitude window: no lane's begins before step wlo, every lane's
       // has begun from step whi on
@@ -1185,6 +1227,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         constexpr bool ALL = decltype(all_t)::value;
         constexpr u32 MODE = decltype(mode_t)::value;
         constexpr bool ZOH = decltype(zoh_t)::value;
+        GP(R) po_n = ph + (u64)(n + 1u) * (NSEG * WAVE);
         for (; n < stop; ++n) {
           R u0, u1, u3;
           if (ZOH) {
@@ -1193,24 +1236,21 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
             u1 = u0;
             u3 = eb[(n + 1u - ebase) * IPW];
           } else {
+            // a step's last half step is the next one's first
+            u0 = uc;
+            const u32 m = 2u * (n - nchunk);
             if constexpr (FT > 0u) {
-              const u32 m = 3u * (n - nchunk);
-              u0 = ft[m * IPW];
-              u1 = ft[(m + 1u) * IPW];
-              u3 = ft[(m + 2u) * IPW];
+              u1 = ft[m * IPW];
+              u3 = ft[(m + 1u) * IPW];
             } else {
-              u0 = interp_at<IPW>(eb, ebase, wts, W, hi, hj, 0u);
-              u1 = interp_at<IPW>(eb, ebase, wts, W, hi, hj, 1u);
-              u3 = interp_at<IPW>(eb, ebase, wts, W, hi, hj, 2u);
+              half_step(ci, cj, W);
+              u1 = interp_w<IPW>(eb, wl, ci - ebase, wall ? cj : m + 1u) * (ci > 0u ? R(1) : R(0));
+              half_step(ci, cj, W);
+              u3 = interp_w<IPW>(eb, wl, ci - ebase, wall ? cj : m + 2u) * (ci > 0u ? R(1) : R(0));
             }
-            hj += 2u;
-            if (hj >= W) {
-              hj -= W;
-              hi += 1u;
-            }
+            uc = u3;
           }
-          if ((MODE == mCk || MODE == mWin || MODE == mFull) && adjoint && !recompute && !(STORE && stored) &&
-              n == next_ck) {
+          if ((MODE == mCk || MODE == mWin || MODE == mFull) && adjoint && n == next_ck) {
 #pragma unroll
             for (int r = 0; r < NF; ++r) ck[((u64)(n / K) * NF + r) * WAVE] = q[r];
             next_ck += K;
@@ -1231,13 +1271,11 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           } else {
             rk4<NF, ALL, S>(q, rhs, hl, h, h2, h6, n < fsteps);
           }
-          if constexpr (STORE && MODE == mCk) {
-            if (stored) {
-              GP(R) o = ph + (u64)(n + 1u) * (NSEG * WAVE);
+          if constexpr (MODE == mSt) {
 #pragma unroll
-              for (int r = 0; r < NF; ++r)
-                if (S::segr(r) >= 0) o[S::segr(r) * WAVE] = q[r];
-            }
+            for (int r = 0; r < NF; ++r)
+              if (S::segr(r) >= 0) po_n[S::segr(r) * WAVE] = q[r];
+            po_n += NSEG * WAVE;
           }
           if constexpr (MODE == mRec) {
             const u32 m = n + 1u - s0;
@@ -1269,41 +1307,67 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       };
       while (n < nend) {
         if (left == 0u) {
-          // a new chunk: its samples come from the prefetch (or are loaded
-          // now), and the next chunk's are requested
-          const u32 base = W ? hi : n;
-          if (have && pbase == base) {
-            put_g<G, NPF>(eb, pre, Lx, base, forced, p, W == 0u);
-          } else {
-            R v[NPF];
-            fetch_g<G, NPF>(v, E, Lx, base, p);
-            put_g<G, NPF>(eb, v, Lx, base, forced, p, W == 0u);
-          }
-          ebase = base;
+          // a new chunk: its samples come from the prefetch, and the next
+          // chunk's are requested
+          ebase = W ? hi : n;
           nchunk = n;
-          if constexpr (FT > 0u) {
+          put_g<G, NPF>(eb, pre, Lx, ebase, forced, p, W == 0u);
+          if constexpr (FORCING != 2) {
             if (W != 0u) {
-              // value k of the table: step nchunk + k / 3, half step
-              // 2 (nchunk + k / 3) + (0, 1, 2)[k % 3] = hi W + hj + ...
+              if (!wall) {
+                // half step t of the chunk, t = 0 .. 2 CHUNK < W
+                u32 j = hj + lane;
+                if (j >= W) j -= W;
+                if (lane <= 2u * CHUNK) {
+                  wl[2u * lane] = wts[W + j];
+                  wl[2u * lane + 1u] = wts[j];
+                }
+                wave_lds();
+              }
+              if (n == nfirst)
+                uc = interp_w<IPW>(eb, wl, 0u, wall ? hj : 0u) * (hi > 0u ? R(1) : R(0));
+              if constexpr (FT > 0u) {
+                R f[NFT];
+                u32 i = ti, j = tj;
 #pragma unroll
-              for (u32 v = 0; v < NFT; ++v) {
-                const u32 k = p + v * G;
-                if (k < FT) {
-                  const u32 m = k / 3u;
-                  const u32 hs = hj + 2u * m + (k - 3u * m);
-                  const u32 di = hs / W;
-                  ft[k * IPW] = interp_at<IPW>(eb, ebase, wts, W, hi + di, hs - di * W, 0u);
+                for (u32 v = 0; v < NFT; ++v) {
+                  const u32 k = p + v * G;
+                  // entries past the chunk's half steps (W = 1, or more lanes
+                  // than entries) are not read: any staged sample will do
+                  f[v] = interp_w<IPW>(eb, wl, umin(i - ebase, STAGE - 2u),
+                                       wall ? j : umin(k + 1u, 2u * CHUNK));
+                  i += gI;
+                  j += gJ;
+                  if (j >= W) {
+                    j -= W;
+                    i += 1u;
+                  }
+                }
+                if (hi == 0u)
+#pragma unroll
+                  for (u32 v = 0; v < NFT; ++v)
+                    if (hj + 1u + p + v * G < W) f[v] = R(0);
+#pragma unroll
+                for (u32 v = 0; v < NFT; ++v)
+                  if (p + v * G < FT) ft[(p + v * G) * IPW] = f[v];
+                wave_lds();
+                ti += dI;
+                tj += dJ;
+                if (tj >= W) {
+                  tj -= W;
+                  ti += 1u;
                 }
               }
-              __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-              __builtin_amdgcn_wave_barrier();
-              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+              hi += dI;
+              hj += dJ;
+              if (hj >= W) {
+                hj -= W;
+                hi += 1u;
+              }
             }
           }
-          left = CHUNK;
-          pbase = W ? (2u * (n + CHUNK)) / W : n + CHUNK;
-          fetch_g<G, NPF>(pre, E, Lx, pbase, p);
-          have = true;
+          left = CS;
+          fetch_g<G, NPF>(pre, E, Lx, W ? hi : n + CS, p);
         }
         u32 stop = umin(nend, n + left);
         if (n < Tmin && Tmin < stop) stop = Tmin;
@@ -1356,6 +1420,9 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #endif
         if (mode == mPlain) in_mode(Mode<mPlain>());
         else if (mode == mCk) in_mode(Mode<mCk>());
+#if STORE
+        else if (mode == mSt) in_mode(Mode<mSt>());
+#endif
         else in_mode(Mode<mRec>());
       }
       // an instance whose last step fell in this range kept its final state
@@ -1689,6 +1756,7 @@ __device__ __forceinline__ void run_mw(const LaneArgs& a, u32 wg, R* smem) {
       u32 next_ck = ((n + K - 1u) / K) * K;
       u32 next_save = SE ? ((n + SE - 1u) / SE) * SE : 0u;
       u32 hi = W ? (2u * n) / W : 0u, hj = W ? 2u * n - hi * W : 0u;
+      const u32 CS = W == 1u ? CHUNK / 2u : CHUNK;  // steps of STAGE samples
       u32 ebase = 0, left = 0, pbase = 0;
       bool have = false;
       R pre[DRIVES ? STAGE : 1];
@@ -1773,11 +1841,11 @@ __device__ __forceinline__ void run_mw(const LaneArgs& a, u32 wg, R* smem) {
               put<LW>(eb, v, Lx, base, forced);
             }
             ebase = base;
-            pbase = W ? (2u * (n + CHUNK)) / W : n + CHUNK;
+            pbase = W ? (2u * (n + CS)) / W : n + CS;
             fetch(pre, E, Lx, pbase);
             have = true;
           }
-          left = CHUNK;
+          left = CS;
         }
         u32 stop = umin(nend, n + left);
         if (n < Tmin && Tmin < stop) stop = Tmin;
@@ -2530,7 +2598,7 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
        "  return (u32)__builtin_amdgcn_readfirstlane((int)lo);\n"
        "}\n";
   o << "#define WAVE " << kLaneWave << "u\n#define CHUNK " << kLaneChunk << "u\n#define STAGE "
-    << kLaneStage << "u\n";
+    << kLaneStage << "u\n#define WTS " << kLaneWts << "u\n";
   MwDims dims;
   if (mw) dims = mw_dims(shapes, lay.waves);
   o << "#define LW " << (mw ? lay.lw : kLaneWave) << "u\n#define NYMAX " << dims.nymax
@@ -2766,7 +2834,7 @@ size_t lane_lds_bytes(const std::vector<LaneShape>& shapes, int bits, const Lane
   for (const LaneShape& s : shapes) {
     const uint32_t G = s.group > 1 ? s.group : 1u;
     const uint32_t K = s.seg ? s.seg : lay.seg;
-    size_t c = size_t(kLaneStage + (G > 1 ? 3 * kLaneChunk : 0)) * (kLaneWave / G);
+    size_t c = lane_stage_values(G);
     if (s.adjoint) c += lane_seg_values(K, lay.exact) * lane_seg_rows(s) * kLaneWave;
     v = std::max(v, c);
   }

@@ -215,6 +215,13 @@ uint32_t lane_partition(LaneShape& sh, uint32_t waves);
 constexpr uint32_t kLaneChunk = 16;
 constexpr uint32_t kLaneStage = kLaneChunk + 3;
 constexpr uint32_t kLaneWave = 64;
+// staged interpolation weights of a wave, in pairs (half steps of a chunk)
+constexpr uint32_t kLaneWts = 2 * (2 * kLaneChunk + 2);
+// LDS values of a wave before its segment: the weights, the samples of its
+// instances and, on groups of G > 1 lanes, their table of forcing values
+inline size_t lane_stage_values(uint32_t G) {
+  return kLaneWts + size_t(kLaneStage + (G > 1 ? 2 * kLaneChunk : 0)) * (kLaneWave / G);
+}
 
 // Generated source of one kernel covering `shapes` (class c runs the
 // workgroups of LaneArgs c) in precision `bits` with layout `lay`.

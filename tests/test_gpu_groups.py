@@ -155,3 +155,24 @@ def test_group_blocked_layouts_match_oracle(G, adjoint, maker, monkeypatch):
     assert rel_err(p.getAmplitudes(), oracle_run(w).q) < TOL64
     if adjoint:
         assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64
+
+
+@pytest.mark.parametrize("G,dof,W_", [(1, 1, 2), (1, 2, 6), (1, 1, 34), (2, 2, 2), (4, 2, 6),
+                                      (4, 2, 32), (8, 4, 2), (16, 8, 34), (32, 16, 10),
+                                      (64, 32, 64)])
+def test_staged_interpolation_windows(G, dof, W_):
+    """Interpolated forcing from staged weights: windows of two half steps up to
+    longer than a chunk of samples (all weights staged, or a chunk's), signals
+    that end before the run, uneven step counts, and launches that resume
+    inside a chunk."""
+    _case(f"interpolation window {W_}, G={G}, {dof} DOF")
+    rng = np.random.default_rng(W_)
+    w = W.heterogeneous(n_systems=41, tmin=5, tmax=150, n_signals=3, dof_choices=[dof],
+                        dof_probs=[1.0])
+    w.excitations = rng.normal(0, 1, (3, 2 + 250 // W_))
+    w.interp = rng.uniform(-1, 1, (2, W_))
+    p = _grouped(w, G)
+    q = p.getAmplitudes()
+    assert rel_err(q, oracle_run(w).q) < TOL64
+    p.setSolver("graph", steps_per_launch=37, launches_per_graph=3)
+    np.testing.assert_array_equal(p.getAmplitudes(), q)
