@@ -623,11 +623,10 @@ __device__ __forceinline__ u32 uni(u32 v) { return (u32)__builtin_amdgcn_readfir
 __device__ __forceinline__ u32 umin(u32 a, u32 b) { return a < b ? a : b; }
 enum : u32 { kForward = 0, kRecompute = 1, kBackward = 2, kDone = 3 };
 template <bool B> struct Flag { static constexpr bool value = B; };
-// per-step bookkeeping of a forward step loop: none, checkpoints (forward
-// pass of an adjoint run), the recomputed segment, a step with outputs or lanes
-// that enter the window at different steps (checkpoints too), the window with
-// every lane in it, and the stored path of an adjoint run
-enum : u32 { mPlain = 0, mCk = 1, mRec = 2, mFull = 3, mWin = 4, mSt = 5 };
+// per-step bookkeeping of a forward step loop: none, the recomputed segment, a
+// step with outputs or lanes that enter the window at different steps, the
+// window with every lane in it, and the stored path of an adjoint run
+enum : u32 { mPlain = 0, mRec = 1, mFull = 2, mWin = 3, mSt = 4 };
 template <u32 M> struct Mode { static constexpr u32 value = M; };
 
 // ------------------------------------------------------------ lane groups
@@ -752,6 +751,12 @@ __device__ __forceinline__ void put(R* e, const R (&v)[STAGE], u32 Lx, u32 b, bo
 // as 0: it only ever drives step 0's first stages, which take no forcing.
 template <u32 G, u32 NPF>
 __device__ __forceinline__ void fetch_g(R (&v)[NPF], GP(const R) E, u32 Lx, u32 b, u32 p) {
+  if (NPF * G <= Lx && b <= Lx - NPF * G) {
+    GP(const R) e = E + (b + p);
+#pragma unroll
+    for (u32 k = 0; k < NPF; ++k) v[k] = e[k * G];
+    return;
+  }
 #pragma unroll
   for (u32 k = 0; k < NPF; ++k) {
     const u32 i = b + p + k * G;
@@ -759,13 +764,23 @@ __device__ __forceinline__ void fetch_g(R (&v)[NPF], GP(const R) E, u32 Lx, u32 
   }
 }
 template <u32 G, u32 NPF>
-__device__ __forceinline__ void put_g(R* e, const R (&v)[NPF], u32 Lx, u32 b, bool forced, u32 p,
-                                      bool zoh) {
+__device__ __forceinline__ void put_g(R* e, const R (&v)[NPF], u32 Lx, u32 b, bool forced, bool all,
+                                      u32 p, bool zoh) {
+  // every lane forced and every sample inside the signal: nothing to mask, nor
+  // to clamp in fetch_g (a lone wave of 64 oscillators spent 250 of 980
+  // instructions a chunk on it: 1.63 -> 1.37 ms; 4,096 two-DOF systems x 20,000
+  // steps 3.25 -> 2.95 ms)
+  if (all && NPF * G <= Lx && b <= Lx - NPF * G && !(zoh && b == 0u)) {
 #pragma unroll
-  for (u32 k = 0; k < NPF; ++k) {
-    const u32 u = p + k * G;
-    if (u < STAGE)
-      e[u * (WAVE / G)] = (forced && b + u < Lx && !(zoh && b + u == 0u)) ? v[k] : R(0);
+    for (u32 k = 0; k < NPF; ++k)
+      if (p + k * G < STAGE) e[(p + k * G) * (WAVE / G)] = v[k];
+  } else {
+#pragma unroll
+    for (u32 k = 0; k < NPF; ++k) {
+      const u32 u = p + k * G;
+      if (u < STAGE)
+        e[u * (WAVE / G)] = (forced && b + u < Lx && !(zoh && b + u == 0u)) ? v[k] : R(0);
+    }
   }
   if constexpr (G > 1u) {
     // the other lanes of the group read these samples next
@@ -1043,6 +1058,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   const u32 fsteps = steps[i];
   const i32 exc = ((GP(const i32))a.exc)[i];
   const bool forced = exc >= 0;
+  const bool all_forced = __builtin_amdgcn_ballot_w64(forced) == ~0ull;
   const u32 fout = ((GP(const u32))a.out_f)[i];
   const u32 aout = ((GP(const u32))a.out_a)[i];
   const u32 nao = ((GP(const u32))a.na_out)[i];
@@ -1213,7 +1229,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       budget -= nend - n;
       const u32 nfirst = n;
       // per-step bookkeeping only as far as the phase needs it
-      const u32 mode = recompute ? mRec : (adjoint ? (STORE && stored ? mSt : mCk) : mPlain);
+      const u32 mode = recompute ? mRec : (STORE && stored ? mSt : mPlain);
 #if FULL
       // the amplitude window: no lane's begins before step wlo, every lane's
       // has begun from step whi on
@@ -1221,23 +1237,25 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       const u32 wlo = recompute || win == 0u ? ~0u : (Tmin > win ? Tmin - win : 0u);
       const u32 whi = recompute || win == 0u ? ~0u : (T > win ? T - win : 0u);
 #endif
-      u32 next_ck = ((n + K - 1u) / K) * K;
+      const bool ckpt = adjoint && !recompute && !(STORE && stored);
+      u32 nck = (n + K - 1u) / K;  // the next checkpoint and its step
+      u32 next_ck = nck * K;
       u32 next_save = SE ? ((n + SE - 1u) / SE) * SE : 0u;
       auto steps_to = [&](auto all_t, auto mode_t, auto zoh_t, u32 stop) {
         constexpr bool ALL = decltype(all_t)::value;
         constexpr u32 MODE = decltype(mode_t)::value;
         constexpr bool ZOH = decltype(zoh_t)::value;
         GP(R) po_n = ph + (u64)(n + 1u) * (NSEG * WAVE);
-        for (; n < stop; ++n) {
+        auto one = [&]() __attribute__((always_inline)) {
           R u0, u1, u3;
+          // a step's last half step is the next one's first: carried over, and
+          // the loads of a step are behind its first stages
+          u0 = uc;
           if (ZOH) {
             // 0 < n < L or 0: sample 0 and those past the end are staged as 0
-            u0 = eb[(n - ebase) * IPW];
             u1 = u0;
             u3 = eb[(n + 1u - ebase) * IPW];
           } else {
-            // a step's last half step is the next one's first
-            u0 = uc;
             const u32 m = 2u * (n - nchunk);
             if constexpr (FT > 0u) {
               u1 = ft[m * IPW];
@@ -1248,13 +1266,8 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
               half_step(ci, cj, W);
               u3 = interp_w<IPW>(eb, wl, ci - ebase, wall ? cj : m + 2u) * (ci > 0u ? R(1) : R(0));
             }
-            uc = u3;
           }
-          if ((MODE == mCk || MODE == mWin || MODE == mFull) && adjoint && n == next_ck) {
-#pragma unroll
-            for (int r = 0; r < NF; ++r) ck[((u64)(n / K) * NF + r) * WAVE] = q[r];
-            next_ck += K;
-          }
+          uc = u3;
           auto rhs = [&](R* k, const R* y, int s) {
             S::template rhs_f<MODE != mRec>(k, y, c, s == 0 ? u0 : (s == 3 ? u3 : u1));
           };
@@ -1303,7 +1316,20 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #pragma unroll
               for (int r = 0; r < NF; ++r) mx[r] = fmaxR(mx[r], absR(fval(r, q[r])));
           }
-        }
+          ++n;
+        };
+        // A taken branch costs a lone wave about as much as eight instructions
+        // (two-DOF: 2.95 -> 2.59 ms at four steps a turn, one wave of 64
+        // oscillators 1.37 -> 1.19, uneven batch in FP32 2.49 -> 2.25).
+        // Compile time keeps it to the loops that take most steps.
+        if constexpr (ALL && MODE != mFull)
+          while (n + 4u <= stop) {
+            one();
+            one();
+            one();
+            one();
+          }
+        while (n < stop) one();
       };
       while (n < nend) {
         if (left == 0u) {
@@ -1311,7 +1337,8 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           // chunk's are requested
           ebase = W ? hi : n;
           nchunk = n;
-          put_g<G, NPF>(eb, pre, Lx, ebase, forced, p, W == 0u);
+          put_g<G, NPF>(eb, pre, Lx, ebase, forced, all_forced, p, W == 0u);
+          if (W == 0u && n == nfirst) uc = eb[0];
           if constexpr (FORCING != 2) {
             if (W != 0u) {
               if (!wall) {
@@ -1371,6 +1398,17 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         }
         u32 stop = umin(nend, n + left);
         if (n < Tmin && Tmin < stop) stop = Tmin;
+        if (ckpt) {
+          // checkpoints are written between the loops
+          if (n == next_ck) {
+            GP(R) o = ck + (u64)nck * NF * WAVE;
+#pragma unroll
+            for (int r = 0; r < NF; ++r) o[r * WAVE] = q[r];
+            next_ck += K;
+            ++nck;
+          }
+          stop = umin(stop, next_ck);
+        }
 #if FULL
         // Steps with outputs in loops of their own (64 oscillators x 10,000
         // steps, window 2,000: 2.35 -> 1.73 ms with 42 instead of 62-78 vector
@@ -1419,7 +1457,6 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         else
 #endif
         if (mode == mPlain) in_mode(Mode<mPlain>());
-        else if (mode == mCk) in_mode(Mode<mCk>());
 #if STORE
         else if (mode == mSt) in_mode(Mode<mSt>());
 #endif
