@@ -1549,7 +1549,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
       budget -= n - nend;
       auto back_to = [&](auto all_t, u32 stop) {
         constexpr bool ALL = decltype(all_t)::value;
-        for (; n > stop; --n) {
+        auto one = [&]() __attribute__((always_inline)) {
           if constexpr (EX) {
             R y1[NX], y2[NX], y3[NX], y4[NX];
             const u32 mb = 3u * (n - 1u - s0);
@@ -1558,17 +1558,29 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
             exact_adj<NA, ALL, S>(lam, [&](R* e, int s) {
               S::eff_a(e, s == 0 ? y4 : (s == 1 ? y3 : (s == 2 ? y2 : y1)), c);
             }, h, h2, h6, n <= fsteps);
-            continue;
-          }
-          R xc[NX], xb[NX], xp[NX];
-          S::xload(xc, xp, seg + (n - base) * (NSEG * WAVE), seg + (n - 1u - base) * (NSEG * WAVE),
-                   lane);
+          } else {
+            R xc[NX], xb[NX], xp[NX];
+            S::xload(xc, xp, seg + (n - base) * (NSEG * WAVE),
+                     seg + (n - 1u - base) * (NSEG * WAVE), lane);
 #pragma unroll
-          for (int j = 0; j < NX; ++j) xb[j] = R(0.5) * (xc[j] + xp[j]);
-          rk4_adj<NA, ALL, S>(lam, [&](R* e, int s) {
-            S::eff_a(e, s == 0 ? xc : (s == 1 ? xb : xp), c);
-          }, h, h2, h6, n <= fsteps);
-        }
+            for (int j = 0; j < NX; ++j) xb[j] = R(0.5) * (xc[j] + xp[j]);
+            rk4_adj<NA, ALL, S>(lam, [&](R* e, int s) {
+              S::eff_a(e, s == 0 ? xc : (s == 1 ? xb : xp), c);
+            }, h, h2, h6, n <= fsteps);
+          }
+          --n;
+        };
+        // four a turn as forward: a state between two of them is read once
+        // (8,192 16-DOF chains x 10,000 steps 13.0 -> 12.5 ms, uneven batch
+        // 8.6 -> 8.1)
+        if constexpr (ALL)
+          while (n >= stop + 4u) {
+            one();
+            one();
+            one();
+            one();
+          }
+        while (n > stop) one();
       };
       if (STORE && stored) path_fetch();
       while (n > nend) {
