@@ -1597,13 +1597,17 @@ uint64_t pack_key(pasif_driver* d, bool adjoint) {
 // ------------------------------------------------------------ lane plan
 // Largest state + coefficient count (values of the working type) a class may
 // keep live: 2 VGPRs per FP64 value, leaving room for temporaries in 256.
+// A group of a whole wave may keep twice that (the compiler moves the rest to
+// the accumulation registers): its system has no wider layout, and 48 150-DOF
+// chains x 1,000 steps with their adjoint (144 live values) take 1.34 ms so
+// against 5.03 on the row kernel, 200-DOF ones (185) 2.80 against 5.03.
 constexpr uint32_t kLaneMaxLive = 96;
-uint32_t lane_max_live() {
+uint32_t lane_max_live(uint32_t G) {
   if (const char* e = std::getenv("PASIF_LANE_MAX_LIVE")) {
     const long v = std::strtol(e, nullptr, 10);
     if (v > 0 && v < 100000) return uint32_t(v);
   }
-  return kLaneMaxLive;
+  return G == kLaneWave ? 2 * kLaneMaxLive : kLaneMaxLive;
 }
 // structure classes the lane kernel takes (the rest run on tiles), and per
 // module (one generated kernel)
@@ -1862,7 +1866,7 @@ std::vector<std::pair<uint32_t, double>> group_options(const LaneShape& sh, int 
   for (uint32_t G = 1; G <= kLaneWave; G *= 2) {
     LaneShape t = sh;
     if (!lane_group(t, G)) continue;
-    if (lane_live(t) > lane_max_live()) continue;
+    if (lane_live(t) > lane_max_live(G)) continue;
     out.push_back({G, lane_step_cost(t, bits)});
   }
   return out;
@@ -1907,7 +1911,7 @@ uint64_t lane_plan_sig(const pasif_driver* d, bool adjoint, int bits) {
   g.word(pack_key(const_cast<pasif_driver*>(d), adjoint));
   g.word(uint64_t(bits));
   g.word(uint64_t(int64_t(d->dev)));
-  g.word(lane_max_live());
+  g.word(lane_max_live(1));
   if (const char* f = std::getenv("PASIF_JIT_FLAGS"))
     for (const char* c = f; *c; ++c) g.word(uint64_t(uint8_t(*c)));
   auto rows = [&](const RowTerms& rt) {
@@ -2202,7 +2206,7 @@ bool lane_plan(pasif_driver* d, bool adjoint) {
     LaneShape& sh = all[c];
     // lane_group == 1: one lane per instance only (workgroups of waves for
     // classes that do not fit one lane)
-    const bool fits = d->lane_group == 1 ? sh.live_values() <= lane_max_live()
+    const bool fits = d->lane_group == 1 ? sh.live_values() <= lane_max_live(1)
                                          : !group_options(sh, bits).empty();
     if (fits) {
       need[c] = 1;  // one lane or a group of lanes per instance
@@ -2282,7 +2286,7 @@ bool lane_plan(pasif_driver* d, bool adjoint) {
       const int lay = need[cx] == 1 ? 0 : 1;
       uint32_t wu = 0;  // waves the union needs
       if (lay == 0) {
-        wu = (d->lane_group == 1 ? U.live_values() <= lane_max_live()
+        wu = (d->lane_group == 1 ? U.live_values() <= lane_max_live(1)
                                  : !group_options(U, bits).empty())
                  ? 1u
                  : 0u;
@@ -2705,9 +2709,11 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
     uint32_t* nao = reinterpret_cast<uint32_t*>(host.data() + f.na);
     std::fill(ex, ex + st, -1);
     const double eps = std::numeric_limits<R>::epsilon();
-    // lane slot r of position p of a group side -> the system's row
+    // lane slot r of position p of a group side -> the system's row (none:
+    // the largest number, whose state is 0)
     auto slot_row = [](const GSide& gs, uint32_t r, uint32_t p) {
-      return r < gs.RL ? gs.band[r] + p * gs.stride[r] : gs.shared[r - gs.RL];
+      if (r >= gs.RL) return gs.shared[r - gs.RL];
+      return p < gs.held[r] ? gs.band[r] + p * gs.stride[r] : ~0u;
     };
     // bounds and per-instance words, in order
     for (uint32_t i = 0; i < L->count; ++i) {
@@ -2747,9 +2753,11 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
               const size_t col = size_t(i) * G + p;
               lane_group_coefs(sh.gf, cv, p, lv);
               for (uint32_t t = 0; t < TF; ++t) cf[size_t(t) * st + col] = R(lv[t]);
-              for (uint32_t r = 0; r < L->nf; ++r)
+              for (uint32_t r = 0; r < L->nf; ++r) {
+                const uint32_t row = slot_row(sh.gf, r, p);
                 qf[size_t(r) * st + col] =
-                    R(d->fwd.init[d->fwd.off[in.sys] + slot_row(sh.gf, r, p)]);
+                    row < sh.f.n ? R(d->fwd.init[d->fwd.off[in.sys] + row]) : R(0);
+              }
             }
           } else {
             for (uint32_t t = 0; t < TF; ++t) cf[size_t(t) * st + i] = R(cv[t]);

@@ -171,6 +171,44 @@ void blocked_bands(uint32_t n, uint32_t G, uint32_t lo, uint32_t m, std::vector<
   for (; g < n; ++g) shared->push_back(g);
 }
 
+// Blocks of exactly len rows from lo while they fit, position p holding m =
+// ceil(len / G) rows m p .. of each: the last positions hold fewer or none.
+// Rows that belong together (a chain's displacements, its velocities) keep
+// their positions whatever the length, where whole bands would leave len mod G
+// m rows to every lane of the group and a sum over it per stage.
+void padded_bands(uint32_t n, uint32_t G, uint32_t lo, uint32_t len, std::vector<uint32_t>* band,
+                  std::vector<uint32_t>* stride, std::vector<uint32_t>* held,
+                  std::vector<uint32_t>* shared) {
+  const uint32_t m = (len + G - 1) / G;
+  uint32_t g = lo;
+  for (; g + len <= n; g += len)
+    for (uint32_t j = 0; j < std::min(m, len); ++j) {
+      band->push_back(g + j);
+      stride->push_back(m);
+      held->push_back((len - j + m - 1) / m);
+    }
+  for (; g < n; ++g) shared->push_back(g);
+}
+
+// Lengths of runs of rows that belong together: the commonest distances
+// between a row and its terms' factors (a chain's velocity rows read the
+// displacements a chain's length before them), neighbours apart.
+std::vector<uint32_t> run_lengths(const LaneSide& sd) {
+  std::map<uint32_t, uint32_t> count;
+  for (uint32_t g = 0; g < sd.n; ++g)
+    for (const LaneTerm& t : sd.rows[g])
+      if (t.kind == 0) {
+        const uint32_t d = t.f[0] > g ? t.f[0] - g : g - t.f[0];
+        if (d > 1) ++count[d];
+      }
+  std::vector<std::pair<uint32_t, uint32_t>> v;
+  for (const auto& c : count) v.emplace_back(c.second, c.first);
+  std::sort(v.rbegin(), v.rend());
+  std::vector<uint32_t> out;
+  for (size_t i = 0; i < std::min<size_t>(2, v.size()); ++i) out.push_back(v[i].second);
+  return out;
+}
+
 // Lane slot and group position of every row of a side.
 struct GMap {
   std::vector<uint32_t> slot, pos;
@@ -183,7 +221,7 @@ GMap group_map(uint32_t n, uint32_t G, const GSide& gs) {
   m.pos.assign(n, 0);
   m.shared.assign(n, false);
   for (uint32_t r = 0; r < gs.RL; ++r)
-    for (uint32_t p = 0; p < G; ++p) {
+    for (uint32_t p = 0; p < gs.held[r]; ++p) {
       m.slot[gs.band[r] + p * gs.stride[r]] = r;
       m.pos[gs.band[r] + p * gs.stride[r]] = p;
     }
@@ -244,7 +282,7 @@ void build_gside(const LaneSide& sd, uint32_t G, const GMap& own, const GMap& se
   for (uint32_t r = 0; r < gs->RL; ++r) {
     GRow& row = gs->rows[r];
     std::map<Key, size_t> where;
-    for (uint32_t p = 0; p < G; ++p) {
+    for (uint32_t p = 0; p < gs->held[r]; ++p) {
       const uint32_t g = gs->band[r] + p * gs->stride[r];
       std::map<Key, uint32_t> occ;
       for (size_t e = 0; e < sd.rows[g].size(); ++e)
@@ -411,29 +449,40 @@ double gside_step_cost(const GSide& gs, uint32_t G, bool forward, int bits) {
 bool best_gside(const LaneSide& sd, uint32_t G, const GSide* mirror, uint32_t nmirror,
                 const GMap* setp, int bits, GSide* out) {
   struct Plan {
-    std::vector<uint32_t> band, stride, shared;
+    std::vector<uint32_t> band, stride, held, shared;
   };
   std::vector<Plan> plans;
+  const std::vector<uint32_t> runs = run_lengths(sd);
   // rows from lo: dynamic programming over consecutive bands, or aligned
   // blocks of G m rows for m = 1, 2, 4, ...
   auto from = [&](const Plan& head, uint32_t lo) {
     Plan pl = head;
     plan_bands(sd, G, lo, &pl.band, &pl.shared);
     pl.stride.resize(pl.band.size(), 1u);
+    pl.held.resize(pl.band.size(), G);
     plans.push_back(pl);
     for (uint32_t m = 1; lo + G * m <= sd.n; m *= 2) {
       Plan q = head;
       blocked_bands(sd.n, G, lo, m, &q.band, &q.stride, &q.shared);
+      q.held.resize(q.band.size(), G);
+      plans.push_back(q);
+    }
+    for (uint32_t len : runs) {
+      if (lo + len > sd.n) continue;
+      Plan q = head;
+      padded_bands(sd.n, G, lo, len, &q.band, &q.stride, &q.held, &q.shared);
       plans.push_back(q);
     }
   };
   from(Plan(), 0);
-  if (mirror && nmirror <= sd.n) from(Plan{mirror->band, mirror->stride, mirror->shared}, nmirror);
+  if (mirror && nmirror <= sd.n) 
+    from(Plan{mirror->band, mirror->stride, mirror->held, mirror->shared}, nmirror);
   double best = -1;
   for (auto& pl : plans) {
     GSide gs;
     gs.band = pl.band;
     gs.stride = pl.stride;
+    gs.held = pl.held;
     gs.shared = pl.shared;
     std::sort(gs.shared.begin(), gs.shared.end());
     gs.RL = uint32_t(gs.band.size());
@@ -1101,10 +1150,12 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   // output row of lane slot r: band slots hold row rowf(r) + p stridef(r), a
   // shared slot's row is written by position 0 only (-1 elsewhere)
   auto orow_f = [&](int r) -> int {
-    return r < S::RLF ? S::rowf(r) + (int)p * S::stridef(r) : (p == 0u ? S::rowf(r) : -1);
+    if (r >= S::RLF) return p == 0u ? S::rowf(r) : -1;
+    return S::heldf(r) == G || p < S::heldf(r) ? S::rowf(r) + (int)p * S::stridef(r) : -1;
   };
   auto orow_a = [&](int r) -> int {
-    return r < S::RLA ? S::rowa(r) + (int)p * S::stridea(r) : (p == 0u ? S::rowa(r) : -1);
+    if (r >= S::RLA) return p == 0u ? S::rowa(r) : -1;
+    return S::helda(r) == G || p < S::helda(r) ? S::rowa(r) + (int)p * S::stridea(r) : -1;
   };
   // a shared sink is the sum of its lanes' parts (whole groups reach this);
   // the row's value at the start belongs to position 0
@@ -1321,8 +1372,9 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         // A taken branch costs a lone wave about as much as eight instructions
         // (two-DOF: 2.95 -> 2.59 ms at four steps a turn, one wave of 64
         // oscillators 1.37 -> 1.19, uneven batch in FP32 2.49 -> 2.25).
-        // Compile time keeps it to the loops that take most steps.
-        if constexpr (ALL && MODE != mFull)
+        // Compile time keeps it to the loops that take most steps, and to steps
+        // short enough for it to show (TURN_F: up to 200 instructions).
+        if constexpr (ALL && MODE != mFull && S::TURN_F)
           while (n + 4u <= stop) {
             one();
             one();
@@ -1573,7 +1625,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         // four a turn as forward: a state between two of them is read once
         // (8,192 16-DOF chains x 10,000 steps 13.0 -> 12.5 ms, uneven batch
         // 8.6 -> 8.1)
-        if constexpr (ALL)
+        if constexpr (ALL && S::TURN_A)
           while (n >= stop + 4u) {
             one();
             one();
@@ -2684,7 +2736,10 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
     if (!mw) {
       kf = grp ? group_kinds(sh.gf, true) : one_lane_kinds(sh, true);
       if (sh.adjoint) ka = grp ? group_kinds(sh.ga, false) : one_lane_kinds(sh, false);
-      o << ", NSEG = " << lane_seg_rows(sh, &segmap) << ", NLIN = " << kf.nlin;
+      const double fc = lane_forward_cost(sh, bits);
+      const double ac = sh.adjoint ? lane_step_cost(sh, bits) - 2.0 * fc : 0.0;
+      o << ", NSEG = " << lane_seg_rows(sh, &segmap) << ", NLIN = " << kf.nlin
+        << ", TURN_F = " << (fc <= 200.0 ? 1 : 0) << ", TURN_A = " << (ac <= 200.0 ? 1 : 0);
     }
     o << " };\n";
     if (!mw) {
@@ -2704,11 +2759,17 @@ std::string lane_source(const std::vector<LaneShape>& shapes, int bits, const La
           << ternary_map(sh.gf.stride) << "; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridea(int r) { return "
           << ternary_map(sh.ga.stride) << "; }\n";
+        o << "  static __device__ __forceinline__ constexpr u32 heldf(int r) { return "
+          << ternary_map(sh.gf.held) << "; }\n";
+        o << "  static __device__ __forceinline__ constexpr u32 helda(int r) { return "
+          << ternary_map(sh.ga.held) << "; }\n";
       } else {
         o << "  static __device__ __forceinline__ constexpr int rowf(int r) { return r; }\n";
         o << "  static __device__ __forceinline__ constexpr int rowa(int r) { return r; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridef(int) { return 1; }\n";
         o << "  static __device__ __forceinline__ constexpr int stridea(int) { return 1; }\n";
+        o << "  static __device__ __forceinline__ constexpr u32 heldf(int) { return 1u; }\n";
+        o << "  static __device__ __forceinline__ constexpr u32 helda(int) { return 1u; }\n";
       }
       auto rows_of = [&](const char* name, const std::vector<uint8_t>& v) {
         std::string e = "false";

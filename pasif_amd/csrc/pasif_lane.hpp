@@ -125,6 +125,7 @@ struct GSide {
   // which position p holds rows m p .. m p + m - 1
   std::vector<uint32_t> band;    // first row of each band slot
   std::vector<uint32_t> stride;  // row step between positions of each band slot
+  std::vector<uint32_t> held;    // positions that hold a row (the rest: zeros)
   std::vector<uint32_t> shared;  // row of each shared slot
   std::vector<GRow> rows;        // [RL + NS]
   // shared slots no term reads (forward: nor the adjoint's set points): the

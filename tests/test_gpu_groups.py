@@ -176,3 +176,28 @@ def test_staged_interpolation_windows(G, dof, W_):
     assert rel_err(q, oracle_run(w).q) < TOL64
     p.setSolver("graph", steps_per_launch=37, launches_per_graph=3)
     np.testing.assert_array_equal(p.getAmplitudes(), q)
+
+
+@pytest.mark.parametrize("G,d", [(4, 3), (8, 5), (16, 7), (16, 13), (32, 17), (64, 70), (64, 129),
+                                 (64, 150)])
+def test_lengths_no_group_divides(G, d):
+    """Chains whose length is not a multiple of the group: the last positions
+    hold fewer rows or none.  States, a trajectory, a window and gradients
+    against the oracle; each output row is written exactly once, beside its
+    neighbours in the output arrays."""
+    _case(f"padded G={G}, {d} DOF")
+    w = W.chains(5, d, 80, steps_per_sample=10)
+    p = _grouped(w, G)
+    src = p._laneSource(False)
+    held = src[src.index("u32 heldf(int r) { return"):].split(";")[0]
+    m = -(-d // G)
+    assert f"? {-(-d // m)}" in held, held
+    ref = oracle_run(w, save_steps=7, window=30)
+    q, mx = p.getMaxAmplitudes(window=30)
+    assert rel_err(q, ref.q) < TOL64
+    assert rel_err(mx, ref.maxabs) < TOL64
+    tr = p.getTrajectory(7)
+    assert rel_err(tr[1:].T, ref.traj.reshape(ref.traj.shape[0], -1)) < TOL64
+    J = ADJ.energy_gradient_inputs(w)
+    p = _grouped(w, G, True, J)
+    assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64

@@ -118,3 +118,17 @@ def test_rows_trajectory_window_and_fp32():
     w.exc_of_system = w.steps_of_system = None
     p = W.make_solver(w)
     _check(p.getAmplitudes(), oracle_run(w).q, _sizes(w) * 2, "cartesian")
+
+
+def test_rows_trajectory_and_window_of_a_system_beyond_lanes():
+    print("[gpu case] rows: 700-DOF chains, trajectory, window", flush=True)
+    w = W.chains(n_systems=2, d=700, steps=33, steps_per_sample=10)
+    w.steps_of_system = np.array([33, 20])
+    p = W.make_solver(w)
+    assert p.kernelInfo()["kernel"] == "big"
+    tr = p.getTrajectory(saveSteps=7)
+    ref = oracle_run(w, save_steps=7, window=12)
+    assert rel_err(tr[1:].T, ref.traj.reshape(ref.traj.shape[0], -1)) < 1e-10
+    q, mx = p.getMaxAmplitudes(window=12)
+    _check(q, ref.q, _sizes(w), "states beside the window")
+    _check(mx, ref.maxabs, _sizes(w), "window")
