@@ -3408,7 +3408,7 @@ uint32_t run_outputs(pasif_driver* d, bool adjoint, uint32_t save_steps) {
 // chip's work, whichever is longer; the pass itself runs at about 1.3 of
 // that), and what the lease grants.  Each class gets its share, its longest
 // waves first.  8,192 chains of 16 DOF x 10,000 steps (21 GB, the chip full):
-// 17.1 ms recomputed, 13.8 ms stored; 4,096 uneven systems 14.2 and 9.7 ms;
+// 15.1 ms recomputed, 12.4 ms stored; 4,096 uneven systems 9.5 and 7.0 ms;
 // a batch of one- and two-DOF systems that fills the chip moves 10 TB/s at
 // its forward rate and keeps most of its waves on checkpoints.
 constexpr double kPathRate = 4.5e12;
