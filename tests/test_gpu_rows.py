@@ -120,15 +120,14 @@ def test_rows_trajectory_window_and_fp32():
     _check(p.getAmplitudes(), oracle_run(w).q, _sizes(w) * 2, "cartesian")
 
 
-def test_rows_trajectory_and_window_of_a_system_beyond_lanes():
-    print("[gpu case] rows: 700-DOF chains, trajectory, window", flush=True)
-    w = W.chains(n_systems=2, d=700, steps=33, steps_per_sample=10)
-    w.steps_of_system = np.array([33, 20])
+def test_rows_trajectory_and_window_of_a_system_no_lane_layout_holds():
+    print("[gpu case] rows: dense couplings, trajectory, window", flush=True)
+    w = _dense(150, 150)
     p = W.make_solver(w)
     assert p.kernelInfo()["kernel"] == "big"
     tr = p.getTrajectory(saveSteps=7)
-    ref = oracle_run(w, save_steps=7, window=12)
+    ref = oracle_run(w, save_steps=7, window=20)
     assert rel_err(tr[1:].T, ref.traj.reshape(ref.traj.shape[0], -1)) < 1e-10
-    q, mx = p.getMaxAmplitudes(window=12)
+    q, mx = p.getMaxAmplitudes(window=20)
     _check(q, ref.q, _sizes(w), "states beside the window")
     _check(mx, ref.maxabs, _sizes(w), "window")
