@@ -1057,9 +1057,10 @@ __device__ __forceinline__ void exact_adj(R* lam, E eff, R h, R h2, R h6, bool a
 // state as the tile kernel.  S::G lanes integrate one instance (1: one
 // instance per lane); per-lane arrays (coefficients, states, checkpoints)
 // are indexed by the lane's column, per-instance ones (steps, excitation,
-// output bases) by the instance.  LDS: eb [STAGE][WAVE / G] staged samples
-// of the current chunk of steps, one column per instance (the next chunk is
-// prefetched into registers), then seg [K+1][NSEG][WAVE] (adjoint) the
+// output bases) by the instance.  LDS: wl [WTS] interpolation weights, eb
+// [STAGE][WAVE / G] staged samples of the current chunk of steps, one column
+// per instance (the next chunk is prefetched into registers), ft [FT][WAVE / G]
+// its forcing values (groups), then seg [K+1][NSEG][WAVE] (adjoint) the
 // recomputed segment's post-step states and, for the exact discrete
 // adjoint, seg3 [K][3][NSEG][WAVE] each step's stage inputs y2, y3, y4 (HBM
 // mirror sb likewise, by forward slot).
