@@ -2259,18 +2259,21 @@ void emit_forward_row(std::ostringstream& o, Monos& monos, const RowKinds& rk, u
   std::ostringstream pre;
   std::string e = factored(pre, monos, ts, base);
   if (gsum > 1 && !rk.sink[r]) e = "gsum<" + std::to_string(gsum) + "u>(" + e + ")";
-  if (rk.sink[r])
-    o << "    if constexpr (SINKS) {\n" << pre.str() << "    " << kr << " = " << e << ";\n    }\n";
-  else
-    o << pre.str() << "    " << kr << " = " << e << ";\n";
+  o << pre.str() << "    " << kr << " = " << e << ";\n";
 }
+
+// The sinks of a right-hand side follow its other rows in one block of their
+// own (left out of a recompute): what they need beyond the other rows' products
+// is shared among all of them, and declared where all of them see it.
+void emit_sinks_begin(std::ostringstream& o) { o << "    if constexpr (SINKS) {\n"; }
+void emit_sinks_end(std::ostringstream& o) { o << "    }\n"; }
 
 // Forward right-hand side of a one-lane class.
 void emit_rhs_forward(std::ostringstream& o, const LaneSide& sd, const RowKinds& rk) {
   const Slots sl = slots_of(sd);
   Monos monos;
-  // sinks last: the products they need are theirs alone or already there
-  for (int pass = 0; pass < 2; ++pass)
+  for (int pass = 0; pass < 2; ++pass) {
+    if (pass) emit_sinks_begin(o);
     for (uint32_t r = 0; r < sd.n; ++r) {
       if (int(rk.sink[r]) != pass) continue;
       std::vector<PTerm> ts;
@@ -2285,6 +2288,8 @@ void emit_rhs_forward(std::ostringstream& o, const LaneSide& sd, const RowKinds&
       emit_forward_row(o, monos, rk, r, ts,
                        sl.force[r] >= 0 ? "c[" + std::to_string(sl.force[r]) + "]" : "", 1);
     }
+    if (pass) emit_sinks_end(o);
+  }
 }
 
 RowKinds one_lane_kinds(const LaneShape& sh, bool forward) {
@@ -2482,6 +2487,7 @@ void emit_group_forward(std::ostringstream& o, const GSide& gs, uint32_t G, cons
   };
   Monos monos;
   for (int pass = 0; pass < 2; ++pass) {
+    if (pass) emit_sinks_begin(o);
     uint32_t t = 0;
     for (uint32_t r = 0; r < gs.nl(); ++r) {
       const GRow& row = gs.rows[r];
@@ -2501,6 +2507,7 @@ void emit_group_forward(std::ostringstream& o, const GSide& gs, uint32_t G, cons
       }
       t = tf + (row.force.empty() ? 0u : 1u);
     }
+    if (pass) emit_sinks_end(o);
   }
 }
 

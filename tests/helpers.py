@@ -8,6 +8,8 @@ from types import SimpleNamespace
 import numpy as np
 import scipy.sparse as sp
 
+from pasif_amd import workloads as W
+
 
 def tensor(dims, val, idx):
     return SimpleNamespace(dimensions=list(dims), val=list(val), indices=list(idx))
@@ -87,3 +89,24 @@ def loop_rhs(asm, S, X, u_dof):
             v = v + float(asm.force[i]) * u_dof[i]
         out.append(v)
     return out
+
+
+def two_probe_chains(n, d, steps):
+    """Chains with a second probe row, ``E2' = sum_i a_i v_i^2``: two rows that
+    no term reads, whose terms share the products of the velocities."""
+    w = W.chains(n, d, steps, steps_per_sample=10)
+    rng = np.random.default_rng(d)
+    N = 2 * d + 2
+    for s in range(n):
+        w.vecM[s] = sp.dia_matrix((np.ones(N), [0]), shape=(N, N))
+        for v in (w.vecB, w.vecK):
+            v[s] = sp.coo_matrix((v[s].data, (v[s].row, v[s].col)), shape=(N, N))
+        g = np.asarray(w.vecGamma[s].indices).reshape(-1, 3)
+        probe = [[N - 1, d + i, d + i] for i in range(d)]
+        w.vecGamma[s] = W._tensor([N] * 3,
+                                  np.append(w.vecGamma[s].val, rng.uniform(0.5, 1.0, d)),
+                                  np.concatenate([g, probe]))
+        w.vecLambda[s] = W._tensor([N] * 4, w.vecLambda[s].val, w.vecLambda[s].indices)
+        w.vecForce[s] = np.append(w.vecForce[s], 0.0)
+        w.vecQ0[s] = np.append(w.vecQ0[s], 0.0)
+    return w

@@ -14,6 +14,7 @@ from pasif_amd import workloads as W
 from tests.test_gpu_adjoint import oracle_gradient
 from tests.test_gpu_forward import TOL64, oracle_run, rel_err
 from tests.test_gpu_lane import _random_cartesian
+from tests.helpers import two_probe_chains
 
 pytestmark = pytest.mark.gpu
 
@@ -200,4 +201,26 @@ def test_lengths_no_group_divides(G, d):
     assert rel_err(tr[1:].T, ref.traj.reshape(ref.traj.shape[0], -1)) < TOL64
     J = ADJ.energy_gradient_inputs(w)
     p = _grouped(w, G, True, J)
+    assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64
+
+
+@pytest.mark.parametrize("G,d", [(1, 1), (1, 2), (2, 4), (4, 4)])
+def test_probes_that_share_products(G, d):
+    """Two rows that no term reads, their terms the same products of velocities:
+    states, a window and gradients of the second probe against the oracle."""
+    _case(f"two probes G={G}, {d} DOF")
+    w = two_probe_chains(9, d, 90)
+    w.steps_of_system = np.array([90, 1, 37, 90, 64, 2, 89, 16, 50])
+    ref = oracle_run(w, window=30)
+    p = W.make_solver(w)
+    p.setKernel("auto", G)
+    assert p.kernelInfo()["lanes_per_instance"] == [G]
+    q, mx = p.getMaxAmplitudes(window=30)
+    assert rel_err(q, ref.q) < TOL64
+    assert rel_err(mx, ref.maxabs) < TOL64
+    J = ADJ.energy_gradient_inputs(w)
+    p = W.make_solver(w)
+    p.setKernel("auto", G)
+    p.setJacobian(*J.as_args())
+    assert p.kernelInfo(True)["kernel"] == "lane"
     assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64

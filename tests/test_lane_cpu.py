@@ -10,6 +10,7 @@ import pytest
 from pasif_amd import _lib
 from pasif_amd import adjoint as ADJ
 from pasif_amd import workloads as W
+from tests.helpers import two_probe_chains
 
 
 def host_solver(w):
@@ -138,6 +139,19 @@ def test_group_layouts_compile_for_gfx950(maker, adjoint, G):
     assert f"G = {G}," in src
     p.setPrecision(32)
     p._laneSource(adjoint, compile=True)
+
+
+@pytest.mark.parametrize("d,G", [(1, 1), (2, 1), (2, 2), (4, 2), (4, 4)])
+def test_probes_that_share_products_compile(d, G):
+    # two rows no term reads, whose terms are the same products of velocities
+    w = two_probe_chains(12, d, 60)
+    p = host_solver(w)
+    p.setKernel("auto", G)
+    assert p.kernelInfo()["lanes_per_instance"] == [G]
+    p._laneSource(False, compile=True)
+    p.setJacobian(*ADJ.energy_gradient_inputs(w).as_args())
+    assert p.kernelInfo(True)["kernel"] == "lane"
+    p._laneSource(True, compile=True)
 
 
 def test_chain_group_program_is_the_stencil():
