@@ -181,6 +181,11 @@ int pasif_set_kernel(pasif_driver* d, int kernel);
  * (the lane kernel shortens it until a segment fits its LDS) */
 int pasif_kernel_info(pasif_driver* d, int adjoint, int* kernel, uint32_t* classes,
                       uint32_t* checkpoint_every);
+/* what PASIF_KERNEL_BIG stands for in the packed problem (extension): instances
+ * with their stage vectors in LDS, instances with every vector in device
+ * memory, and the LDS bytes of the former's launch */
+int pasif_row_info(pasif_driver* d, int adjoint, uint32_t* rows, uint32_t* big,
+                   size_t* lds_bytes);
 /* Lanes per instance in the lane kernel (extension).  0 (default): chosen per
  * structure class from a cost model (one lane per instance while the GPU's
  * SIMDs are busy; a group of 2..64 lanes, rows in bands across the group and

@@ -280,6 +280,15 @@ class __GpuDriver:  # noqa: N801  (the reference's class name)
         return {"kernel": name, "classes": ncls.value, "checkpoint_every": ck.value,
                 "lanes_per_instance": groups}
 
+    def _rowInfo(self, adjoint: bool = False) -> dict:
+        """Instances of the row-parallel path with their stage vectors in LDS
+        (``rows``) and with every vector in device memory (``big``), and the
+        LDS bytes of the former's launch."""
+        r, b, lds = C.c_uint32(0), C.c_uint32(0), C.c_size_t(0)
+        self._chk(self._pl.pasif_row_info(self._h, int(adjoint), C.byref(r), C.byref(b),
+                                          C.byref(lds)))
+        return {"rows": r.value, "big": b.value, "lds": lds.value}
+
     def _setAdjointMode(self, mode: str = "reference"):
         modes = {"reference": 0, "exact": 1}
         if mode not in modes:

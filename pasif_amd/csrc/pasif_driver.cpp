@@ -258,7 +258,7 @@ struct Packed {
   uint32_t nrow = 0;
   DevBuf r_inst, r_blk, r_val, r_word, r_init, r_force, r_row, r_piece, r_sink;
   uint64_t r_vec_f = 0, r_vec_a = 0, r_ck = 0, r_seg = 0, r_path = 0;
-  uint32_t r_tmax = 0, r_every = 1, r_waves = 0, r_slots = 0, r_ys = 0, r_xs = 0, r_ps = 0;
+  uint32_t r_tmax = 0, r_every = 1, r_waves = 0, r_slots = 0, r_lds = 0;
   bool r_resident = false;
   // some system is on the row-parallel path because nothing else takes it
   // (or because the caller asked for that path): no per-step outputs, no
@@ -1480,11 +1480,12 @@ void pack_rows(pasif_driver* d, bool adjoint) {
   struct Prog {
     RowProg f, a;
     uint32_t waves;
+    RowLds lds;
   };
   std::map<uint32_t, Prog> progs;
   std::vector<RowInst> ri(inst.size());
   pk.r_vec_f = pk.r_vec_a = pk.r_ck = pk.r_seg = pk.r_path = 0;
-  pk.r_waves = pk.r_slots = pk.r_ys = pk.r_xs = pk.r_ps = 0;
+  pk.r_waves = pk.r_slots = pk.r_lds = 0;
   pk.r_resident = true;
   const uint32_t per = adjoint && d->adj_mode ? 4u : 1u;  // values kept per step and row
   for (size_t i = 0; i < inst.size(); ++i) {
@@ -1505,21 +1506,22 @@ void pack_rows(pasif_driver* d, bool adjoint) {
       p.waves = (units + 64u * slots - 1) / (64u * slots);
       pk.r_waves = std::max(pk.r_waves, p.waves);
       pk.r_slots = std::max(pk.r_slots, slots);
-      pk.r_ys = std::max(pk.r_ys, zy + 1u);
-      if (adjoint) pk.r_xs = std::max(pk.r_xs, uf.pub + 1u);
+      p.lds = row_lds(uf, adjoint ? &ua : nullptr);
+      pk.r_lds = std::max(pk.r_lds, uint32_t(p.lds.values()));
       for (const RowUnits* u : {&uf, &ua})
         for (const RowUnit& x : u->main)
           if (x.cnt[0] > kRowRes1 || x.cnt[1] > kRowRes2 || x.cnt[2] > kRowRes3 ||
               x.cnt[3] > kRowRes4)
             pk.r_resident = false;
-      for (const RowUnits* u : {&uf, &ua})
-        pk.r_ps = std::max<uint32_t>(pk.r_ps, uint32_t(std::max<size_t>(u->aux.size(), u->pieces)));
       it = progs.emplace(in.sys, p).first;
     }
     RowInst& r = ri[i];
     r.f = it->second.f;
     r.a = it->second.a;
     r.waves = it->second.waves;
+    r.ys = it->second.lds.ys;
+    r.xs = it->second.lds.xs;
+    r.ps = it->second.lds.ps;
     r.n_f = d->fwd.size[in.sys];
     r.steps = in.steps;
     r.out_f = in.out_f;
@@ -3185,9 +3187,7 @@ RowArgs<R> row_run_args(pasif_driver* d, bool adjoint, uint32_t save_steps, uint
   a.out_len = pk.out_len_f;
   a.ck_every = pk.r_every;
   a.resident = pk.r_resident ? 1u : 0u;
-  a.y_slots = pk.r_ys;
-  a.x_slots = pk.r_xs;
-  a.part_slots = pk.r_ps;
+  a.lds_slots = pk.r_lds;
   uint64_t work = pk.r_tmax;
   if (adjoint) {
     a.vec_a = static_cast<R*>(mem.get(d->rvec_a, size_t(pk.r_vec_a) * el));
@@ -4314,6 +4314,16 @@ int pasif_kernel_info(pasif_driver* d, int adjoint, int* kernel, uint32_t* class
                           : pk.lane ? pk.lseg
                           : (pk.big && !pk.tile) ? (pk.rows ? pk.r_every : pk.b_every)
                                                  : (d->ck_every ? d->ck_every : 256u);
+  });
+}
+
+int pasif_row_info(pasif_driver* d, int adjoint, uint32_t* rows, uint32_t* big, size_t* lds_bytes) {
+  return guarded(d, [&] {
+    ensure_packed(d, adjoint != 0);
+    const Packed& pk = d->pk;
+    if (rows) *rows = pk.nrow;
+    if (big) *big = pk.nbig;
+    if (lds_bytes) *lds_bytes = pk.rows ? size_t(pk.r_lds) * (d->precision / 8) : 0;
   });
 }
 

@@ -297,10 +297,10 @@ __global__ void __launch_bounds__(kRowThreads) row_kernel(RowArgs<R> a) {
   const uint32_t NT = NW * 64u, tid = threadIdx.x;
   constexpr uint32_t EL = sizeof(R);
   unsigned char* const Yb = row_smem;
-  const uint32_t ys = a.y_slots * EL, xs = a.x_slots * EL;
+  const uint32_t ys = runi(I.ys) * EL, xs = runi(I.xs) * EL;
   unsigned char* const Xb = Yb + 2u * ys;
   R* const part = reinterpret_cast<R*>(Xb + 2u * xs);
-  R* const ft = part + a.part_slots;
+  R* const ft = part + runi(I.ps);
 
   // unit of slot j, computed where it is used: the slots are unrolled, and
   // addresses derived from it ahead of the step loop would be held (or
@@ -737,7 +737,7 @@ template <typename R>
 hipError_t launch_rows_impl(const RowArgs<R>& a, uint32_t ninst, uint32_t waves, uint32_t slots,
                             hipStream_t s) {
   if (ninst == 0u) return hipSuccess;
-  const size_t lds = row_lds_values(a.y_slots, a.x_slots, a.part_slots) * sizeof(R);
+  const size_t lds = size_t(a.lds_slots) * sizeof(R);
   if (waves == 0u || waves * 64u > kRowThreads || slots > kRowSlots || lds > kMaxLdsBytes)
     return hipErrorInvalidValue;
   return a.adjoint ? launch_rows_adj<R, true>(a, ninst, waves, slots, lds, s)

@@ -53,6 +53,11 @@ struct RowInst {
   uint64_t ck, seg, path;  // checkpoints, recomputed segment, stored path
   uint32_t waves;          // waves of the workgroup that work
   uint32_t n_f, steps, out_f, out_a;
+  // LDS values of each stage buffer, each set-point buffer (adjoint) and the
+  // sums: the instance's own, since a launch's instances need not be alike (a
+  // long chain's stage buffers and the many pieces of a dense system's rows do
+  // not fit beside each other, and either alone does)
+  uint32_t ys, xs, ps;
   int32_t exc;
 };
 
@@ -71,9 +76,9 @@ struct RowArgs {
   const R* interp;         // [2][interp_w] or null (zero-order hold)
   uint32_t exc_len, interp_w;
   R h, h2, h6;
-  R* vec_f;                // per instance [2][units_f]: state, running max
+  R* vec_f;                // per instance [2][units_f]: state, running max, then the
+                           // running max of each multi-piece sink
   R* vec_a;                // per instance [units_a]
-  R* smax;                 // per instance: running max of each multi-piece sink
   R* ckpt;                 // per instance [ceil(steps / K)][n_f]
   R* segbuf;               // recompute: [K + 1][pub] (exact: [K][4][pub]); whole
                            // path (store): [steps + 1][pub] (exact: [steps][4][pub])
@@ -87,13 +92,13 @@ struct RowArgs {
   uint32_t out_len, save_every, nslots, window;
   uint32_t budget, ck_every, adjoint, exact;
   uint32_t resident;       // every block within kRowRes*
-  uint32_t y_slots, x_slots, part_slots;  // LDS rows of each stage / set-point buffer, sums
+  uint32_t lds_slots;      // LDS values of the instance that needs most
 };
 
 // LDS values: two stage buffers, two set-point buffers (adjoint), sums, the
 // forcing table
-inline size_t row_lds_values(uint32_t y_slots, uint32_t x_slots, uint32_t part_slots) {
-  return 2 * size_t(y_slots) + 2 * size_t(x_slots) + part_slots + 3 * kRowChunk;
+inline size_t row_lds_values(uint32_t ys, uint32_t xs, uint32_t ps) {
+  return 2 * size_t(ys) + 2 * size_t(xs) + ps + 3 * kRowChunk;
 }
 
 hipError_t launch_rows(const RowArgs<double>& a, uint32_t ninst, uint32_t waves, uint32_t slots,

@@ -129,18 +129,31 @@ inline RowUnits row_units(const RowTerms& rt, uint32_t s, const std::vector<uint
   return o;
 }
 
+// LDS values of an instance's buffers (RowInst): a slot more than published
+// rows holds the 0 that padding terms read.
+struct RowLds {
+  uint32_t ys, xs, ps;
+  size_t values() const { return row_lds_values(ys, xs, ps); }
+};
+inline RowLds row_lds(const RowUnits& f, const RowUnits* a) {
+  RowLds l;
+  l.ys = std::max(f.pub, a ? a->pub : 0u) + 1u;
+  l.xs = a ? f.pub + 1u : 0u;
+  size_t part = std::max<size_t>(f.aux.size(), f.pieces);
+  if (a) part = std::max<size_t>(part, std::max<size_t>(a->aux.size(), a->pieces));
+  l.ps = uint32_t(part);
+  return l;
+}
+
 // Whether the kernel can hold an instance with these units: threads and
 // slots, 16-bit LDS offsets and piece ranges, LDS size.
 inline bool row_units_fit(const RowUnits& f, const RowUnits* a, size_t el) {
   const size_t most = size_t(kRowThreads) * kRowSlots;
-  const uint32_t pa = a ? a->pub : 0u;
   if (f.main.size() > most || (a && a->main.size() > most)) return false;
   if (f.aux.size() > 0xFFFF || (a && a->aux.size() > 0xFFFF)) return false;
-  const size_t ysl = std::max(f.pub, pa) + 1u, xsl = a ? f.pub + 1u : 0u;
-  if (ysl * el > 0xFFFF || xsl * el > 0xFFFF) return false;
-  size_t part = std::max<size_t>(f.aux.size(), f.pieces);
-  if (a) part = std::max<size_t>(part, std::max<size_t>(a->aux.size(), a->pieces));
-  return row_lds_values(uint32_t(ysl), uint32_t(xsl), uint32_t(part)) * el <= kMaxLdsBytes;
+  const RowLds l = row_lds(f, a);
+  return size_t(l.ys) * el <= 0xFFFF && size_t(l.xs) * el <= 0xFFFF &&
+         l.values() * el <= kMaxLdsBytes;
 }
 
 // Packed program arrays of many sides.

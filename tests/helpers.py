@@ -110,3 +110,36 @@ def two_probe_chains(n, d, steps):
         w.vecForce[s] = np.append(w.vecForce[s], 0.0)
         w.vecQ0[s] = np.append(w.vecQ0[s], 0.0)
     return w
+
+
+def dense_chain(d, steps, seed=0):
+    """One chain whose velocities are all coupled (dense K and B): rows of many
+    terms, each split in pieces, and an energy row of d^2 terms."""
+    rng = np.random.default_rng(seed)
+    w = W.chains(1, d, steps, steps_per_sample=10, seed=seed + 1)
+    n = 2 * d + 1
+    r, c = np.divmod(np.arange(d * d), d)
+    B = 0.02 * np.eye(d) + 0.001 * rng.normal(size=(d, d))
+    w.vecK[0] = sp.coo_matrix((((2.0 * np.eye(d)) + 0.01 * rng.normal(size=(d, d))).reshape(-1),
+                               (d + r, c)), shape=(n, n))
+    w.vecB[0] = sp.coo_matrix((np.append(np.full(d, -1.0), B.reshape(-1)),
+                               (np.append(np.arange(d), d + r), np.append(d + np.arange(d), d + c))),
+                              shape=(n, n))
+    g = np.asarray(w.vecGamma[0].indices).reshape(-1, 3)
+    keep = g[:, 0] < 2 * d
+    w.vecGamma[0] = W._tensor([n] * 3,
+                              np.append(w.vecGamma[0].val[keep], -B.reshape(-1)),
+                              np.concatenate([g[keep], np.stack([np.full(d * d, 2 * d), d + r,
+                                                                 d + c], 1)]))
+    return w
+
+
+def side_by_side(ws, steps_of_system):
+    """The systems of several workloads of one sample rate in one, each on its
+    own excitation."""
+    cols = [sum((list(getattr(w, a)) for w in ws), [])
+            for a in ("vecM", "vecB", "vecK", "vecGamma", "vecLambda", "vecForce", "vecQ0")]
+    exc = np.concatenate([w.excitations for w in ws])
+    return W.Workload("side by side", *cols, exc, ws[0].sample_rate, max(steps_of_system),
+                      exc_of_system=np.arange(len(exc)),
+                      steps_of_system=np.asarray(steps_of_system), interp=ws[0].interp)

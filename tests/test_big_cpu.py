@@ -7,6 +7,7 @@ import pytest
 
 from pasif_amd import adjoint as ADJ
 from pasif_amd import workloads as W
+from tests.helpers import dense_chain, side_by_side
 from tests.test_memory_plan import _host
 
 
@@ -51,3 +52,21 @@ def test_small_systems_stay_on_tiles_beside_a_large_one():
     big_only = p._runFootprint(True)["ckpt"]
     assert big_only == (3 * 10 * 9 + 4 * 1401) * 8
     assert ADJ is not None
+
+
+def test_a_long_chain_beside_a_dense_system_fits_one_launch():
+    # a long chain's stage buffers take most of LDS and a dense system's many
+    # pieces a good part: the launch needs what one instance needs, not the sum
+    # of the largest of each buffer over the instances
+    long = W.chains(1, 2001, 20, steps_per_sample=10)
+    dense = dense_chain(150, 20)
+    for kernel in ("auto", "big"):
+        lds = []
+        for w in (side_by_side([long], [20]), side_by_side([dense], [20]),
+                  side_by_side([long, dense], [20, 17])):
+            p = _host(w)
+            p.setKernel(kernel)
+            i = p._rowInfo(True)
+            assert i["big"] == 0 and i["rows"] == w.n_systems
+            lds.append(i["lds"])
+        assert lds[2] == max(lds[:2]) <= 160 * 1024

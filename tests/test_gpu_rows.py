@@ -12,7 +12,7 @@ from oracle import parity as PAR
 from pasif_amd import adjoint as ADJ
 from pasif_amd import workloads as W
 from pasif_amd.PASIf import coo_tensor
-from tests.helpers import random_system
+from tests.helpers import dense_chain, random_system, side_by_side
 from tests.test_gpu_adjoint import oracle_gradient
 from tests.test_gpu_exact_adjoint import oracle_exact
 from tests.test_gpu_forward import oracle_run, rel_err
@@ -131,3 +131,23 @@ def test_rows_trajectory_and_window_of_a_system_no_lane_layout_holds():
     q, mx = p.getMaxAmplitudes(window=20)
     _check(q, ref.q, _sizes(w), "states beside the window")
     _check(mx, ref.maxabs, _sizes(w), "window")
+
+
+@pytest.mark.parametrize("kernel", ["auto", "big"])
+def test_rows_a_long_chain_beside_a_dense_system(kernel):
+    """Instances of one launch that divide LDS differently: a chain of 2,001 DOF
+    and a dense system of 150, which do not fit LDS together."""
+    print(f"[gpu case] rows: 2001-DOF chain beside a dense 150-DOF system, {kernel}", flush=True)
+    w = side_by_side([W.chains(1, 2001, 20, steps_per_sample=10), dense_chain(150, 20)], [12, 20])
+    J = ADJ.energy_gradient_inputs(w)
+    p = W.make_solver(w)
+    p.setKernel(kernel)
+    _check(p.getAmplitudes(), oracle_run(w).q, _sizes(w), "forward")
+    p.setJacobian(*J.as_args())
+    assert p._rowInfo(True)["rows"] == 2
+    g = p.getGradient()
+    _check(g, oracle_gradient(w, J, 16), J.sizes, "reference adjoint")
+    p.setTuning(checkpoint_every=5)
+    np.testing.assert_array_equal(p.getGradient(), g)
+    p.setAdjointMode("exact")
+    _check(p.getGradient(), oracle_exact(w, J, 16), J.sizes, "exact adjoint")
