@@ -1,5 +1,7 @@
 """The row-parallel path (``setKernel("big")``, and what ``"auto"`` runs for
-systems too large for a tile) on the GPU against the oracle: FP64 within
+systems too large for a tile) on the GPU against the oracle -- systems whose
+stage vectors LDS holds, and larger ones with every vector in device memory,
+alone and beside each other: FP64 within
 1e-10 per output (``oracle.parity``) for the forward amplitudes, the
 reference adjoint recursion and the exact discrete adjoint; bitwise
 invariant under the checkpoint interval and the solver, with uneven step
@@ -12,6 +14,7 @@ import pytest
 from oracle import parity as PAR
 from pasif_amd import adjoint as ADJ
 from pasif_amd import workloads as W
+from tests.helpers import dense_chain, side_by_side
 from tests.test_gpu_adjoint import oracle_gradient
 from tests.test_gpu_exact_adjoint import oracle_exact
 from tests.test_gpu_forward import oracle_run
@@ -119,3 +122,50 @@ def test_big_chain_of_2001_dof_alone_and_beside_small_chains():
     pm.setAdjointMode("exact")
     assert pm.kernelInfo(adjoint=True)["kernel"] == "mixed"
     _check(pm.getGradient(), oracle_exact(wm, Jm, 128), Jm.sizes, "mixed exact adjoint")
+
+
+def test_device_memory_forward_past_the_lds_limit():
+    _case("big: 4100-DOF chain x 6 steps, forward, vectors in device memory")
+    w = W.chains(n_systems=2, d=4100, steps=6, steps_per_sample=2)
+    w.steps_of_system = np.array([6, 1])
+    w.vecQ0 = [np.random.default_rng(s).normal(0, 0.3, 8201) for s in range(2)]
+    p = W.make_solver(w)
+    assert p._rowInfo() == {"rows": 0, "big": 2, "lds": 0}
+    _check(p.getAmplitudes(), oracle_run(w).q, _sizes(w), "4100-DOF forward")
+
+
+def test_device_memory_adjoints_past_the_lds_limit():
+    _case("big: 2100-DOF chain x 8 steps, both adjoints, vectors in device memory")
+    w = W.chains(n_systems=1, d=2100, steps=8, steps_per_sample=2)
+    J = ADJ.energy_gradient_inputs(w)
+    p = W.make_solver(w)
+    p.setKernel("big")
+    p.setJacobian(*J.as_args())
+    assert p._rowInfo(True) == {"rows": 0, "big": 1, "lds": 0}
+    g = p.getGradient()
+    _check(g, oracle_gradient(w, J, 16), J.sizes, "reference")
+    for k in (1, 3):
+        p.setTuning(checkpoint_every=k)
+        np.testing.assert_array_equal(p.getGradient(), g)
+    p.setSolver("plain")
+    np.testing.assert_array_equal(p.getGradient(), g)
+    p.setSolver("persistent")
+    p.setAdjointMode("exact")
+    _check(p.getGradient(), oracle_exact(w, J, 16), J.sizes, "exact")
+
+
+def test_device_memory_beside_lds_and_lane_systems():
+    _case("big: 2100-DOF chain beside a dense 150-DOF system and 8-DOF chains")
+    w = side_by_side([W.chains(3, 8, 20, steps_per_sample=10),
+                      W.chains(1, 2100, 20, steps_per_sample=10), dense_chain(150, 20)],
+                     [20, 13, 1, 8, 19])
+    J = ADJ.energy_gradient_inputs(w)
+    p = W.make_solver(w)
+    assert p.kernelInfo()["kernel"] == "mixed"
+    _check(p.getAmplitudes(), oracle_run(w).q, _sizes(w), "forward")
+    p.setJacobian(*J.as_args())
+    info = p._rowInfo(True)
+    assert (info["rows"], info["big"]) == (1, 1), info
+    _check(p.getGradient(), oracle_gradient(w, J, 16), J.sizes, "reference adjoint")
+    p.setAdjointMode("exact")
+    _check(p.getGradient(), oracle_exact(w, J, 16), J.sizes, "exact adjoint")
