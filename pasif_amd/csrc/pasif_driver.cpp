@@ -566,9 +566,10 @@ int guarded(pasif_driver* d, F&& f) {
 // driver clears freed device memory before it hands it out again (freeing
 // and allocating 32 GB in turn took 0.9 s a time).  Bounded: a lease is
 // granted only while all of it together stays within 32 GiB and the new
-// buffer within a quarter of the free memory; without one a solve recomputes
-// from checkpoints.  Given back when an allocation of the library's needs
-// the room and when the device's last handle is destroyed.
+// buffer within a quarter of the memory free once the solve holds its run
+// buffers; without one a solve recomputes from checkpoints.  Given back when
+// an allocation of the library's needs the room and when the device's last
+// handle is destroyed.
 struct PathPool {
   struct Buf {
     int dev;
@@ -618,6 +619,7 @@ struct PathPool {
     return std::max(largest, std::min((f + spare) / 4, busy < cap ? cap - busy : 0));
   }
   void* take(int dev, size_t bytes) {
+    if (bytes == 0) return nullptr;
     std::lock_guard<std::mutex> lk(mu);
     Buf* best = nullptr;
     size_t busy = 0;
@@ -3146,12 +3148,10 @@ BigArgs<R> big_run_args(pasif_driver* d, bool adjoint, RunMem& mem, void* out_q,
   return a;
 }
 
-// Arguments of a run of the row-kernel instances, as big_run_args; `lease`
-// (null: none) is where the stored path's memory comes from.
+// Arguments of a run of the row-kernel instances, as big_run_args.
 template <typename R>
 RowArgs<R> row_run_args(pasif_driver* d, bool adjoint, uint32_t save_steps, uint32_t nslots,
-                        RunMem& mem, void* out_q, void* out_grad, PathLease* lease,
-                        uint64_t* work_out) {
+                        RunMem& mem, void* out_q, void* out_grad, uint64_t* work_out) {
   Packed& pk = d->pk;
   RowArgs<R> a{};
   a.inst = pk.r_inst.as<RowInst>();
@@ -3191,24 +3191,28 @@ RowArgs<R> row_run_args(pasif_driver* d, bool adjoint, uint32_t save_steps, uint
   uint64_t work = pk.r_tmax;
   if (adjoint) {
     a.vec_a = static_cast<R*>(mem.get(d->rvec_a, size_t(pk.r_vec_a) * el));
-    // With an interval of the caller's choice its checkpoints are kept and
-    // segments recomputed; with the automatic one the whole path is stored
-    // when it fits (one pass less of forward work; the plan's footprint
-    // stays that of the checkpoints, which always suffice).
-    if (lease && d->ck_every == 0)
-      a.segbuf = static_cast<R*>(lease->take(d->dev, size_t(pk.r_path) * el));
-    a.store = a.segbuf ? 1u : 0u;
-    if (!a.store) {
-      a.ckpt = static_cast<R*>(mem.get(d->rckpt, size_t(pk.r_ck) * el, true));
-      a.segbuf = static_cast<R*>(mem.get(d->rseg, size_t(pk.r_seg) * el));
-    }
+    a.ckpt = static_cast<R*>(mem.get(d->rckpt, size_t(pk.r_ck) * el, true));
+    a.segbuf = static_cast<R*>(mem.get(d->rseg, size_t(pk.r_seg) * el));
     a.out_grad = static_cast<R*>(out_grad);
     a.adjoint = 1;
     a.exact = d->adj_mode != 0 ? 1u : 0u;
-    work = (a.store ? 2ull : 3ull) * pk.r_tmax;
+    work = 3ull * pk.r_tmax;
   }
   *work_out = work;
   return a;
+}
+
+// Room for the row kernel's stored path from `lease`, if it gets all of it:
+// one pass less of forward work than recomputed segments.  With an interval
+// of the caller's choice its checkpoints are kept and segments recomputed.
+template <typename R>
+void row_path(pasif_driver* d, PathLease& lease, RowArgs<R>& a, uint64_t* work) {
+  if (!a.adjoint || d->ck_every != 0) return;
+  void* p = lease.take(d->dev, size_t(d->pk.r_path) * sizeof(R));
+  if (!p) return;
+  a.segbuf = static_cast<R*>(p);
+  a.store = 1;
+  *work = 2ull * d->pk.r_tmax;
 }
 
 template <typename R>
@@ -3398,56 +3402,6 @@ uint32_t run_outputs(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   return nslots;
 }
 
-// Room for the lane parts' stored paths, from `lease`: elements of the
-// working type for each class of each part (0: recompute).  A stored path
-// saves the recompute pass (and its phase switches) and costs a write and a
-// read of the segment rows of every step.  The write runs beside the forward
-// pass, so it pays as long as the memory keeps up: the room is at most what
-// one and a half times the forward pass takes at kPathRate (the counted
-// instructions at 4 cycles each and 2.4 GHz, the longest wave or the whole
-// chip's work, whichever is longer; the pass itself runs at about 1.3 of
-// that), and what the lease grants.  Each class gets its share, its longest
-// waves first.  8,192 chains of 16 DOF x 10,000 steps (21 GB, the chip full):
-// 15.1 ms recomputed, 12.4 ms stored; 4,096 uneven systems 9.5 and 7.0 ms;
-// a batch of one- and two-DOF systems that fills the chip moves 10 TB/s at
-// its forward rate and keeps most of its waves on checkpoints.
-constexpr double kPathRate = 4.5e12;
-template <typename R>
-std::vector<std::vector<uint64_t>> path_plan(pasif_driver* d, PathLease& lease,
-                                             std::vector<void*>* base) {
-  Packed& pk = d->pk;
-  std::vector<std::vector<uint64_t>> room(pk.lparts.size());
-  double elems = 0, work = 0, chain = 0;
-  for (size_t i = 0; i < pk.lparts.size(); ++i) {
-    room[i].assign(pk.lparts[i]->cls.size(), 0);
-    for (const auto& L : pk.lparts[i]->cls) {
-      if (!L->pathoff) continue;
-      elems += double(L->path_elems);
-      for (uint32_t t : L->wave_t) work += double(t) * L->fwd_cost;
-      chain = std::max(chain, double(L->tmax) * L->fwd_cost);
-    }
-  }
-  base->assign(pk.lparts.size(), nullptr);
-  if (elems == 0 || d->window) return room;
-  const double fwd_s = std::max(work / device_simds(d->dev), chain) * 4.0 / 2.4e9;
-  const double want = std::min(elems * sizeof(R), 1.5 * fwd_s * kPathRate);
-  const size_t bytes = size_t(std::min(want, double(path_pool().limit(d->dev))));
-  void* p = bytes > (size_t(1) << 16) ? lease.take(d->dev, bytes) : nullptr;
-  if (!p) return room;
-  const double share = double(bytes) / (elems * sizeof(R));
-  unsigned char* at = static_cast<unsigned char*>(p);
-  for (size_t i = 0; i < pk.lparts.size(); ++i) {
-    (*base)[i] = at;
-    for (size_t c = 0; c < room[i].size(); ++c) {
-      const LaneCls& L = *pk.lparts[i]->cls[c];
-      if (!L.pathoff) continue;
-      room[i][c] = uint64_t(double(L.path_elems) * std::min(share, 1.0)) / 64 * 64;
-      at += room[i][c] * sizeof(R);
-    }
-  }
-  return room;
-}
-
 // Run buffers of one lane part and its per-class kernel arguments (budget
 // filled in by the caller).  K is the part's checkpoint interval.  Buffers
 // come from `mem` (null: the driver's own), outputs are the driver's unless
@@ -3456,9 +3410,7 @@ template <typename R>
 std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
                                      uint32_t save_steps, uint32_t nslots, const void* excit,
                                      const void* interp, RunMem* mem_in = nullptr,
-                                     void* out_q = nullptr, void* out_grad = nullptr,
-                                     void* path = nullptr,
-                                     const std::vector<uint64_t>* path_room = nullptr) {
+                                     void* out_q = nullptr, void* out_grad = nullptr) {
   Packed& pk = d->pk;
   RunMem own;
   own.d = d;
@@ -3497,12 +3449,6 @@ std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
     a.out_a = L.out_a;
     a.na_out = L.na_out;
     a.ck_off = L.ckoff;
-    if (path && path_room && (*path_room)[c]) {
-      a.path = path;
-      a.path_off = L.pathoff;
-      a.path_cap = (*path_room)[c];
-      path = static_cast<unsigned char*>(path) + (*path_room)[c] * sizeof(R);
-    }
     a.out_q = out_q;
     a.out_max = d->window ? d->out_max.p : nullptr;
     a.traj = save_steps ? d->traj.p : nullptr;
@@ -3529,6 +3475,50 @@ std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
     a.h6 = double(R(double(h) / 6.0));
   }
   return args;
+}
+
+// Room for the lane parts' stored paths, from `lease`, handed to the classes'
+// arguments (none: recompute).  A stored path saves the recompute pass (and
+// its phase switches) and costs a write and a read of the segment rows of
+// every step.  The write runs beside the forward pass, so it pays as long as
+// the memory keeps up: the room is at most what one and a half times the
+// forward pass takes at kPathRate (the counted instructions at 4 cycles each
+// and 2.4 GHz, the longest wave or the whole chip's work, whichever is longer;
+// the pass itself runs at about 1.3 of that), and what the lease grants.  Each
+// class gets its share, its longest waves first.  8,192 chains of 16 DOF x 10,000 steps (21 GB, the chip full):
+// 15.1 ms recomputed, 12.4 ms stored; 4,096 uneven systems 9.5 and 7.0 ms;
+// a batch of one- and two-DOF systems that fills the chip moves 10 TB/s at
+// its forward rate and keeps most of its waves on checkpoints.
+constexpr double kPathRate = 4.5e12;
+template <typename R>
+void lane_paths(pasif_driver* d, PathLease& lease, std::vector<std::vector<LaneArgs>>& args) {
+  Packed& pk = d->pk;
+  double elems = 0, work = 0, chain = 0;
+  for (const auto& lp : pk.lparts)
+    for (const auto& L : lp->cls) {
+      if (!L->pathoff) continue;
+      elems += double(L->path_elems);
+      for (uint32_t t : L->wave_t) work += double(t) * L->fwd_cost;
+      chain = std::max(chain, double(L->tmax) * L->fwd_cost);
+    }
+  if (elems == 0 || d->window) return;
+  const double fwd_s = std::max(work / device_simds(d->dev), chain) * 4.0 / 2.4e9;
+  const double want = std::min(elems * sizeof(R), 1.5 * fwd_s * kPathRate);
+  const size_t bytes = size_t(std::min(want, double(path_pool().limit(d->dev))));
+  void* p = bytes > (size_t(1) << 16) ? lease.take(d->dev, bytes) : nullptr;
+  if (!p) return;
+  const double share = double(bytes) / (elems * sizeof(R));
+  unsigned char* at = static_cast<unsigned char*>(p);
+  for (size_t i = 0; i < pk.lparts.size(); ++i)
+    for (size_t c = 0; c < args[i].size(); ++c) {
+      const LaneCls& L = *pk.lparts[i]->cls[c];
+      if (!L.pathoff) continue;
+      LaneArgs& a = args[i][c];
+      a.path = at;
+      a.path_off = L.pathoff;
+      a.path_cap = uint64_t(double(L.path_elems) * std::min(share, 1.0)) / 64 * 64;
+      at += a.path_cap * sizeof(R);
+    }
 }
 
 hipError_t lane_launch(const LanePart& P, const void* dargs, uint32_t n, hipStream_t st) {
@@ -3570,8 +3560,8 @@ void run_footprint(pasif_driver* d, bool adjoint, uint32_t save_steps, size_t* t
     (void)tile_run_args<R>(d, adjoint, save_steps, m, nullptr, nullptr, nullptr, nullptr, &work,
                            &nslots);
   if (pk.nbig) (void)big_run_args<R>(d, adjoint, m, nullptr, nullptr, &work);
-  if (pk.rows) (void)row_run_args<R>(d, adjoint, save_steps, nslots, m, nullptr, nullptr, nullptr,
-                                      &work);
+  if (pk.rows)
+    (void)row_run_args<R>(d, adjoint, save_steps, nslots, m, nullptr, nullptr, &work);
   for (auto& lp : pk.lparts) {
     auto args = lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, nullptr, nullptr, &m,
                                   nullptr, nullptr);
@@ -3646,19 +3636,20 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
     void* og = adjoint ? d->out_grad.p : nullptr;
     if (pk.nbig) ba = big_run_args<R>(d, adjoint, mem, d->out_q.p, og, &bwork);
     if (pk.rows)
-      ra = row_run_args<R>(d, adjoint, save_steps, nslots, mem, d->out_q.p, og, &lease, &rwork);
-    bwork = std::max(bwork, rwork);
+      ra = row_run_args<R>(d, adjoint, save_steps, nslots, mem, d->out_q.p, og, &rwork);
   }
   std::vector<std::vector<LaneArgs>> largs;
   if (lane) {
     nslots = run_outputs<R>(d, adjoint, save_steps);
-    std::vector<void*> pbase;
-    const auto room = path_plan<R>(d, lease, &pbase);
-    for (size_t i = 0; i < pk.lparts.size(); ++i)
-      largs.push_back(lane_part_args<R>(d, *pk.lparts[i], adjoint, save_steps, nslots, d->d_exc.p,
-                                        d->d_interp.p, nullptr, nullptr, nullptr, pbase[i],
-                                        &room[i]));
+    for (auto& lp : pk.lparts)
+      largs.push_back(lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, d->d_exc.p,
+                                        d->d_interp.p));
   }
+  // Paths come last: every buffer the solve cannot do without is there by now,
+  // and what a path takes of the memory left cannot refuse the solve.
+  if (pk.rows) row_path<R>(d, lease, ra, &rwork);
+  if (lane) lane_paths<R>(d, lease, largs);
+  bwork = std::max(bwork, rwork);
   const uint64_t lwork = lane ? (adjoint ? 3ull * pk.ltmax : pk.ltmax) : 0;
   uint64_t launches = 1;
   const uint32_t budget = launch_budget(d, std::max(std::max(twork, lwork), bwork), &launches);
@@ -3758,7 +3749,7 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
     if (tile)
       ta = tile_run_args<R>(d, adjoint, 0, mem, out_q, nullptr, nullptr, out_grad, &twork,
                             &nslots);
-    if (pk.rows) ra = row_run_args<R>(d, adjoint, 0, 0, mem, out_q, out_grad, nullptr, &rwork);
+    if (pk.rows) ra = row_run_args<R>(d, adjoint, 0, 0, mem, out_q, out_grad, &rwork);
     if (lane)
       for (auto& lp : pk.lparts) {
         largs.push_back(lane_part_args<R>(d, *lp, adjoint, 0, 0, d->d_exc.p, d->d_interp.p,

@@ -1,0 +1,51 @@
+"""The stored path of an adjoint solve is extra: it takes what the solve's own
+buffers leave, so a solve whose buffers fit runs however little is left
+beside them -- with a path for some waves or for none."""
+import numpy as np
+import pytest
+import torch
+
+from pasif_amd import adjoint as ADJ
+from pasif_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _leave(nbytes):
+    """Tensors that leave about ``nbytes`` of the device's memory free (a large
+    one takes a little less off the free memory than its size)."""
+    held = []
+    while (over := torch.cuda.mem_get_info()[0] - int(nbytes)) > 4 << 20:
+        held.append(torch.empty(over, dtype=torch.uint8, device="cuda"))
+    return held
+
+
+def _problem(steps):
+    w = W.chains(n_systems=4096, d=16, steps=steps, steps_per_sample=10)
+    w.excitations = np.asarray(w.excitations)[:3]
+    w.exc_of_system = np.arange(4096) % 3
+    return w, W.make_solver(w), ADJ.energy_gradient_inputs(w)
+
+
+def test_path_takes_what_the_run_buffers_leave():
+    steps = 100_000
+    print(f"[gpu case] path memory: 4096 16-DOF chains x {steps} steps, little memory free",
+          flush=True)
+    w, p, J = _problem(steps)
+    p.setJacobian(*J.as_args())
+    p.setTuning(checkpoint_every=256)     # checkpoints, no path
+    ref = p.getGradient()
+    del p
+    p = W.make_solver(w)
+    p.setJacobian(*J.as_args())
+    fp = p._runFootprint(True)            # packed and uploaded, nothing run
+    # the solve's own buffers take 79 % of what is left free (it may take 80)
+    hold = _leave(fp["run"] / 0.79)
+    try:
+        g = p.getGradient()
+        again = p.getGradient()
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+    np.testing.assert_array_equal(g, ref)
+    np.testing.assert_array_equal(again, ref)
