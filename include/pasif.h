@@ -220,6 +220,14 @@ int pasif_set_adjoint_mode(pasif_driver* d, int mode);
  * reference's planner keeps to 0.8 x free (src/__GpuDriver.cu:896-938). */
 int pasif_run_footprint(pasif_driver* d, int adjoint, size_t* run_bytes, size_t* ckpt_bytes,
                         size_t* free_bytes);
+/* Gives the idle memory the library keeps on a GPU between solves back to the
+ * driver (extension); *released (may be NULL) is its size.  Adjoint solves with
+ * the automatic checkpoint interval store their forward path in a buffer of at
+ * most 32 GiB in all and a quarter of the memory their other buffers leave,
+ * which stays for the next solve of any handle on that GPU.  It makes way for
+ * the library's own allocations, and goes with the GPU's last handle; a program
+ * that wants the memory for something else meanwhile calls this. */
+int pasif_trim_memory(int gpu_id, size_t* released);
 /* Diagnostics: the generated HIP source of the lane kernel for the loaded
  * problem (NUL-terminated; out == NULL: length query), and with compile != 0
  * its hipRTC compilation for gfx950, which needs no GPU. */

@@ -49,6 +49,7 @@ class __GpuDriver:  # noqa: N801  (the reference's class name)
     def __init__(self, excitationSet_, sampleRate_, numsteps_, dCompute_=False, dSystem_=False,
                  dSolver_=False, GPUId_=0):
         self._pl = _lib.load()
+        self._gpu = int(GPUId_)
         exc = self._flatten_excitations(excitationSet_)
         if exc is None:
             raise ValueError("Excitations vectors are not of the same size")
@@ -294,6 +295,14 @@ class __GpuDriver:  # noqa: N801  (the reference's class name)
         if mode not in modes:
             raise ValueError(f"adjoint mode {mode!r}: 'reference' or 'exact'")
         self._chk(self._pl.pasif_set_adjoint_mode(self._h, modes[mode]))
+
+    def _trimMemory(self) -> int:
+        """Bytes of idle path memory given back to the driver (this handle's
+        GPU)."""
+        n = C.c_size_t(0)
+        if getattr(self, "_gpu", -1) >= 0:
+            _lib.check(self._pl, self._h, self._pl.pasif_trim_memory(self._gpu, C.byref(n)))
+        return n.value
 
     def _runFootprint(self, adjoint: bool = False) -> dict:
         """Device bytes of a solve's run buffers and outputs (``run``), the

@@ -78,6 +78,7 @@ _SIGS = {
     "pasif_set_adjoint_mode": (C.c_int, [_h, C.c_int]),
     "pasif_run_footprint": (C.c_int, [_h, C.c_int, C.POINTER(C.c_size_t),
                                       C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]),
+    "pasif_trim_memory": (C.c_int, [C.c_int, C.POINTER(C.c_size_t)]),
     "pasif_solve_noalloc": (C.c_int, [_h, C.c_int, C.c_void_p, C.c_void_p]),
     "pasif_version": (C.c_char_p, []),
 }

@@ -43,6 +43,124 @@ struct Fail {
 };
 
 // ------------------------------------------------------------------ device
+// Device memory for the forward paths that adjoint solves store instead of
+// recomputing: leased for the length of one (synchronous) solve and kept for
+// the next solve of any handle on the device, since paths are large and the
+// driver clears freed device memory before it hands it out again (freeing
+// and allocating 32 GB in turn took 0.9 s a time).  Bounded: a lease is
+// granted only while all of it together stays within 32 GiB and the new
+// buffer within a quarter of the memory free once the solve holds its run
+// buffers; without one a solve recomputes from checkpoints.  Given back when
+// an allocation of the library's needs the room and when the device's last
+// handle is destroyed.
+struct PathPool {
+  struct Buf {
+    int dev;
+    void* p;
+    size_t bytes;
+    bool busy;
+  };
+  std::mutex mu;
+  std::vector<Buf> bufs;
+  std::map<int, uint32_t> handles;
+
+  size_t trim_locked(int dev) {
+    size_t b = 0;
+    for (size_t i = bufs.size(); i-- > 0;)
+      if (bufs[i].dev == dev && !bufs[i].busy) {
+        b += bufs[i].bytes;
+        (void)hipFree(bufs[i].p);
+        bufs.erase(bufs.begin() + long(i));
+      }
+    return b;
+  }
+  size_t trim(int dev) {  // bytes given back
+    std::lock_guard<std::mutex> lk(mu);
+    return trim_locked(dev);
+  }
+  size_t idle(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    size_t b = 0;
+    for (const Buf& x : bufs)
+      if (x.dev == dev && !x.busy) b += x.bytes;
+    return b;
+  }
+  // bytes a lease could get now
+  size_t limit(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    size_t busy = 0, spare = 0, largest = 0, f = 0, t = 0;
+    for (const Buf& x : bufs) {
+      if (x.dev != dev) continue;
+      if (x.busy) {
+        busy += x.bytes;
+      } else {
+        spare += x.bytes;
+        largest = std::max(largest, x.bytes);
+      }
+    }
+    if (hipMemGetInfo(&f, &t) != hipSuccess) return largest;
+    const size_t cap = size_t(32) << 30;
+    return std::max(largest, std::min((f + spare) / 4, busy < cap ? cap - busy : 0));
+  }
+  void* take(int dev, size_t bytes) {
+    if (bytes == 0) return nullptr;
+    std::lock_guard<std::mutex> lk(mu);
+    Buf* best = nullptr;
+    size_t busy = 0;
+    for (Buf& x : bufs) {
+      if (x.dev != dev) continue;
+      if (x.busy)
+        busy += x.bytes;
+      else if (x.bytes >= bytes && (!best || x.bytes < best->bytes))
+        best = &x;
+    }
+    if (best) {
+      best->busy = true;
+      return best->p;
+    }
+    if (bytes + busy > (size_t(32) << 30)) return nullptr;
+    trim_locked(dev);
+    size_t f = 0, t = 0;
+    if (hipMemGetInfo(&f, &t) != hipSuccess || bytes > f / 4) return nullptr;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    bufs.push_back({dev, p, bytes, true});
+    return p;
+  }
+  void give(void* p) {
+    std::lock_guard<std::mutex> lk(mu);
+    for (Buf& x : bufs)
+      if (x.p == p) x.busy = false;
+  }
+  void attach(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    ++handles[dev];
+  }
+  void detach(int dev) {
+    std::lock_guard<std::mutex> lk(mu);
+    if (--handles[dev] == 0) trim_locked(dev);
+  }
+};
+PathPool& path_pool() {
+  static PathPool* p = new PathPool;  // outlives every handle
+  return *p;
+}
+
+// Every device allocation of the library that may be large: when there is no
+// room, the current device's idle path memory makes way.
+hipError_t dev_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  int dev = 0;
+  if (e != hipSuccess && hipGetDevice(&dev) == hipSuccess && path_pool().trim(dev)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 // Sub-allocator of a pool's device memory: chunks taken with hipMalloc once
 // and carved into 256-byte aligned blocks (first fit over an offset-ordered,
 // coalescing free list).  Admitting or retiring a job then neither allocates
@@ -90,7 +208,7 @@ struct Arena {
     Chunk c{};
     c.cap = std::max(chunk_bytes, need);
     void* base = nullptr;
-    if (hipMalloc(&base, c.cap) != hipSuccess) return nullptr;
+    if (dev_malloc(&base, c.cap) != hipSuccess) return nullptr;
     c.base = static_cast<char*>(base);
     reserved += c.cap;
     if (c.cap > need) c.add(need, c.cap - need);
@@ -560,111 +678,6 @@ int guarded(pasif_driver* d, F&& f) {
 }
 
 // ------------------------------------------------------- stored-path memory
-// Device memory for the forward paths that adjoint solves store instead of
-// recomputing: leased for the length of one (synchronous) solve and kept for
-// the next solve of any handle on the device, since paths are large and the
-// driver clears freed device memory before it hands it out again (freeing
-// and allocating 32 GB in turn took 0.9 s a time).  Bounded: a lease is
-// granted only while all of it together stays within 32 GiB and the new
-// buffer within a quarter of the memory free once the solve holds its run
-// buffers; without one a solve recomputes from checkpoints.  Given back when
-// an allocation of the library's needs the room and when the device's last
-// handle is destroyed.
-struct PathPool {
-  struct Buf {
-    int dev;
-    void* p;
-    size_t bytes;
-    bool busy;
-  };
-  std::mutex mu;
-  std::vector<Buf> bufs;
-  std::map<int, uint32_t> handles;
-
-  void trim_locked(int dev) {
-    for (size_t i = bufs.size(); i-- > 0;)
-      if (bufs[i].dev == dev && !bufs[i].busy) {
-        (void)hipFree(bufs[i].p);
-        bufs.erase(bufs.begin() + long(i));
-      }
-  }
-  bool trim(int dev) {
-    std::lock_guard<std::mutex> lk(mu);
-    const size_t n = bufs.size();
-    trim_locked(dev);
-    return bufs.size() != n;
-  }
-  size_t idle(int dev) {
-    std::lock_guard<std::mutex> lk(mu);
-    size_t b = 0;
-    for (const Buf& x : bufs)
-      if (x.dev == dev && !x.busy) b += x.bytes;
-    return b;
-  }
-  // bytes a lease could get now
-  size_t limit(int dev) {
-    std::lock_guard<std::mutex> lk(mu);
-    size_t busy = 0, spare = 0, largest = 0, f = 0, t = 0;
-    for (const Buf& x : bufs) {
-      if (x.dev != dev) continue;
-      if (x.busy) {
-        busy += x.bytes;
-      } else {
-        spare += x.bytes;
-        largest = std::max(largest, x.bytes);
-      }
-    }
-    if (hipMemGetInfo(&f, &t) != hipSuccess) return largest;
-    const size_t cap = size_t(32) << 30;
-    return std::max(largest, std::min((f + spare) / 4, busy < cap ? cap - busy : 0));
-  }
-  void* take(int dev, size_t bytes) {
-    if (bytes == 0) return nullptr;
-    std::lock_guard<std::mutex> lk(mu);
-    Buf* best = nullptr;
-    size_t busy = 0;
-    for (Buf& x : bufs) {
-      if (x.dev != dev) continue;
-      if (x.busy)
-        busy += x.bytes;
-      else if (x.bytes >= bytes && (!best || x.bytes < best->bytes))
-        best = &x;
-    }
-    if (best) {
-      best->busy = true;
-      return best->p;
-    }
-    if (bytes + busy > (size_t(32) << 30)) return nullptr;
-    trim_locked(dev);
-    size_t f = 0, t = 0;
-    if (hipMemGetInfo(&f, &t) != hipSuccess || bytes > f / 4) return nullptr;
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    bufs.push_back({dev, p, bytes, true});
-    return p;
-  }
-  void give(void* p) {
-    std::lock_guard<std::mutex> lk(mu);
-    for (Buf& x : bufs)
-      if (x.p == p) x.busy = false;
-  }
-  void attach(int dev) {
-    std::lock_guard<std::mutex> lk(mu);
-    ++handles[dev];
-  }
-  void detach(int dev) {
-    std::lock_guard<std::mutex> lk(mu);
-    if (--handles[dev] == 0) trim_locked(dev);
-  }
-};
-PathPool& path_pool() {
-  static PathPool* p = new PathPool;  // outlives every handle
-  return *p;
-}
-
 // The leases of one solve, returned when it is over (after a failed launch:
 // once the device is idle).
 struct PathLease {
@@ -706,11 +719,7 @@ void dev_alloc(pasif_driver* d, DevBuf& b, size_t bytes) {
     b.bytes = bytes;
     return;
   }
-  hipError_t e = hipMalloc(&b.p, bytes);
-  if (e != hipSuccess && path_pool().trim(d->dev)) {
-    (void)hipGetLastError();
-    e = hipMalloc(&b.p, bytes);
-  }
+  const hipError_t e = dev_malloc(&b.p, bytes);
   if (e != hipSuccess) {
     b.p = nullptr;
     set_err(d, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorName(e));
@@ -3599,7 +3608,7 @@ void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   run_footprint<R>(d, adjoint, save_steps, &need, &ck);
   PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
   double avail = 0.8 * double(freeb + held_run_bytes(d));
-  if (double(need) > avail && path_pool().trim(d->dev)) {
+  if (double(need) > avail && path_pool().trim(d->dev) != 0) {
     PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
     avail = 0.8 * double(freeb + held_run_bytes(d));
   }
@@ -4163,6 +4172,16 @@ int pasif_set_adjoint_mode(pasif_driver* d, int mode) {
                   "adjoint mode %d (0 reference recursion, 1 exact discrete adjoint)", mode);
     d->adj_mode = mode;
   });
+}
+
+int pasif_trim_memory(int gpu_id, size_t* released) {
+  if (released) *released = 0;
+  int ndev = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess || gpu_id < 0 || gpu_id >= ndev)
+    return PASIF_ERR_ARGUMENT;
+  const size_t bytes = path_pool().trim(gpu_id);
+  if (released) *released = bytes;
+  return PASIF_OK;
 }
 
 int pasif_run_footprint(pasif_driver* d, int adjoint, size_t* run_bytes, size_t* ckpt_bytes,
@@ -5027,14 +5046,14 @@ void pool_tick_impl(pasif_pool* P) {
     if (P->table_bytes < tb) {
       if (P->table_dev) (void)hipFree(P->table_dev);
       P->table_dev = nullptr;
-      POOL_HIP(hipMalloc(&P->table_dev, tb));
+      POOL_HIP(dev_malloc(&P->table_dev, tb));
       P->table_bytes = tb;
     }
     const size_t mb = P->map_host.size() * sizeof(uint32_t);
     if (P->map_bytes < mb) {
       if (P->map_dev) (void)hipFree(P->map_dev);
       P->map_dev = nullptr;
-      POOL_HIP(hipMalloc(&P->map_dev, mb));
+      POOL_HIP(dev_malloc(&P->map_dev, mb));
       P->map_bytes = mb;
     }
     POOL_HIP(hipMemcpyAsync(P->table_dev, P->table_host.data(), tb, hipMemcpyHostToDevice,
@@ -5048,7 +5067,7 @@ void pool_tick_impl(pasif_pool* P) {
     if (M.table_bytes < b) {
       if (M.table_dev) (void)hipFree(M.table_dev);
       M.table_dev = nullptr;
-      POOL_HIP(hipMalloc(&M.table_dev, b));
+      POOL_HIP(dev_malloc(&M.table_dev, b));
       M.table_bytes = b;
     }
     POOL_HIP(hipMemcpyAsync(M.table_dev, M.table.data(), b, hipMemcpyHostToDevice, P->stream));
@@ -5209,7 +5228,7 @@ int pasif_pool_set_bank(pasif_pool* P, const double* excitations, uint32_t n_exc
     const size_t el = P->precision == 64 ? 8 : 4;
     P->bank.release();
     P->bank_interp.release();
-    POOL_HIP(hipMalloc(&P->bank.p, n * el));
+    POOL_HIP(dev_malloc(&P->bank.p, n * el));
     P->bank.bytes = n * el;
     if (P->precision == 64) {
       POOL_HIP(hipMemcpy(P->bank.p, excitations, n * el, hipMemcpyHostToDevice));
@@ -5218,7 +5237,7 @@ int pasif_pool_set_bank(pasif_pool* P, const double* excitations, uint32_t n_exc
       POOL_HIP(hipMemcpy(P->bank.p, f.data(), n * el, hipMemcpyHostToDevice));
     }
     if (interp) {
-      POOL_HIP(hipMalloc(&P->bank_interp.p, 2 * size_t(window) * el));
+      POOL_HIP(dev_malloc(&P->bank_interp.p, 2 * size_t(window) * el));
       P->bank_interp.bytes = 2 * size_t(window) * el;
       if (P->precision == 64) {
         POOL_HIP(hipMemcpy(P->bank_interp.p, interp, 2 * size_t(window) * el,

@@ -49,3 +49,29 @@ def test_path_takes_what_the_run_buffers_leave():
         torch.cuda.empty_cache()
     np.testing.assert_array_equal(g, ref)
     np.testing.assert_array_equal(again, ref)
+
+
+def test_idle_path_memory_makes_way():
+    print("[gpu case] path memory: a pool's bank and a trajectory beside idle path memory",
+          flush=True)
+    from pasif_amd import serving
+    w, p, J = _problem(2_000)
+    p.setJacobian(*J.as_args())
+    g = p.getGradient()
+    free = torch.cuda.mem_get_info()[0]
+    kept = p._trimMemory()
+    assert kept > 1 << 30
+    assert torch.cuda.mem_get_info()[0] > free
+    assert p._trimMemory() == 0
+    np.testing.assert_array_equal(p.getGradient(), g)   # takes it anew
+    hold = _leave(256 << 20)
+    try:
+        pool = serving.Pool()
+        pool.set_bank(np.zeros((64, 1 << 20)), 1000, None)    # 512 MiB of 256 free
+        pool.close()
+        assert p._trimMemory() == 0
+        # a path from what is left now
+        np.testing.assert_array_equal(p.getGradient(), g)
+    finally:
+        del hold
+        torch.cuda.empty_cache()
