@@ -3294,8 +3294,12 @@ void finish_run(pasif_driver* d, uint32_t nslots, const HostOut& o) {
     if (!o.rows) {
       fetch<R>(d, o.traj, d->traj.p, all);
     } else if (all) {
-      const size_t step = std::max<size_t>(1, std::min(rows, kTrajBytes / (size_t(nslots) * 8)));
-      dev_reserve(d, d->traj_rows, step * nslots * sizeof(double));
+      const size_t row = size_t(nslots) * sizeof(double);
+      size_t room = std::min(kTrajBytes, rows * row), f = 0, t = 0;
+      if (room > d->traj_rows.bytes && hipMemGetInfo(&f, &t) == hipSuccess)
+        room = std::max(d->traj_rows.bytes, std::min(room, f / 2));  // little left: fewer rows
+      const size_t step = std::max<size_t>(1, std::min(rows, room / row));
+      dev_reserve(d, d->traj_rows, step * row);
       for (size_t r = 0; r < rows; r += step) {
         const size_t n = std::min(step, rows - r);
         PASIF_HIP(launch_traj_rows(d->traj.as<R>(), d->traj_rows.as<double>(), nslots,
@@ -3608,7 +3612,9 @@ void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   run_footprint<R>(d, adjoint, save_steps, &need, &ck);
   PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
   double avail = 0.8 * double(freeb + held_run_bytes(d));
-  if (double(need) > avail && path_pool().trim(d->dev) != 0) {
+  if (double(need) > avail) {  // what is kept only for speed makes way
+    d->traj_rows.release();
+    (void)path_pool().trim(d->dev);
     PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
     avail = 0.8 * double(freeb + held_run_bytes(d));
   }

@@ -75,3 +75,20 @@ def test_idle_path_memory_makes_way():
     finally:
         del hold
         torch.cuda.empty_cache()
+
+
+def test_trajectory_rows_with_little_memory_left():
+    print("[gpu case] trajectory rows, 40 MiB beside a trajectory of 130", flush=True)
+    w = W.two_dof(n_systems=4096, steps=2000)
+    p = W.make_solver(w)
+    ref = p.getTrajectory(saveSteps=2)                  # 131 MB, kept by the handle
+    del p
+    p = W.make_solver(w)
+    p.getAmplitudes()
+    hold = _leave(180 << 20)
+    try:
+        tr = p.getTrajectory(saveSteps=2)
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+    np.testing.assert_array_equal(tr, ref)
