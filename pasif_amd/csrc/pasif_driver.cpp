@@ -1876,7 +1876,15 @@ void lane_coefs_mapped(const RowTerms& rt, uint32_t s, const LaneSide& sd, bool 
 // register budget, with the step cost of each.
 std::vector<std::pair<uint32_t, double>> group_options(const LaneShape& sh, int bits) {
   std::vector<std::pair<uint32_t, double>> out;
+  // What every layout of G lanes keeps live at least (lane_live): four values a
+  // slot, G lanes sharing the rows, and a coefficient a term.  Layouts it rules
+  // out are not planned: the planners' cost grows with the square of a long
+  // row's terms (a 2,001-DOF chain's gradient, which no layout holds: 22 s).
+  auto least = [](const LaneSide& sd, uint32_t G) {
+    return 4 * ((sd.n + G - 1) / G) + (sd.coefs() + G - 1) / G;
+  };
   for (uint32_t G = 1; G <= kLaneWave; G *= 2) {
+    if (std::max(least(sh.f, G), sh.adjoint ? least(sh.a, G) : 0u) > lane_max_live(G)) continue;
     LaneShape t = sh;
     if (!lane_group(t, G)) continue;
     if (lane_live(t) > lane_max_live(G)) continue;

@@ -2,6 +2,8 @@
 systems too large for a tile go to it under the automatic kernel choice,
 beside the tile and lane kernels; its checkpoint and run buffers follow the
 instances' own sizes and step counts."""
+import time
+
 import numpy as np
 import pytest
 
@@ -70,3 +72,13 @@ def test_a_long_chain_beside_a_dense_system_fits_one_launch():
             assert i["big"] == 0 and i["rows"] == w.n_systems
             lds.append(i["lds"])
         assert lds[2] == max(lds[:2]) <= 160 * 1024
+
+
+def test_large_systems_are_planned_quickly():
+    # no lane layout holds this gradient, which takes a count and no plans: the
+    # planners need 22 s for it (0.04 s without them)
+    w = W.chains(1, 2001, 20, steps_per_sample=10)
+    p = _host(w)
+    t = time.perf_counter()
+    assert p.kernelInfo(True)["kernel"] == "big"
+    assert time.perf_counter() - t < 3.0
