@@ -3248,17 +3248,27 @@ TileArgs<R> prepare_run(pasif_driver* d, bool adjoint, uint32_t save_steps, uint
                           adjoint ? d->out_grad.p : nullptr, work_out, nslots_out);
 }
 
-// Where a solve's results go: the caller's buffers (null: not wanted), with
-// the values each holds.  `rows`: the trajectory as [replica dof][slot]
+// One result's place in the caller's memory (null: not wanted), the values it
+// holds and, where given, how many the result has -- also when they are too few.
+struct HostBuf {
+  double* p = nullptr;
+  size_t cap = 0;
+  size_t* len = nullptr;
+};
+// Where a solve's results go.  `rows`: the trajectory as [replica dof][slot]
 // instead of [slot][replica dof].
 struct HostOut {
-  double *q = nullptr, *grad = nullptr, *traj = nullptr;
-  size_t capq = 0, capg = 0, capt = 0;
+  HostBuf q, grad, traj;
   bool rows = false;
 };
 
-void check_cap(pasif_driver* d, size_t cap, size_t need) {
+// Whether a result of `need` values goes to `b`.
+bool wanted(pasif_driver* d, const HostBuf& b, size_t need) {
+  if (b.len) *b.len = need;
+  if (!b.p) return false;
+  const size_t cap = b.cap;
   PASIF_REQUIRE(cap >= need, PASIF_ERR_ARGUMENT, "output buffer holds %zu, need %zu", cap, need);
+  return true;
 }
 
 // n device values into a host buffer: doubles straight into it (the copy is
@@ -3287,20 +3297,16 @@ constexpr size_t kTrajBytes = size_t(256) << 20;
 template <typename R>
 void finish_run(pasif_driver* d, uint32_t nslots, const HostOut& o) {
   Packed& pk = d->pk;
-  if (o.q) {
-    check_cap(d, o.capq, pk.out_len_f);
-    fetch<R>(d, o.q, d->out_q.p, pk.out_len_f);
-  }
   d->have_max = d->window != 0;
   if (d->window) {
     d->res_max.resize(pk.out_len_f);
     fetch<R>(d, d->res_max.data(), d->out_max.p, pk.out_len_f);
   }
-  if (o.traj) {
-    const size_t rows = pk.out_len_f, all = rows * nslots;
-    check_cap(d, o.capt, all);
+  if (wanted(d, o.q, pk.out_len_f)) fetch<R>(d, o.q.p, d->out_q.p, pk.out_len_f);
+  const size_t rows = pk.out_len_f, all = rows * nslots;
+  if (wanted(d, o.traj, all)) {
     if (!o.rows) {
-      fetch<R>(d, o.traj, d->traj.p, all);
+      fetch<R>(d, o.traj.p, d->traj.p, all);
     } else if (all) {
       const size_t row = size_t(nslots) * sizeof(double);
       size_t room = std::min(kTrajBytes, rows * row), f = 0, t = 0;
@@ -3312,7 +3318,7 @@ void finish_run(pasif_driver* d, uint32_t nslots, const HostOut& o) {
         const size_t n = std::min(step, rows - r);
         PASIF_HIP(launch_traj_rows(d->traj.as<R>(), d->traj_rows.as<double>(), nslots,
                                    uint32_t(rows), uint32_t(r), uint32_t(n), d->stream));
-        PASIF_HIP(hipMemcpyAsync(o.traj + r * nslots, d->traj_rows.p, n * nslots * sizeof(double),
+        PASIF_HIP(hipMemcpyAsync(o.traj.p + r * nslots, d->traj_rows.p, n * nslots * sizeof(double),
                                  hipMemcpyDeviceToHost, d->stream));
         PASIF_HIP(hipStreamSynchronize(d->stream));
       }
@@ -3320,10 +3326,7 @@ void finish_run(pasif_driver* d, uint32_t nslots, const HostOut& o) {
     if (d->traj.bytes > kTrajBytes) d->traj.release();
     if (d->traj_rows.bytes > kTrajBytes) d->traj_rows.release();
   }
-  if (o.grad) {
-    check_cap(d, o.capg, pk.out_len_a);
-    fetch<R>(d, o.grad, d->out_grad.p, pk.out_len_a);
-  }
+  if (wanted(d, o.grad, pk.out_len_a)) fetch<R>(d, o.grad.p, d->out_grad.p, pk.out_len_a);
 }
 
 // Steps of work per launch for the solver mode, and the launches that cover
@@ -4123,10 +4126,8 @@ int pasif_get_amplitudes(pasif_driver* d, double* out, size_t cap, size_t* len) 
       return;
     }
     HostOut o;
-    o.q = out;
-    o.capq = cap;
+    o.q = {out, cap, len};
     solve(d, false, 0, o);
-    if (len) *len = d->pk.out_len_f;
   });
 }
 
@@ -4140,10 +4141,8 @@ int pasif_get_trajectory(pasif_driver* d, uint32_t save_steps, double* out, size
       return;
     }
     HostOut o;
-    o.traj = out;
-    o.capt = cap;
+    o.traj = {out, cap, len};
     solve(d, false, save_steps, o);
-    if (len) *len = size_t(d->pk.tmax / save_steps) * d->pk.out_len_f;
   });
 }
 
@@ -4154,11 +4153,9 @@ int pasif_get_trajectory_rows(pasif_driver* d, uint32_t save_steps, double* out,
     PASIF_REQUIRE(out != nullptr, PASIF_ERR_ARGUMENT,
                   "null output (pasif_get_trajectory answers the length query)");
     HostOut o;
-    o.traj = out;
-    o.capt = cap;
+    o.traj = {out, cap, len};
     o.rows = true;
     solve(d, false, save_steps, o);
-    if (len) *len = size_t(d->pk.tmax / save_steps) * d->pk.out_len_f;
   });
 }
 
@@ -4173,10 +4170,8 @@ int pasif_get_gradient(pasif_driver* d, uint32_t save, double* out, size_t cap, 
       return;
     }
     HostOut o;
-    o.grad = out;
-    o.capg = cap;
+    o.grad = {out, cap, len};
     solve(d, true, 0, o);
-    if (len) *len = d->pk.out_len_a;
   });
 }
 
@@ -5808,19 +5803,14 @@ int pasif_pool_collect(pasif_pool* P, pasif_driver* d, double* q, size_t capq, s
                        "job lane workgroups did not finish");
       }
     HostOut o;
-    o.q = q;
-    o.capq = capq;
-    if (j.adjoint) {
-      o.grad = grad;
-      o.capg = capg;
-    }
+    o.q = {q, capq, lenq};
+    if (j.adjoint) o.grad = {grad, capg, leng};
     const int rc = guarded(d, [&] {
       if (P->precision == 64)
         finish_run<double>(d, 0, o);
       else
         finish_run<float>(d, 0, o);
-      if (lenq) *lenq = d->pk.out_len_f;
-      if (leng) *leng = j.adjoint ? d->pk.out_len_a : 0;
+      if (leng && !j.adjoint) *leng = 0;
     });
     if (rc != PASIF_OK) {
       P->err = d->err;

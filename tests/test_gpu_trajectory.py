@@ -1,9 +1,12 @@
 """The trajectory by rows (transposed on the device) against the solver's own
 slot order, exactly: tiles of 32 x 32 values whole, one over and one short,
 one slot, one row, both precisions."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from pasif_amd import adjoint as ADJ
 from pasif_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +51,31 @@ def test_window_and_saved_steps_are_the_states_of_every_step(even, window, save)
     if save:
         saved = p._getTrajectory(save).reshape(-1, per * n)
         np.testing.assert_array_equal(saved, every[::save][:saved.shape[0]])
+
+
+def test_a_buffer_too_small_says_what_is_needed():
+    """A solve into a buffer too small is refused with the length it needs, and
+    its amplitude window is there all the same."""
+    print("[gpu case] output buffers too small", flush=True)
+    w = W.chains(3, 2, 40, steps_per_sample=10)
+    p = W.make_solver(w)
+    p.setJacobian(*ADJ.energy_gradient_inputs(w).as_args())
+    q, mx = p.getMaxAmplitudes(window=9)
+    small = np.full(4, 7.0)
+    buf = small.ctypes.data_as(C.POINTER(C.c_double))
+    p._setAmplitudeWindow(5)
+    n = C.c_size_t(0)
+    lib, h = p._pl, p._h
+    assert lib.pasif_get_amplitudes(h, buf, 4, C.byref(n)) == 1 and n.value == q.size
+    five = np.empty(q.size)
+    assert lib.pasif_get_max_amplitudes(h, five.ctypes.data_as(C.POINTER(C.c_double)), q.size,
+                                        None) == 0
+    p._setAmplitudeWindow(0)
+    np.testing.assert_array_equal(five, p.getMaxAmplitudes(window=5)[1])
+    for f in (lib.pasif_get_trajectory, lib.pasif_get_trajectory_rows):
+        n.value = 0
+        assert f(h, 8, buf, 4, C.byref(n)) == 1 and n.value == 5 * q.size
+    n.value = 0
+    g = p.getGradient()
+    assert lib.pasif_get_gradient(h, 0, buf, 4, C.byref(n)) == 1 and n.value == g.size
+    np.testing.assert_array_equal(small, 7.0)
