@@ -216,8 +216,10 @@ int pasif_set_adjoint_mode(pasif_driver* d, int mode);
  * of which checkpoints (*ckpt_bytes), and the device memory a solve may use
  * now (*free_bytes: free memory plus the run buffers the handle already
  * holds; 0 on a host-only handle).  A solve whose run buffers exceed 80 % of
- * that is refused with PASIF_ERR_MEMORY before anything is allocated, as the
- * reference's planner keeps to 0.8 x free (src/__GpuDriver.cu:896-938). */
+ * that runs its lane classes in pieces that do not, or is refused with
+ * PASIF_ERR_MEMORY before anything is allocated where one wave's exceed it or
+ * other kernels' do, as the reference's planner keeps to 0.8 x free
+ * (src/__GpuDriver.cu:896-938). */
 int pasif_run_footprint(pasif_driver* d, int adjoint, size_t* run_bytes, size_t* ckpt_bytes,
                         size_t* free_bytes);
 /* Gives the idle memory the library keeps on a GPU between solves back to the
@@ -358,8 +360,10 @@ int pasif_pool_poll(pasif_pool* pool, int* running);
  *    out_grad: device buffer of lambda_0 (pasif_get_gradient's length,
  *    adjoint only), both of the working precision (double for 64 bits,
  *    float for 32).  Results equal those of the allocating entry points.
+ *  - Lane classes whose run buffers exceed the array run in pieces that do not.
  *  - Returns when the results are in place.  PASIF_ERR_MEMORY if the run
- *    buffers exceed the scratch array, PASIF_ERR_STATE without the set-up,
+ *    buffers of the other kernels, or of one wave, exceed the scratch array,
+ *    PASIF_ERR_STATE without the set-up,
  *    PASIF_ERR_UNSUPPORTED with an amplitude window, the graph solver or a
  *    pool job.
  *  - Every call on one GPU shares that GPU's array: calls that overlap in

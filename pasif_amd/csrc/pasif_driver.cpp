@@ -301,11 +301,9 @@ struct LaneCls {
   uint32_t nf = 0, na = 0;
   uint32_t klass = 0;  // the class's case in its kernel's dispatch
   uint32_t seg = 1;    // checkpoint interval (adjoint)
-  // single-wave adjoint: checkpoint elements, each wave's block sized by its
-  // longest instance (offsets in ckoff)
-  uint64_t ck_elems = 0;
+  uint32_t ipw = 0;    // instances per workgroup
   // stored path of every wave: elements, and what one forward step of a wave
-  // costs against its bytes (path_plan)
+  // costs against its bytes (lane_paths)
   uint64_t path_elems = 0;
   double fwd_cost = 0;
   // the longest instance of each workgroup (instances are sorted by step
@@ -2684,6 +2682,7 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
     L->seg = adjoint ? ((lay.waves == 1 && sh.seg) ? sh.seg : lay.seg) : 1u;
     block += L->waves;
     const uint32_t ipb = grp ? kLaneWave / G : unit;
+    L->ipw = ipb;
     L->wave_t.assign(L->waves, 0u);
     for (uint32_t w = 0; w < L->waves; ++w)
       if (size_t(w) * ipb < mem.size()) L->wave_t[w] = mem[size_t(w) * ipb]->steps;
@@ -2838,7 +2837,6 @@ LanePart* lane_build(pasif_driver* d, bool adjoint, int part,
         off[w] = tot;
         tot += uint64_t(std::max<uint32_t>(1, (Tw + L->seg - 1) / L->seg)) * L->nf * kLaneWave;
       }
-      L->ck_elems = tot;
       if (lay.store) {
         uint64_t* po = reinterpret_cast<uint64_t*>(host.data() + f.pt);
         const uint64_t rows = lane_seg_rows(sh);
@@ -3426,78 +3424,106 @@ uint32_t run_outputs(pasif_driver* d, bool adjoint, uint32_t save_steps) {
   return nslots;
 }
 
-// Run buffers of one lane part and its per-class kernel arguments (budget
-// filled in by the caller).  K is the part's checkpoint interval.  Buffers
-// come from `mem` (null: the driver's own), outputs are the driver's unless
-// given.
+// Run buffers and kernel arguments (budget filled in by the caller) of waves
+// [w0, w0 + nw) of one class of a lane part: all of them, or of a single-wave
+// part some.  Buffers come from `mem`.
+template <typename R>
+LaneArgs lane_cls_args(pasif_driver* d, const LanePart& P, LaneCls& L, bool adjoint,
+                       uint32_t save_steps, uint32_t nslots, const void* excit,
+                       const void* interp, RunMem& mem, void* out_q, void* out_grad, uint32_t w0,
+                       uint32_t nw) {
+  const R h = R(1.0 / double(d->sample_rate));
+  const uint32_t K = adjoint ? L.seg : 1u;
+  const bool all = nw == L.waves;
+  const size_t st = all ? size_t(L.stride) : size_t(nw) * kLaneWave;
+  // input columns and instances before the first wave
+  const size_t c0 = all ? 0 : size_t(w0) * kLaneWave;
+  const uint32_t i0 = w0 * L.ipw;
+  auto cols = [&](const void* p) -> const void* { return p ? static_cast<const R*>(p) + c0 : p; };
+  auto words = [&](const void* p) -> const void* {
+    return p ? static_cast<const uint32_t*>(p) + i0 : p;
+  };
+  LaneArgs a;
+  std::memset(&a, 0, sizeof a);
+  a.qstate = mem.get(L.qstate, size_t(L.nf) * st * sizeof(R));
+  a.progress = mem.get(L.progress, size_t(nw) * 4 * sizeof(uint32_t));
+  mem.zero(a.progress, size_t(nw) * 4 * sizeof(uint32_t));
+  if (d->window) a.mxstate = mem.get(L.mxstate, size_t(L.nf) * st * sizeof(R));
+  uint32_t nck = 1;
+  if (adjoint) {
+    nck = std::max<uint32_t>(1, (L.tmax + K - 1) / K);
+    a.lstate = mem.get(L.lstate, size_t(std::max<uint32_t>(L.na, 1)) * st * sizeof(R));
+    if (P.lay.waves == 1) {
+      // blocks of the waves (offsets in ckoff), sized by their longest instances
+      auto block = [&](uint32_t w) {
+        return uint64_t(std::max<uint32_t>(1, (L.wave_t[w] + K - 1) / K)) * L.nf * kLaneWave;
+      };
+      // the buffer's address less the blocks before it
+      uint64_t off = 0, elems = 0;
+      for (uint32_t w = 0; w < w0; ++w) off += block(w);
+      for (uint32_t w = w0; w < w0 + nw; ++w) elems += block(w);
+      a.ckpt = mem.get(L.ckpt, size_t(elems) * sizeof(R), true);
+      if (a.ckpt)
+        a.ckpt = reinterpret_cast<void*>(reinterpret_cast<uintptr_t>(a.ckpt) - off * sizeof(R));
+      a.ck_off = static_cast<const uint64_t*>(L.ckoff) + w0;
+    } else {
+      a.ckpt = mem.get(L.ckpt, size_t(nck) * L.nf * st * sizeof(R), true);
+    }
+    a.segbuf = mem.get(L.segbuf, lane_seg_values(K, P.lay.exact) * L.nf * st * sizeof(R));
+  }
+  a.coef_f = cols(L.coef_f);
+  a.coef_a = cols(L.coef_a);
+  a.init_f = cols(L.init_f);
+  a.init_a = cols(L.init_a);
+  a.steps = words(L.steps);
+  a.exc = words(L.exc);
+  a.out_f = words(L.out_f);
+  a.out_a = words(L.out_a);
+  a.na_out = words(L.na_out);
+  a.out_q = out_q;
+  a.out_max = d->window ? d->out_max.p : nullptr;
+  a.traj = save_steps ? d->traj.p : nullptr;
+  a.out_grad = adjoint ? out_grad : nullptr;
+  a.excit = excit;
+  a.interp = d->interp_w ? interp : nullptr;
+  a.stride = L.stride;
+  a.sstride = st;
+  a.count = std::min(L.count - i0, nw * L.ipw);
+  a.block_begin = all ? L.block_begin : 0;
+  a.klass = L.klass;
+  a.exc_len = d->exc_len;
+  a.interp_w = d->interp_w;
+  a.window = d->window;
+  a.out_len = d->pk.out_len_f;
+  a.save_every = save_steps;
+  a.nslots = nslots;
+  a.ck_every = K;
+  a.nck = nck;
+  a.adjoint = adjoint ? 1 : 0;
+  // h = 1/sampleRate in the working type, h2 and h6 from that h in double
+  // (src/__GpuDriver.cu:632-636), carried exactly in a double
+  a.h = double(h);
+  a.h2 = double(R(double(h) / 2.0));
+  a.h6 = double(R(double(h) / 6.0));
+  return a;
+}
+
+// The same of every class of a lane part.  Buffers come from `mem` (null: the
+// driver's own), outputs are the driver's unless given.
 template <typename R>
 std::vector<LaneArgs> lane_part_args(pasif_driver* d, LanePart& P, bool adjoint,
                                      uint32_t save_steps, uint32_t nslots, const void* excit,
                                      const void* interp, RunMem* mem_in = nullptr,
                                      void* out_q = nullptr, void* out_grad = nullptr) {
-  Packed& pk = d->pk;
   RunMem own;
   own.d = d;
   RunMem& mem = mem_in ? *mem_in : own;
   if (!out_q) out_q = d->out_q.p;
   if (!out_grad && adjoint) out_grad = d->out_grad.p;
-  const R h = R(1.0 / double(d->sample_rate));
-  std::vector<LaneArgs> args(P.cls.size());
-  for (size_t c = 0; c < P.cls.size(); ++c) {
-    LaneCls& L = *P.cls[c];
-    const uint32_t K = adjoint ? L.seg : 1u;
-    const size_t st = L.stride;
-    LaneArgs& a = args[c];
-    std::memset(&a, 0, sizeof a);
-    a.qstate = mem.get(L.qstate, size_t(L.nf) * st * sizeof(R));
-    a.progress = mem.get(L.progress, size_t(L.waves) * 4 * sizeof(uint32_t));
-    mem.zero(a.progress, size_t(L.waves) * 4 * sizeof(uint32_t));
-    if (d->window) a.mxstate = mem.get(L.mxstate, size_t(L.nf) * st * sizeof(R));
-    uint32_t nck = 1;
-    if (adjoint) {
-      nck = std::max<uint32_t>(1, (L.tmax + K - 1) / K);
-      a.lstate = mem.get(L.lstate, size_t(std::max<uint32_t>(L.na, 1)) * st * sizeof(R));
-      if (P.lay.waves == 1)
-        a.ckpt = mem.get(L.ckpt, size_t(L.ck_elems) * sizeof(R), true);
-      else
-        a.ckpt = mem.get(L.ckpt, size_t(nck) * L.nf * st * sizeof(R), true);
-      a.segbuf = mem.get(L.segbuf, lane_seg_values(K, P.lay.exact) * L.nf * st * sizeof(R));
-    }
-    a.coef_f = L.coef_f;
-    a.coef_a = L.coef_a;
-    a.init_f = L.init_f;
-    a.init_a = L.init_a;
-    a.steps = L.steps;
-    a.exc = L.exc;
-    a.out_f = L.out_f;
-    a.out_a = L.out_a;
-    a.na_out = L.na_out;
-    a.ck_off = L.ckoff;
-    a.out_q = out_q;
-    a.out_max = d->window ? d->out_max.p : nullptr;
-    a.traj = save_steps ? d->traj.p : nullptr;
-    a.out_grad = adjoint ? out_grad : nullptr;
-    a.excit = excit;
-    a.interp = d->interp_w ? interp : nullptr;
-    a.stride = st;
-    a.count = L.count;
-    a.block_begin = L.block_begin;
-    a.klass = L.klass;
-    a.exc_len = d->exc_len;
-    a.interp_w = d->interp_w;
-    a.window = d->window;
-    a.out_len = pk.out_len_f;
-    a.save_every = save_steps;
-    a.nslots = nslots;
-    a.ck_every = K;
-    a.nck = nck;
-    a.adjoint = adjoint ? 1 : 0;
-    // h = 1/sampleRate in the working type, h2 and h6 from that h in double
-    // (src/__GpuDriver.cu:632-636), carried exactly in a double
-    a.h = double(h);
-    a.h2 = double(R(double(h) / 2.0));
-    a.h6 = double(R(double(h) / 6.0));
-  }
+  std::vector<LaneArgs> args;
+  for (auto& L : P.cls)
+    args.push_back(lane_cls_args<R>(d, P, *L, adjoint, save_steps, nslots, excit, interp, mem,
+                                    out_q, out_grad, 0, L->waves));
   return args;
 }
 
@@ -3545,12 +3571,13 @@ void lane_paths(pasif_driver* d, PathLease& lease, std::vector<std::vector<LaneA
     }
 }
 
-hipError_t lane_launch(const LanePart& P, const void* dargs, uint32_t n, hipStream_t st) {
+hipError_t lane_launch(const LanePart& P, const void* dargs, uint32_t n, uint32_t blocks,
+                       hipStream_t st) {
   // multi-wave kernels declare their LDS statically
   const uint32_t lds = P.lay.waves > 1 ? 0u : uint32_t(P.lds);
   void* dp = const_cast<void*>(dargs);
   void* params[] = {&dp, &n};
-  return hipModuleLaunchKernel(P.kern.fn, P.blocks, 1, 1, kLaneWave * P.lay.waves, 1, 1, lds,
+  return hipModuleLaunchKernel(P.kern.fn, blocks, 1, 1, kLaneWave * P.lay.waves, 1, 1, lds,
                                st, params, nullptr);
 }
 
@@ -3563,12 +3590,88 @@ void ensure_aux(pasif_driver* d, int n) {
   }
 }
 
+// Waves [w0, w0 + n) of one class of a single-wave lane part, and the bytes of
+// their run buffers and kernel arguments.
+struct LaneSlice {
+  LanePart* part;
+  LaneCls* cls;
+  uint32_t w0, n;
+  size_t bytes;
+};
+
+// The packed problem's single-wave lane parts in pieces whose run buffers fit
+// `cap` bytes (false: one wave's do not): as many waves of a class at a time
+// as fit.  Checkpoints are most of it, and the layouts that are fastest keep
+// more of them than others (a system over more lanes has fewer steps between
+// two and padding in each); memory decides only how much runs at once.
+template <typename R>
+bool lane_slices(pasif_driver* d, bool adjoint, uint32_t save_steps, size_t cap,
+                 std::vector<LaneSlice>* out) {
+  DevBuf unused;
+  for (auto& lp : d->pk.lparts) {
+    if (lp->lay.waves != 1) continue;
+    for (auto& L : lp->cls) {
+      auto bytes = [&](uint32_t w0, uint32_t n) {
+        RunMem m;
+        m.d = d;
+        m.sizing = true;
+        (void)lane_cls_args<R>(d, *lp, *L, adjoint, save_steps, 0, nullptr, nullptr, m, nullptr,
+                               nullptr, w0, n);
+        m.get(unused, sizeof(LaneArgs));
+        return m.used;
+      };
+      for (uint32_t w0 = 0; w0 < L->waves;) {
+        uint32_t n = L->waves - w0;
+        if (bytes(w0, n) > cap) {
+          uint32_t lo = 0, hi = n;  // lo waves fit, hi do not
+          while (hi - lo > 1u) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            (bytes(w0, mid) > cap ? hi : lo) = mid;
+          }
+          n = lo;
+        }
+        if (n == 0) return false;
+        out->push_back({lp.get(), L.get(), w0, n, bytes(w0, n)});
+        w0 += n;
+      }
+    }
+  }
+  return true;
+}
+
+// Run slices one after the other, their run buffers in `base`.
+template <typename R>
+void run_slices(pasif_driver* d, bool adjoint, uint32_t save_steps, uint32_t nslots,
+                const std::vector<LaneSlice>& slices, void* base, size_t cap, void* out_q,
+                void* out_grad) {
+  DevBuf unused;
+  for (const LaneSlice& x : slices) {
+    RunMem mem;
+    mem.d = d;
+    mem.base = static_cast<unsigned char*>(base);
+    mem.cap = cap;
+    LaneArgs a = lane_cls_args<R>(d, *x.part, *x.cls, adjoint, save_steps, nslots, d->d_exc.p,
+                                  d->d_interp.p, mem, out_q, out_grad, x.w0, x.n);
+    void* table = mem.get(unused, sizeof a);
+    uint64_t launches = 1;
+    a.budget = launch_budget(d, (adjoint ? 3ull : 1ull) * x.cls->wave_t[x.w0], &launches);
+    PASIF_HIP(hipMemcpyAsync(table, &a, sizeof a, hipMemcpyHostToDevice, d->stream));
+    const double ms = d->last_ms;
+    const uint32_t before = d->last_launches;
+    drive(d, launches,
+          [&]() -> hipError_t { return lane_launch(*x.part, table, 1, x.n, d->stream); });
+    d->last_ms += ms;
+    d->last_launches += before;
+  }
+}
+
 // Device bytes the run buffers of a solve of the packed problem take
 // (outputs included; the packed program itself is not), and of those the
-// checkpoints: a sizing pass over the same requests a solve makes.
+// checkpoints: a sizing pass over the same requests a solve makes.  `pieces`:
+// without the single-wave lane parts, which run in pieces then.
 template <typename R>
 void run_footprint(pasif_driver* d, bool adjoint, uint32_t save_steps, size_t* total,
-                   size_t* ckpt) {
+                   size_t* ckpt, bool pieces = false) {
   Packed& pk = d->pk;
   RunMem m;
   m.d = d;
@@ -3587,6 +3690,7 @@ void run_footprint(pasif_driver* d, bool adjoint, uint32_t save_steps, size_t* t
   if (pk.rows)
     (void)row_run_args<R>(d, adjoint, save_steps, nslots, m, nullptr, nullptr, &work);
   for (auto& lp : pk.lparts) {
+    if (pieces && lp->lay.waves == 1) continue;
     auto args = lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, nullptr, nullptr, &m,
                                   nullptr, nullptr);
     m.get(unused, args.size() * sizeof(LaneArgs));
@@ -3614,10 +3718,12 @@ size_t held_run_bytes(const pasif_driver* d) {
 
 // The memory plan of a solve: its run buffers must fit in 80 % of the device
 // memory free now plus what the driver already holds for them (the 0.8 x
-// free rule of the reference's planner, src/__GpuDriver.cu:896-938), or the
-// solve is refused before anything is allocated.
+// free rule of the reference's planner, src/__GpuDriver.cu:896-938), or -- of
+// the single-wave lane parts -- those of `pieces` must (empty: all at once), or
+// the solve is refused before anything is allocated.
 template <typename R>
-void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps) {
+void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps,
+                      std::vector<LaneSlice>* pieces) {
   if (d->dev < 0 || d->pool) return;
   size_t need = 0, ck = 0, freeb = 0, totalb = 0;
   run_footprint<R>(d, adjoint, save_steps, &need, &ck);
@@ -3629,7 +3735,12 @@ void check_run_memory(pasif_driver* d, bool adjoint, uint32_t save_steps) {
     PASIF_HIP(hipMemGetInfo(&freeb, &totalb));
     avail = 0.8 * double(freeb + held_run_bytes(d));
   }
-  PASIF_REQUIRE(double(need) <= avail, PASIF_ERR_MEMORY,
+  if (double(need) <= avail) return;
+  size_t rest = 0, rest_ck = 0;
+  run_footprint<R>(d, adjoint, save_steps, &rest, &rest_ck, true);
+  const bool fit = rest < need && double(rest) < avail &&
+                   lane_slices<R>(d, adjoint, save_steps, size_t(avail) - rest, pieces);
+  PASIF_REQUIRE(fit, PASIF_ERR_MEMORY,
                 "the solve needs %zu bytes of run buffers (%zu of them checkpoints), more than "
                 "80%% of the free device memory (%.0f bytes available); lengthen the checkpoint "
                 "interval or solve fewer systems at once",
@@ -3646,7 +3757,12 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
   PASIF_REQUIRE(!pk.big_only || (save_steps == 0 && d->window == 0), PASIF_ERR_UNSUPPORTED,
                 "systems on the row-parallel path (too large for a tile) record neither a "
                 "trajectory nor an amplitude window");
-  check_run_memory<R>(d, adjoint, save_steps);
+  std::vector<LaneSlice> pieces;
+  check_run_memory<R>(d, adjoint, save_steps, &pieces);
+  for (const LaneSlice& x : pieces)  // their buffers are the block's (below)
+    for (DevBuf* b : {&x.cls->qstate, &x.cls->lstate, &x.cls->mxstate, &x.cls->progress,
+                      &x.cls->ckpt, &x.cls->segbuf})
+      b->release();
   uint64_t twork = 0, bwork = 0;
   uint32_t nslots = 0;
   TileArgs<R> ta{};
@@ -3667,14 +3783,23 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
   std::vector<std::vector<LaneArgs>> largs;
   if (lane) {
     nslots = run_outputs<R>(d, adjoint, save_steps);
-    for (auto& lp : pk.lparts)
-      largs.push_back(lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, d->d_exc.p,
-                                        d->d_interp.p));
+    for (auto& lp : pk.lparts) {
+      largs.emplace_back();
+      if (pieces.empty() || lp->lay.waves != 1)
+        largs.back() = lane_part_args<R>(d, *lp, adjoint, save_steps, nslots, d->d_exc.p,
+                                         d->d_interp.p);
+    }
+  }
+  DevBuf block;
+  if (!pieces.empty()) {
+    size_t bytes = 0;
+    for (const LaneSlice& x : pieces) bytes = std::max(bytes, x.bytes);
+    dev_alloc(d, block, bytes);
   }
   // Paths come last: every buffer the solve cannot do without is there by now,
   // and what a path takes of the memory left cannot refuse the solve.
   if (pk.rows) row_path<R>(d, lease, ra, &rwork);
-  if (lane) lane_paths<R>(d, lease, largs);
+  if (lane && pieces.empty()) lane_paths<R>(d, lease, largs);
   bwork = std::max(bwork, rwork);
   const uint64_t lwork = lane ? (adjoint ? 3ull * pk.ltmax : pk.ltmax) : 0;
   uint64_t launches = 1;
@@ -3683,6 +3808,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
   ba.budget = budget;
   ra.budget = budget;
   for (size_t i = 0; i < largs.size(); ++i) {
+    if (largs[i].empty()) continue;
     for (LaneArgs& a : largs[i]) a.budget = budget;
     upload(d, pk.lparts[i]->args, largs[i]);
   }
@@ -3691,7 +3817,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
   // up to three side streams (modules beyond that share them in turn)
   std::vector<size_t> lmods;
   for (size_t i = 0; i < largs.size(); ++i)
-    if (pk.lparts[i]->blocks) lmods.push_back(i);
+    if (pk.lparts[i]->blocks && !largs[i].empty()) lmods.push_back(i);
   const bool main_busy = tile || big;
   const int nside = int(std::min<size_t>(pasif_driver::kSide,
                                          lmods.size() - (main_busy || lmods.empty() ? 0 : 1)));
@@ -3702,7 +3828,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
   };
   const uint32_t nb = pk.nbig;
   const uint32_t nt = pk.ntiles;
-  drive(d, launches, [&]() -> hipError_t {
+  auto launch = [&]() -> hipError_t {
     hipError_t e = hipSuccess;
     if (nside > 0) {
       e = hipEventRecord(d->fork, d->stream);
@@ -3712,7 +3838,7 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
     for (size_t j = 0; j < lmods.size() && e == hipSuccess; ++j) {
       const LanePart& P = *pk.lparts[lmods[j]];
       const int k = lane_stream(j);
-      e = lane_launch(P, P.args.p, uint32_t(largs[lmods[j]].size()),
+      e = lane_launch(P, P.args.p, uint32_t(largs[lmods[j]].size()), P.blocks,
                       k < 0 ? d->stream : d->aux[k]);
     }
     if (tile && e == hipSuccess) e = launch_tiles(ta, nt, int(pk.slot_cfg), d->stream);
@@ -3725,7 +3851,13 @@ void solve_impl(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOu
       if (e == hipSuccess) e = hipStreamWaitEvent(d->stream, d->join[k], 0);
     }
     return e;
-  });
+  };
+  d->last_ms = 0.0;
+  d->last_launches = 0;
+  if (main_busy || !lmods.empty() || pieces.empty()) drive(d, launches, launch);
+  if (!pieces.empty())
+    run_slices<R>(d, adjoint, save_steps, nslots, pieces, block.p, block.bytes, d->out_q.p,
+                  adjoint ? d->out_grad.p : nullptr);
   finish_run<R>(d, nslots, out);
 }
 
@@ -3768,7 +3900,8 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
   uint64_t twork = 0, rwork = 0;
   std::vector<std::vector<LaneArgs>> largs;
   std::vector<void*> tables;
-  auto plan = [&](RunMem& mem) {
+  std::vector<LaneSlice> pieces;
+  auto plan = [&](RunMem& mem, bool whole) {
     largs.clear();
     tables.clear();
     uint32_t nslots = 0;
@@ -3778,16 +3911,28 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
     if (pk.rows) ra = row_run_args<R>(d, adjoint, 0, 0, mem, out_q, out_grad, &rwork);
     if (lane)
       for (auto& lp : pk.lparts) {
-        largs.push_back(lane_part_args<R>(d, *lp, adjoint, 0, 0, d->d_exc.p, d->d_interp.p,
-                                          &mem, out_q, out_grad));
-        tables.push_back(mem.get(unused, largs.back().size() * sizeof(LaneArgs)));
+        largs.emplace_back();
+        tables.push_back(nullptr);
+        if (!whole && lp->lay.waves == 1) continue;
+        largs.back() = lane_part_args<R>(d, *lp, adjoint, 0, 0, d->d_exc.p, d->d_interp.p, &mem,
+                                         out_q, out_grad);
+        tables.back() = mem.get(unused, largs.back().size() * sizeof(LaneArgs));
       }
   };
   RunMem sizing;
   sizing.d = d;
   sizing.sizing = true;
-  plan(sizing);
-  PASIF_REQUIRE(sizing.used <= cap, PASIF_ERR_MEMORY,
+  plan(sizing, true);
+  const bool whole = sizing.used <= cap;
+  bool fit = whole;
+  if (!whole) {
+    RunMem rest;
+    rest.d = d;
+    rest.sizing = true;
+    plan(rest, false);
+    fit = rest.used <= cap && lane_slices<R>(d, adjoint, 0, cap, &pieces) && !pieces.empty();
+  }
+  PASIF_REQUIRE(fit, PASIF_ERR_MEMORY,
                 "this problem needs %zu bytes of run buffers; pasif_solve_noalloc holds %zu "
                 "bytes per GPU (solve it with pasif_get_%s instead)",
                 sizing.used, cap, adjoint ? "gradient" : "amplitudes");
@@ -3795,28 +3940,37 @@ void solve_noalloc_impl(pasif_driver* d, bool adjoint, void* out_q, void* out_gr
   mem.d = d;
   mem.base = static_cast<unsigned char*>(base);
   mem.cap = cap;
-  plan(mem);
+  plan(mem, whole);
   const uint64_t lwork = lane ? (adjoint ? 3ull * pk.ltmax : pk.ltmax) : 0;
   uint64_t launches = 1;
   const uint32_t budget = launch_budget(d, std::max(std::max(twork, rwork), lwork), &launches);
   ta.budget = budget;
   ra.budget = budget;
   for (size_t i = 0; i < largs.size(); ++i) {
+    if (largs[i].empty()) continue;
     for (LaneArgs& a : largs[i]) a.budget = budget;
     PASIF_HIP(hipMemcpyAsync(tables[i], largs[i].data(), largs[i].size() * sizeof(LaneArgs),
                              hipMemcpyHostToDevice, d->stream));
   }
   const uint32_t nt = pk.ntiles;
-  drive(d, launches, [&]() -> hipError_t {
+  auto launch = [&]() -> hipError_t {
     hipError_t e = hipSuccess;
     for (size_t i = 0; i < largs.size() && e == hipSuccess; ++i)
-      if (pk.lparts[i]->blocks)
-        e = lane_launch(*pk.lparts[i], tables[i], uint32_t(largs[i].size()), d->stream);
+      if (pk.lparts[i]->blocks && !largs[i].empty())
+        e = lane_launch(*pk.lparts[i], tables[i], uint32_t(largs[i].size()),
+                        pk.lparts[i]->blocks, d->stream);
     if (tile && e == hipSuccess) e = launch_tiles(ta, nt, int(pk.slot_cfg), d->stream);
     if (pk.rows && e == hipSuccess)
       e = launch_rows(ra, pk.nrow, pk.r_waves, pk.r_slots, d->stream);
     return e;
-  });
+  };
+  const bool rest = tile || pk.rows ||
+                    std::any_of(largs.begin(), largs.end(),
+                                [](const std::vector<LaneArgs>& x) { return !x.empty(); });
+  d->last_ms = 0.0;
+  d->last_launches = 0;
+  if (rest || whole) drive(d, launches, launch);
+  run_slices<R>(d, adjoint, 0, 0, pieces, base, cap, out_q, out_grad);
 }
 
 void solve(pasif_driver* d, bool adjoint, uint32_t save_steps, const HostOut& out) {

@@ -1081,7 +1081,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   constexpr u32 NFT = (FT + G - 1u) / G;
   const u32 lane = threadIdx.x;
   const u32 p = lane & (G - 1u);
-  const u64 st = a.stride;
+  const u64 st = a.stride, ss = a.sstride;
   const u32 col = wave * WAVE + lane;
   const u32 i = wave * IPW + lane / G;
   const bool valid = i < (u32)a.count;
@@ -1133,7 +1133,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   }
   GP(R) ph = (GP(R))a.path + po + lane;
   GP(R) sb = (GP(R))a.segbuf + col;
-  GP(R) sb3 = sb + (u64)(K + 1u) * NF * st;
+  GP(R) sb3 = sb + (u64)(K + 1u) * NF * ss;
   GP(R) outq = (GP(R))a.out_q;
   GP(R) outm = (GP(R))a.out_max;
   GP(R) outg = (GP(R))a.out_grad;
@@ -1182,13 +1182,13 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   } else {
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      q[r] = qs[r * st];
-      if (a.window) mx[r] = ms[r * st];
+      q[r] = qs[r * ss];
+      if (a.window) mx[r] = ms[r * ss];
     }
   }
   if (adjoint && phase != kForward)
 #pragma unroll
-    for (int r = 0; r < NA; ++r) lam[r] = ls[r * st];
+    for (int r = 0; r < NA; ++r) lam[r] = ls[r * ss];
   bool seg_here = false;  // LDS holds the current segment up to step n
   // a launch that may stop mid-segment mirrors the segment to HBM so the
   // next launch can rebuild its LDS copy; one that runs to the end does not
@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #pragma unroll
           for (int r = 0; r < NF; ++r) {
             if (S::segr(r) >= 0) seg[S::segr(r) * WAVE + lane] = q[r];
-            if (mirror) sb[r * st] = q[r];
+            if (mirror) sb[r * ss] = q[r];
           }
         } else if (!seg_here) {
           // resumed inside a recompute: the LDS copy of the steps recomputed
@@ -1262,13 +1262,13 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
           for (u32 m = 0; m <= n - s0; ++m)
 #pragma unroll
             for (int r = 0; r < NF; ++r)
-              if (S::segr(r) >= 0) seg[(m * NSEG + S::segr(r)) * WAVE + lane] = sb[((u64)m * NF + r) * st];
+              if (S::segr(r) >= 0) seg[(m * NSEG + S::segr(r)) * WAVE + lane] = sb[((u64)m * NF + r) * ss];
           if constexpr (EX)
             for (u32 m = 0; m < 3u * (n - s0); ++m)
 #pragma unroll
               for (int r = 0; r < NF; ++r)
                 if (S::segr(r) >= 0)
-                  seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = sb3[((u64)m * NF + r) * st];
+                  seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = sb3[((u64)m * NF + r) * ss];
         }
         seg_here = true;
       }
@@ -1330,7 +1330,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #pragma unroll
               for (int r = 0; r < NF; ++r) {
                 if (S::segr(r) >= 0) seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = y[r];
-                if (mirror) sb3[((u64)m * NF + r) * st] = y[r];
+                if (mirror) sb3[((u64)m * NF + r) * ss] = y[r];
               }
             }, hl, h, h2, h6, n < fsteps);
           } else {
@@ -1347,7 +1347,7 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
 #pragma unroll
             for (int r = 0; r < NF; ++r) {
               if (S::segr(r) >= 0) seg[(m * NSEG + S::segr(r)) * WAVE + lane] = q[r];
-              if (mirror) sb[((u64)m * NF + r) * st] = q[r];
+              if (mirror) sb[((u64)m * NF + r) * ss] = q[r];
             }
           }
           if constexpr (MODE == mWin)
@@ -1588,13 +1588,13 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
         for (u32 m = 0; m <= n - s0; ++m)
 #pragma unroll
           for (int r = 0; r < NF; ++r)
-            if (S::segr(r) >= 0) seg[(m * NSEG + S::segr(r)) * WAVE + lane] = sb[((u64)m * NF + r) * st];
+            if (S::segr(r) >= 0) seg[(m * NSEG + S::segr(r)) * WAVE + lane] = sb[((u64)m * NF + r) * ss];
         if constexpr (EX)
           for (u32 m = 0; m < 3u * (n - s0); ++m)
 #pragma unroll
             for (int r = 0; r < NF; ++r)
               if (S::segr(r) >= 0)
-                seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = sb3[((u64)m * NF + r) * st];
+                seg3[(m * NSEG + S::segr(r)) * WAVE + lane] = sb3[((u64)m * NF + r) * ss];
         seg_here = true;
       }
       __builtin_amdgcn_s_waitcnt(0);
@@ -1680,12 +1680,12 @@ __device__ __forceinline__ void run(const LaneArgs& a, u32 wave, R* smem) {
   }
 #pragma unroll
   for (int r = 0; r < NF; ++r) {
-    qs[r * st] = q[r];
-    if (a.window) ms[r * st] = mx[r];
+    qs[r * ss] = q[r];
+    if (a.window) ms[r * ss] = mx[r];
   }
   if (adjoint)
 #pragma unroll
-    for (int r = 0; r < S::NA; ++r) ls[r * st] = lam[r];
+    for (int r = 0; r < S::NA; ++r) ls[r * ss] = lam[r];
   if (lane == 0u) {
     pst[0] = n;
     pst[1] = phase;

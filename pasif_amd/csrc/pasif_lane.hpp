@@ -33,14 +33,14 @@ namespace pasif {
   X(const void*, out_a)    /* u32 [stride] output base, adjoint rows */     \
   X(const void*, na_out)   /* u32 [stride] adjoint rows the instance owns    \
                               (a merged class may pad its adjoint) */       \
-  X(void*, qstate)         /* [NF][stride] state between launches */        \
-  X(void*, lstate)         /* [NA][stride] */                               \
-  X(void*, mxstate)        /* [NF][stride] running max |q| */               \
+  X(void*, qstate)         /* [NF][sstride] state between launches */       \
+  X(void*, lstate)         /* [NA][sstride] */                              \
+  X(void*, mxstate)        /* [NF][sstride] running max |q| */              \
   X(void*, progress)       /* u32 [waves][4]: step, phase, segment */       \
   X(void*, ckpt)           /* checkpoints (single-wave: per-wave blocks) */ \
   X(const void*, ck_off)   /* u64 [waves] first element of each wave's      \
                               checkpoint block [nck_w][NF][64] (single-wave) */ \
-  X(void*, segbuf)         /* [K+1][NF][stride] recomputed segment */       \
+  X(void*, segbuf)         /* [K+1][NF][sstride] recomputed segment */      \
   X(void*, path)           /* stored set points (null: none): per-wave      \
                               blocks [T_w + 1][segment rows][64] */         \
   X(const void*, path_off) /* u64 [waves] first element of each block */    \
@@ -53,6 +53,8 @@ namespace pasif {
   X(const void*, excit)    /* [n_exc][exc_len] */                           \
   X(const void*, interp)   /* [2][interp_w] or null */                      \
   X(uint64_t, stride)      /* instance slots (multiple of 64) */            \
+  X(uint64_t, sstride)     /* those of the waves launched, which the state   \
+                              buffers hold (multi-wave: stride) */          \
   X(uint64_t, count)       /* instances */                                  \
   X(uint64_t, block_begin) /* first workgroup of the class */               \
   X(uint64_t, klass)       /* the class's case in the kernel's dispatch */  \

@@ -1,6 +1,7 @@
 """The stored path of an adjoint solve is extra: it takes what the solve's own
 buffers leave, so a solve whose buffers fit runs however little is left
-beside them -- with a path for some waves or for none."""
+beside them -- with a path for some waves or for none.  One whose buffers do
+not fit runs its lane groups in pieces."""
 import numpy as np
 import pytest
 import torch
@@ -92,3 +93,29 @@ def test_trajectory_rows_with_little_memory_left():
         del hold
         torch.cuda.empty_cache()
     np.testing.assert_array_equal(tr, ref)
+
+
+def test_solve_in_pieces_when_memory_is_short():
+    print("[gpu case] 4096 16-DOF chains x 30000 steps in pieces", flush=True)
+    w, p, J = _problem(30_000)
+    w.steps_of_system = np.random.default_rng(0).integers(1, 30_001, 4096)
+    w.steps_of_system[::2] = 30_000
+    p = W.make_solver(w)
+    p.setJacobian(*J.as_args())
+    ref = p.getGradient()
+    del p
+    p = W.make_solver(w)
+    p.setJacobian(*J.as_args())
+    fp = p._runFootprint(True)
+    hold = _leave(fp["run"] * 0.9)
+    try:
+        g = p.getGradient()
+        again = p.getGradient()
+        p.setSolver("graph", steps_per_launch=9_000, launches_per_graph=4)
+        graph = p.getGradient()
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+    np.testing.assert_array_equal(g, ref)
+    np.testing.assert_array_equal(again, ref)
+    np.testing.assert_array_equal(graph, ref)

@@ -2,9 +2,9 @@
 the allocating entry points it mirrors: pasif_get_amplitudes (forward) and
 pasif_get_gradient (forward + adjoint).  Both run the same kernels, so the
 results must be bitwise equal.  Two problems in a row share the library's
-static scratch array, the second smaller than the first; a problem whose run
-buffers exceed the array is refused before anything runs; a call without
-the set-up is refused."""
+static scratch array, the second smaller than the first; lane groups whose
+run buffers exceed the array run in pieces, tiles are refused before anything
+runs; a call without the set-up is refused."""
 import ctypes as C
 
 import numpy as np
@@ -116,6 +116,33 @@ def test_noalloc_fp32_equals_allocating():
     q_ref = p.getAmplitudes()
     nq, _ = _lengths(p, False)
     q, _ = _noalloc(p, False, nq, 0, bits=32)
+    assert np.array_equal(q, q_ref)
+
+
+@pytest.mark.parametrize("solver", ["persistent", "plain"])
+@pytest.mark.parametrize("d,steps", [(5, 3000), (13, 5000)])
+def test_noalloc_in_pieces_when_the_scratch_is_short(d, steps, solver):
+    """Lane groups keep more checkpoints than the array holds for all systems at
+    once: they run in pieces, uneven step counts and several checkpoint blocks
+    in each."""
+    n = 2048 if d == 5 else 1501
+    if solver == "plain":
+        steps //= 12
+        n *= 5
+    _case(f"noalloc {solver}: chains {n} x {d} DOF x {steps} steps, in pieces")
+    w = W.chains(n_systems=n, d=d, steps=steps, steps_per_sample=10)
+    w.steps_of_system = np.random.default_rng(d).integers(1, steps + 1, n)
+    w.steps_of_system[::3] = steps
+    p = W.make_solver(w)
+    p.setJacobian(*ADJ.energy_gradient_inputs(w).as_args())
+    p.setTuning(checkpoint_every=256)
+    g_ref = p.getGradient()
+    q_ref = p.getAmplitudes()
+    p.setSolver(solver)
+    nq, ng = _lengths(p, True)
+    assert p._runFootprint(True)["run"] - 8 * (nq + ng) > SCRATCH_BYTES
+    q, g = _noalloc(p, True, nq, ng)
+    assert np.array_equal(g, g_ref)
     assert np.array_equal(q, q_ref)
 
 
