@@ -1922,6 +1922,12 @@ struct Sig {
   }
 };
 
+// The loaded forcing rule as the lane kernels compile it (1 interpolation, 2
+// zero-order hold): every step loop exists once for each rule compiled, and
+// both would double the compiler's time (gradient of 16-DOF chains 7.3 s, a
+// batch of seven sizes 44 s).  Loading the other rule packs again.
+uint32_t forcing_rule(const pasif_driver* d) { return d->interp_w ? 1u : 2u; }
+
 // What a lane plan depends on besides coefficient values and initial
 // states: the systems' structure (term indices, sizes, force pattern), the
 // instances (excitations, step counts), the settings and the device.
@@ -1931,6 +1937,7 @@ uint64_t lane_plan_sig(const pasif_driver* d, bool adjoint, int bits) {
   g.word(uint64_t(bits));
   g.word(uint64_t(int64_t(d->dev)));
   g.word(lane_max_live(1));
+  g.word(forcing_rule(d));
   if (const char* f = std::getenv("PASIF_JIT_FLAGS"))
     for (const char* c = f; *c; ++c) g.word(uint64_t(uint8_t(*c)));
   auto rows = [&](const RowTerms& rt) {
@@ -2440,6 +2447,7 @@ bool lane_plan(pasif_driver* d, bool adjoint) {
     LaneLayout lay;
     lay.ilp = waves <= device_simds(d->dev);
     lay.exact = exact;
+    lay.forcing = forcing_rule(d);
     // an interval of the caller's choice keeps its checkpoints
     lay.store = adjoint && !exact && d->ck_every == 0;
     const uint32_t by_waves =
@@ -2462,7 +2470,9 @@ bool lane_plan(pasif_driver* d, bool adjoint) {
   }
   if (!many.empty()) {
     const size_t m0 = mods.size();
-    deal(many, LaneLayout{});
+    LaneLayout lay0;
+    lay0.forcing = forcing_rule(d);
+    deal(many, lay0);
     double total = 0;
     for (uint32_t c : many) total += loads[c].inst;
     for (size_t m = m0; m < mods.size(); ++m) {
@@ -4235,6 +4245,7 @@ int pasif_set_interpolation_matrix(pasif_driver* d, const double* m, size_t size
   return guarded(d, [&] {
     PASIF_REQUIRE(!d->ext_interp && !d->ext_exc, PASIF_ERR_STATE,
                   "this job uses its pool's signal bank and interpolation");
+    const uint32_t rule = forcing_rule(d);
     if (size == 0) {
       d->interp.clear();
       d->interp_w = 0;
@@ -4251,6 +4262,7 @@ int pasif_set_interpolation_matrix(pasif_driver* d, const double* m, size_t size
       d->interp_w = w;
     }
     d->d_exc_dirty = true;
+    if (d->pk.lane && forcing_rule(d) != rule) d->pk.valid = false;
   });
 }
 

@@ -224,3 +224,25 @@ def test_probes_that_share_products(G, d):
     p.setJacobian(*J.as_args())
     assert p.kernelInfo(True)["kernel"] == "lane"
     assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64
+
+
+@pytest.mark.parametrize("G,d", [(1, 2), (4, 2), (16, 16)])
+def test_forcing_rule_loaded_between_solves(G, d):
+    """One handle with interpolated forcing, then zero-order hold, then
+    interpolation again: kernels of the loaded rule each time."""
+    _case(f"forcing rules in turn G={G}, {d} DOF")
+    w = W.chains(9, d, 70, steps_per_sample=10)
+    w.excitations = np.random.default_rng(d).normal(0, 1, (9, 60))
+    J = ADJ.energy_gradient_inputs(w)
+    p = W.make_solver(w)
+    p.setKernel("lane", G)
+    p.setJacobian(*J.as_args())
+    interp = w.interp
+    for rule in (interp, None, interp):
+        w.interp = rule
+        if rule is None:
+            p._setInterpolationMatrix(np.zeros(0), 0)
+        else:
+            p.setInterpolationMatrix(list(rule))
+        assert rel_err(p.getAmplitudes(), oracle_run(w).q) < TOL64
+        assert rel_err(p.getGradient(), oracle_gradient(w, J, 64)) < TOL64

@@ -154,6 +154,24 @@ def test_probes_that_share_products_compile(d, G):
     p._laneSource(True, compile=True)
 
 
+@pytest.mark.parametrize("maker", [lambda: W.chains(64, 2, 60, steps_per_sample=10),
+                                   lambda: W.chains(64, 16, 60, steps_per_sample=10)])
+@pytest.mark.parametrize("group", [0, 1])
+def test_one_forcing_rule_is_compiled(maker, group):
+    # the loaded rule alone (every step loop would be there twice), and the
+    # other one's program once that is loaded; one lane per instance of 16 DOF:
+    # workgroups of waves
+    w = maker()
+    p = host_solver(w)
+    p.setKernel("auto", group)
+    for _ in range(2):
+        assert "#define FORCING 1\n" in p._laneSource(False)
+        p._setInterpolationMatrix(np.zeros(0), 0)
+        src = p._laneSource(False, compile=True)
+        assert "#define FORCING 2\n" in src
+        p.setInterpolationMatrix(list(w.interp))
+
+
 def test_chain_group_program_is_the_stencil():
     # 16-DOF chain on 16 lanes: lane p holds x_p, v_p and the shared energy
     # row; neighbours come by rotations +-1.  Nothing reads the energy row, so
