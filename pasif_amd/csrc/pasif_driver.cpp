@@ -1608,10 +1608,12 @@ uint64_t pack_key(pasif_driver* d, bool adjoint) {
 // ------------------------------------------------------------ lane plan
 // Largest state + coefficient count (values of the working type) a class may
 // keep live: 2 VGPRs per FP64 value, leaving room for temporaries in 256.
-// A group of a whole wave may keep twice that (the compiler moves the rest to
-// the accumulation registers): its system has no wider layout, and 48 150-DOF
-// chains x 1,000 steps with their adjoint (144 live values) take 1.34 ms so
-// against 5.03 on the row kernel, 200-DOF ones (185) 2.80 against 5.03.
+// A group of a whole wave may keep twice that, since its system has no wider
+// layout.  The kernel then takes all 512 registers of a lane, the accumulation
+// half included, and spills what is left: 98 of them (396 bytes a lane) for the
+// gradient of 150-DOF chains (144 live values), 412 (1,620 bytes) of 200-DOF
+// ones (185).  It is still the faster one: 48 of them x 1,000 steps 1.34 and
+// 2.80 ms against 5.03 on the row kernel.
 constexpr uint32_t kLaneMaxLive = 96;
 uint32_t lane_max_live(uint32_t G) {
   if (const char* e = std::getenv("PASIF_LANE_MAX_LIVE")) {

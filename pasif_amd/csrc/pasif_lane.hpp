@@ -130,8 +130,8 @@ struct GSide {
   std::vector<uint32_t> held;    // positions that hold a row (the rest: zeros)
   std::vector<uint32_t> shared;  // row of each shared slot
   std::vector<GRow> rows;        // [RL + NS]
-  // shared slots no term reads (forward: nor the adjoint's set points): the
-  // group sums their slopes once per step instead of once per stage
+  // slots no term reads (forward: nor the adjoint's set points): of a shared
+  // one each lane keeps its own part, summed over the group where it is output
   std::vector<uint8_t> sink;     // [RL + NS]
   uint32_t nl() const { return RL + NS; }
   uint32_t coefs() const;        // per-lane coefficient slots: row by row, terms then force

@@ -175,8 +175,8 @@ def test_one_forcing_rule_is_compiled(maker, group):
 def test_chain_group_program_is_the_stencil():
     # 16-DOF chain on 16 lanes: lane p holds x_p, v_p and the shared energy
     # row; neighbours come by rotations +-1.  Nothing reads the energy row, so
-    # its per-lane partial slopes are summed by the butterfly once per step
-    # (in rk4, through sink()) rather than in every stage's right-hand side.
+    # each lane keeps its own part of it (rk4, through sink()) and the parts are
+    # summed by the butterfly where the row is output, not in any right-hand side.
     w = W.chains(64, 16, 60, steps_per_sample=10)
     p = host_solver(w)
     p.setJacobian(*ADJ.energy_gradient_inputs(w).as_args())
