@@ -119,3 +119,31 @@ def test_solve_in_pieces_when_memory_is_short():
     np.testing.assert_array_equal(g, ref)
     np.testing.assert_array_equal(again, ref)
     np.testing.assert_array_equal(graph, ref)
+
+
+def test_handles_of_several_threads_share_the_path_memory():
+    print("[gpu case] path memory: three threads, four gradients each, trims between", flush=True)
+    import threading
+    cases = []
+    for n, d, steps in ((512, 16, 900), (64, 4, 2500), (3, 300, 60)):
+        w = W.chains(n_systems=n, d=d, steps=steps, steps_per_sample=10, seed=n)
+        J = ADJ.energy_gradient_inputs(w)
+        p = W.make_solver(w)
+        p.setJacobian(*J.as_args())
+        cases.append((p, p.getGradient()))
+    bad = []
+
+    def run(k):
+        p, ref = cases[k]
+        for i in range(4):
+            if not np.array_equal(p.getGradient(), ref):
+                bad.append((k, i))
+            if k == i % 3:
+                p._trimMemory()
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
