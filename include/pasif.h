@@ -208,8 +208,9 @@ int pasif_lane_groups(pasif_driver* d, int adjoint, uint32_t* out, size_t cap, s
  * -- the reverse-mode derivative of the computed RK4 step, the adjoint system
  * evaluated at each step's forward stage inputs y4, y3, y2, y1 (recomputed
  * and stored per segment); it equals that derivative to round-off when the
- * adjoint system is the transposed Jacobian of the forward one.  Mode 1 runs
- * on the tile kernel (PASIF_ERR_UNSUPPORTED with PASIF_KERNEL_LANE). */
+ * adjoint system is the transposed Jacobian of the forward one.  Every
+ * kernel runs it but lane classes that need several waves, which go to tiles
+ * (PASIF_ERR_UNSUPPORTED with PASIF_KERNEL_LANE). */
 int pasif_set_adjoint_mode(pasif_driver* d, int mode);
 /* Memory plan (extension): device bytes the run buffers and outputs of a
  * solve of the loaded problem take with the current settings (*run_bytes),
